@@ -69,20 +69,48 @@ __device__ __forceinline__ bool pair_fp64(const AbfsFactors &F, double r2, doubl
 
 // Tiled path: one pair with 1/r from the FP32 v_rsq seed refined by one
 // Newton step in FP64 (relative error ~1e-14; no FP64 divide or square root).
-// On gfx950 FP64 FMA issues at the FP32 rate, so the scalar core stays in FP64
-// and only the rsqrt seed and the force vectors are FP32.
+// The kernel is bound by VALU issue, and every instruction here but the FP32
+// multiply-adds, moves and 32-bit adds takes a full issue slot (measured: 1.9 ns
+// per wave instruction and SIMD for FP64 arithmetic, compares, selects, shifts
+// and conversions alike, 1.05 ns for v_fma/add/mul_f32, v_add_u32, v_mov_b32 and
+// v_and_b32, 3.6 ns for v_rsq_f32), so the forms below are chosen for their
+// instruction count.
 //
-// Lennard-Jones in both undamped regions is one polynomial in s = 1/r,
-//   E = C12 s^12 + C6 s^6 + C3 s^3 + C0,
-// whose coefficients per type pair and region come from a row table (plain:
-// A, -B, 0, B*bShift6 - A*aShift12; switched: the expanded squares
-// A*aK12*(s^6-aF6)^2 - B*bK6*(s^3-bF3)^2), so the region choice is a row
-// index instead of two evaluated branches.  The Coulomb switch keeps the
-// reference polynomials, blended by a 0/1 region factor.  The damped region
-// (r < dampingCutoff) is a wave-uniform rare path on the raw A, B.
-__device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, double qq, double4 C, bool sw,
+// u = clamp((r2 - r2On)/(r2Off - r2On)) is one multiply-add with the clamp
+// modifier: 0 in the plain region, in (0, 1] in the switched one.
+//   * Coulomb force: the reference's factor a + r2 (b + r2 (3c + 5d r2)) is the
+//     smoothstep 1 + u^2 (2u - 3), exactly 1 in the plain region.
+//   * Coulomb energy: s + sc (P - 1) + qShift2 with sc = min(s, 1/inner) and
+//     P - 1 = (a - 1) - r2 (b + r2 (c + d r2)) as a cubic in u.  In the plain
+//     region sc (P - 1) + qShift2 is the constant qShift1 (the reference's
+//     energies meet at the inner cutoff), so no region is selected.
+//   * Lennard-Jones in both undamped regions is one polynomial in s = 1/r,
+//       E = C12 s^12 + C6 s^6 + C3 s^3 + C0,
+//     whose coefficients per type pair and region come from a row table (plain:
+//     A, -B, 0, B*bShift6 - A*aShift12; switched: the expanded squares
+//     A*aK12*(s^6-aF6)^2 - B*bK6*(s^3-bF3)^2); the region's row offset comes from
+//     the high word of u (0 for u = 0) without a compare.
+// The damped region (r < dampingCutoff) is a wave-uniform rare path on the raw
+// A, B.  The rows hold three times the coefficients, so that the factor 3 of the
+// Lennard-Jones force costs nothing: elj is 3 E, divided by 3 with the item's
+// total, and fs is minus twice dE/d(r^2).
+__device__ __forceinline__ double switch_coordinate(const AbfsFactors &F, double uShift, double r2)
+{
+    return fmin(fmax(fma(r2, F.uScale, uShift), 0.0), 1.0);
+}
+
+// min(x, s) with s in scalar registers.  fmin of a kernel argument would first
+// canonicalise it, one more instruction per use; neither operand is a signalling NaN.
+__device__ __forceinline__ double min_uniform(double x, double s)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "s"(s));
+    return r;
+}
+
+__device__ __forceinline__ void pair_rows(const AbfsFactors &F, double p3, double r2, double u, double qq, double4 C,
                                           unsigned long long mact, const GAS double *__restrict__ ljA,
-                                          const GAS double *__restrict__ ljB, int tij, double &fs, double &eel,
+                                          const GAS double *__restrict__ ljB, int off, double &fs, double &eel,
                                           double &elj)
 {
     const double y = (double)__builtin_amdgcn_rsqf((float)r2);
@@ -91,30 +119,22 @@ __device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, doubl
     const double s2 = s * s;
     const double s3 = s2 * s;
     const double s6 = s3 * s3;
-    // Coulomb in both undamped regions as one expression, m = 1 in the switched region and 0 in the plain
-    // one (the reference's E = qq (s P + K) with P = 1, K = qShift1 below the inner cutoff):
-    //   E / qq = s + qShift1 + m (s (P - 1) + qShift2 - qShift1),   P - 1 = (a - 1) - r2 (b + r2 (c + d r2)),
-    //   qq Q   = qq + qq m (Q - 1),                                 Q - 1 = (a - 1) + r2 (b + r2 (3c + 5d r2)).
-    // A product with m in {0, 1} is exact, so each region evaluates its own reference form.
-    const double m = sw ? 1.0 : 0.0;
-    const double pm1 = fma(-r2, fma(r2, fma(F.d, r2, F.c), F.b), F.a - 1.0);
-    const double qm1 = fma(r2, fma(r2, fma(5.0 * F.d, r2, 3.0 * F.c), F.b), F.a - 1.0);
-    double e1 = qq * fma(m, fma(s, pm1, F.qShift2 - F.qShift1), s + F.qShift1);
-    const double qQ = fma(qq * m, qm1, qq);
-    // Lennard-Jones row E = C12 s^12 + C6 s^6 + C3 s^3 + C0 (t1 = C12 s^6 + C6), and
-    // inner = s^3 (4 C12 s^6 + 2 C6) + C3 = 2 s^3 (C12 s^6 + t1) + C3.
+    const double Q = fma(u * u, fma(2.0, u, -3.0), 1.0);
+    const double sc = min_uniform(s, F.sOn);
+    const double pm1 = fma(fma(fma(p3, u, F.p2), u, F.p1), u, F.p0);
+    double e1 = qq * (s + fma(sc, pm1, F.qShift2));
+    // inner = s^3 (4 C12 s^6 + 2 C6) + C3 = 2 s^3 (C12 s^6 + t1) + C3, t1 = C12 s^6 + C6.
     const double t1 = fma(C.x, s6, C.y);
     double e2 = fma(t1, s6, fma(C.z, s3, C.w));
-    const double inner = fma(2.0 * s3, fma(C.x, s6, t1), C.z);
-    // Twice dE/d(r^2) of both terms (the gradient's factor 2 folded in; exact):
-    //   Coulomb -qq s^3 Q, Lennard-Jones -3 s^5 inner, so fs = -s^3 (qq Q + 3 s^2 inner).
-    double f = -s3 * fma(3.0 * s2, inner, qQ);
+    const double inner = fma(s3 + s3, fma(C.x, s6, t1), C.z);
+    // Minus twice dE/d(r^2): Coulomb qq s^3 Q, Lennard-Jones 3 s^5 inner (the rows' factor 3).
+    double f = s3 * fma(s2, inner, qq * Q);
     if (__builtin_amdgcn_ballot_w64(r2 < F.r2Damp) & mact) {
         if (r2 < F.r2Damp) {
-            const double A = ljA[tij], B = ljB[tij];
+            const double A = ljA[off >> 6], B = ljB[off >> 6];
             e1 = qq * fma(-F.qAlpha, r2, F.qF0);
-            e2 = A * fma(-F.aAlpha, r2, F.aF0) - B * fma(-F.bAlpha, r2, F.bF0);
-            f = (-qq * F.qAlpha) * 2.0 + (-A * F.aAlpha + B * F.bAlpha) * 2.0;
+            e2 = 3.0 * (A * fma(-F.aAlpha, r2, F.aF0) - B * fma(-F.bAlpha, r2, F.bF0));
+            f = 2.0 * (qq * F.qAlpha + (A * F.aAlpha - B * F.bAlpha));
         }
     }
     fs = f;
@@ -283,6 +303,22 @@ __device__ __forceinline__ double4 load_slot(const GAS double *__restrict__ xr, 
     return make_double4(xr[4 * k], xr[4 * k + 1], xr[4 * k + 2], xr[4 * k + 3]);
 }
 
+// The j-cluster's records and types: a wave-uniform base plus a 32-bit lane offset.
+__device__ __forceinline__ double4 load_j(const GAS double *__restrict__ xr, int J, unsigned off)
+{
+    unsigned long long base = (unsigned long long)(xr + (size_t)J * (4 * NB_CL));
+    asm("" : "+s"(base));      // keeps the uniform part of the address in scalar registers
+    const GAS double *p = (const GAS double *)((const GAS char *)base + off);
+    return make_double4(p[0], p[1], p[2], p[3]);
+}
+
+__device__ __forceinline__ int load_jtype(const GAS int *__restrict__ ty, int J, unsigned off)
+{
+    unsigned long long base = (unsigned long long)(ty + (size_t)J * NB_CL);
+    asm("" : "+s"(base));
+    return *(const GAS int *)((const GAS char *)base + off);
+}
+
 // Entry fields through the vector memory path: J and cbits are read by every
 // lane from one address (one request) and made uniform; each lane reads its
 // own tile-mask byte (64 consecutive bytes per entry).
@@ -292,47 +328,131 @@ __device__ __forceinline__ int2 entry_jc(const GAS unsigned char *__restrict__ e
     return make_int2(p[0], p[2]);
 }
 
-__device__ __forceinline__ int entry_bits(const GAS unsigned char *__restrict__ eb, int e, int lane)
+__device__ __forceinline__ int entry_bits(const GAS unsigned char *__restrict__ eb, int e, unsigned lane)
 {
-    return eb[(size_t)e * sizeof(Entry) + 16 + lane];
+    unsigned long long base = (unsigned long long)(eb + (size_t)e * sizeof(Entry));
+    asm("" : "+s"(base));
+    return ((const GAS unsigned char *)base + 16)[lane];
 }
 
-// Sum over the eight consecutive lanes 8b..8b+7 with DPP moves: quad
-// exchanges (xor 1, xor 2) then the half-row mirror (lane i <-> 7-i).  Every
-// lane of the group ends with the total, in the same order on every lane.
+// Sums over the eight consecutive lanes 8b..8b+7 with DPP moves: quad
+// exchanges (xor 1, xor 2), then the half-row mirror (lane i <-> 7-i).
 template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v)
+__device__ __forceinline__ float dpp_move(float v)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
-__device__ __forceinline__ float sum8(float v)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
 {
-    v += dpp_f32<0xB1>(v);    // quad_perm [1,0,3,2]
-    v += dpp_f32<0x4E>(v);    // quad_perm [2,3,0,1]
-    v += dpp_f32<0x141>(v);   // row_half_mirror
-    return v;
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
 }
 
-// FP64 version (full-FP64 tiled kernel): a butterfly over the same 8 lanes;
-// every lane adds the same operands in the same tree, so all end bit-equal.
-__device__ __forceinline__ double sum8(double v)
+// The j-atom's record of an entry: lane a (of the eight of j-atom b) returns
+// component min(a, 7 - a) of (sum gx, sum gy, sum gz, J), so that lanes 0..3
+// hold the record.  After the two quad steps every lane of a quad has the
+// quad's three sums; it keeps one of them and the mirror adds the other quad's
+// sum of the same component: 10 instructions instead of three full sums and
+// two selects.
+__device__ __forceinline__ float j_bits(float, int J) { return __int_as_float(J); }
+__device__ __forceinline__ double j_bits(double, int J) { return (double)J; }
+__device__ __forceinline__ int bits_j(float v) { return __float_as_int(v); }
+__device__ __forceinline__ int bits_j(double v) { return (int)v; }
+
+template <class T>
+__device__ __forceinline__ T j_record(T gx, T gy, T gz, int J, int comp)
 {
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    v += __shfl_xor(v, 4, 64);
-    return v;
+    gx += dpp_move<0xB1>(gx);    // quad_perm [1,0,3,2]
+    gy += dpp_move<0xB1>(gy);
+    gz += dpp_move<0xB1>(gz);
+    gx += dpp_move<0x4E>(gx);    // quad_perm [2,3,0,1]
+    gy += dpp_move<0x4E>(gy);
+    gz += dpp_move<0x4E>(gz);
+    asm("" : "+v"(gx), "+v"(gy), "+v"(gz));    // every lane needs all three: no branches on comp
+    T v = comp == 0 ? gx : (comp == 1 ? gy : gz);
+    v += dpp_move<0x141>(v);     // row_half_mirror
+    return comp == 3 ? j_bits(v, J) : v;
+}
+
+// Totals of x (returned by lanes 0..31) and y (lanes 32..63) over the wave:
+// one half swap makes the two sums one, then five steps on it.
+__device__ __forceinline__ void swap_halves(double &x, double &y)
+{
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(y), false, false);
+    x = __hiloint2double(hi[0], lo[0]);
+    y = __hiloint2double(hi[1], lo[1]);
+}
+
+__device__ __forceinline__ void swap_halves(float &x, float &y)
+{
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(y), false, false);
+    x = __int_as_float(v[0]);
+    y = __int_as_float(v[1]);
+}
+
+__device__ __forceinline__ void swap_rows(double &x, double &y)
+{
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(y), false, false);
+    x = __hiloint2double(hi[0], lo[0]);
+    y = __hiloint2double(hi[1], lo[1]);
+}
+
+__device__ __forceinline__ void swap_rows(float &x, float &y)
+{
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_int(x), __float_as_int(y), false, false);
+    x = __int_as_float(v[0]);
+    y = __int_as_float(v[1]);
+}
+
+__device__ __forceinline__ double wave_sum2_f64(double x, double y)
+{
+    swap_halves(x, y);
+    double v = x + y;
+    v += dpp_move<0xB1>(v);      // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E>(v);      // quad_perm [2,3,0,1]
+    v += dpp_move<0x141>(v);     // row_half_mirror
+    v += dpp_move<0x128>(v);     // row_ror:8
+    double w = v;
+    swap_rows(v, w);             // the two rows of each half
+    return v + w;
+}
+
+// i-forces of one component: f[c] holds, on lane 8b + a, the partial of atom a
+// of i-cluster c over the j-atoms b; lane 8b + a ends with the sum over b of
+// cluster c = b.  A reduction in which every step halves the values as well as
+// the lanes: clusters c and c + 4 trade wave halves, c and c + 2 rows, c and
+// c + 1 row halves, so no LDS is involved (through LDS it was 24 writes, 24
+// reads and two waits per item).
+template <class T>
+__device__ __forceinline__ T i_force(T (&f)[NB_SCC], int lane)
+{
+    T g[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        swap_halves(f[c], f[c + 4]);
+        g[c] = f[c] + f[c + 4];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        swap_rows(g[c], g[c + 2]);
+        g[c] += g[c + 2];
+    }
+    const bool odd = (lane & 8) != 0;
+    const T keep = odd ? g[1] : g[0], send = odd ? g[0] : g[1];
+    return keep + dpp_move<0x128>(send);     // row_ror:8
 }
 
 // LDS of the tiled kernel (dynamic).  A workgroup holds WPG wavefronts, each
 // evaluating one work item.  At offset 0 the LJ row table of the group's
 // system when it fits (ROWS_LDS: staged once per group), then one region per
-// wave: the item's i-cluster records and slot types, then the per-entry
-// j-force sums with their j-clusters, flushed to the fixed-point accumulators
-// once at the end of the item; the i-force transpose at the end of the item
-// reuses the start of the region once the j-forces are flushed.
+// wave: the item's i-cluster records and slot types, then one record per entry
+// and j-atom (the three j-force sums and the j-cluster), flushed to the
+// fixed-point accumulators once at the end of the item.
 #define NB_LDS_I_BYTES (NB_SC * 32 + NB_SC * 4)
-#define NB_LDS_F_BYTES(acc) (NB_SCC * 3 * NB_SC * (acc))
 #define NB_LDS_ROW_LIMIT 16384
 #define NB_LDS_GROUP_LIMIT (160 * 1024 / 4)
 
@@ -341,8 +461,7 @@ static inline size_t tiled_lds_rows(int ntypes, bool rows_lds) { return rows_lds
 // acc: bytes of a force accumulator (4: FP32, the mixed kernel; 8: FP64, the full-FP64 kernel).
 static inline size_t tiled_lds_wave(int max_count, int acc)
 {
-    const size_t items = NB_LDS_I_BYTES + (size_t)max_count * (3 * NB_CL * acc + 4);
-    return std::max(items, (size_t)NB_LDS_F_BYTES(acc));
+    return NB_LDS_I_BYTES + (size_t)max_count * 4 * NB_CL * acc;
 }
 
 // Wave-scope synchronisation of a wave's own LDS region (workgroups of several
@@ -409,7 +528,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
     unsigned char *region = lds + rows_bytes + (size_t)wave * wave_bytes;
     double4 *sI = (double4 *)region;
     int *sT = (int *)(region + NB_SC * 32);
-    acc_t *sF = (acc_t *)region;
+    acc_t *sJ = (acc_t *)(region + NB_LDS_I_BYTES);   // [entry][j-atom] of (x, y, z, J)
     // The group's row table, staged once when the items are one per wave.
     int rows_sys = -1;
     if (ROWS_LDS && qp.heads == nullptr && WPG > 1) {
@@ -465,8 +584,6 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         const int n_pad = D->n_pad;
         const int nt = D->ntypes;
         const int I0 = w.sc * NB_SCC;
-        acc_t *sJF = (acc_t *)(region + NB_LDS_I_BYTES);   // [entry][3 * NB_CL]
-        int *sJ = (int *)(sJF + 3 * NB_CL * w.count);      // [entry]
         // The item's image (-1: main list); all of its entries share it.
         int img = -1;
         double isc = 1.0;
@@ -498,18 +615,24 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         sI[lane] = irec;
         sT[lane] = 64 * nt * ityp;   // byte offset of the type's first row pair
         int J = __builtin_amdgcn_readfirstlane(jc0.x);
-        double4 xj = load_slot(xq, J * NB_CL + b);
-        int tj = 64 * ty[J * NB_CL + b];
+        const unsigned jrec = 32u * b, jtyp = 4u * b;      // byte offsets in a j-cluster's records and types
+        double4 xj = load_j(xq, J, jrec);
+        int tj = 64 * load_jtype(ty, J, jtyp);
+        const int comp = min(a, NB_CL - 1 - a);
+        const double fscale = F64 ? 1.0 : -1.0;            // i-force = fscale times the sum over j
         wave_region_sync<WPG>();
 
         acc_t fx[NB_SCC], fy[NB_SCC], fz[NB_SCC];
 #pragma unroll
         for (int c = 0; c < NB_SCC; c++) fx[c] = fy[c] = fz[c] = (acc_t)0;
+        // Two factors kept in vector registers: their multiply-adds already read one scalar operand.
+        double uShift = F.uShift, p3 = F.p3;
+        asm("" : "+v"(uShift), "+v"(p3));
         double eel = 0.0, elj = 0.0;
         for (int e = w.first; e <= e_last; e++) {
             const int Jn = __builtin_amdgcn_readfirstlane(jc1.x);
-            const double4 xjn = load_slot(xq, Jn * NB_CL + b);
-            const int tjn = 64 * ty[Jn * NB_CL + b];
+            const double4 xjn = load_j(xq, Jn, jrec);
+            const int tjn = 64 * load_jtype(ty, Jn, jtyp);
             const int2 jc2 = entry_jc(eb, min(e + 2, e_last));
             const int lb2 = entry_bits(eb, min(e + 2, e_last), bl);
             const int cb = __builtin_amdgcn_readfirstlane(jc0.y);
@@ -520,9 +643,8 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
 #pragma unroll
             for (int c = 0; c < NB_SCC; c++) {
                 if (cb & (1 << c)) {
-                    const bool inl = __builtin_amdgcn_ubfe(lb, c, 1) != 0;
+                    const bool inl = (lb & (1 << c)) != 0;
                     const double4 xi = sI[c * NB_CL + a];
-                    const int roff = sT[c * NB_CL + a] + tj;   // byte offset of the pair's plain row
                     const double dx = xi.x - xjt.x, dy = xi.y - xjt.y, dz = xi.z - xjt.z;
                     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
                     const bool inr = r2 <= F.r2Off;
@@ -531,32 +653,36 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                     const unsigned long long mact = __builtin_amdgcn_ballot_w64(inl) & __builtin_amdgcn_ballot_w64(inr);
                     const bool act = __builtin_amdgcn_inverse_ballot_w64(mact);
                     if (mact != 0ull) {
+                        // Byte offset of the pair's plain row.
+                        const int ti = sT[c * NB_CL + a];
                         if (F64) {
                             // PairwiseInteraction.h:72-119 in FP64 with the reference's operations.
                             if (act) {
-                                const int tij = roff >> 6;
+                                const int tij = (ti + tj) >> 6;
                                 double x1, x2, dF;
                                 pair_fp64(F, r2, xi.w * xjt.w, ljA[tij], ljB[tij], x1, x2, dF);
                                 const double f = 2.0 * dF;
-                                const double px = f * dx, py = f * dy, pz = f * dz;
-                                fx[c] += px; fy[c] += py; fz[c] += pz;
-                                gx -= px; gy -= py; gz -= pz;
+                                fx[c] = fma(f, dx, fx[c]); fy[c] = fma(f, dy, fy[c]); fz[c] = fma(f, dz, fz[c]);
+                                gx = fma(f, dx, gx); gy = fma(f, dy, gy); gz = fma(f, dz, gz);
                                 eel += x1;
                                 elj += x2;
                             }
                         } else {
-                            const bool sw = r2 > F.r2On;
-                            const int off = roff + (sw ? 32 : 0);
+                            const double u = switch_coordinate(F, uShift, r2);
+                            const int off = ti + tj + (int)min((unsigned)__double2hiint(u), 32u);
                             const double4 C = ROWS_LDS ? *(const double4 *)((const unsigned char *)sR + off)
                                                        : load_slot(rows, off >> 5);
                             double fs, x1, x2;
-                            pair_rows(F, r2, xi.w * xjt.w, C, sw, mact, ljA, ljB, roff >> 6, fs, x1, x2);
+                            pair_rows(F, p3, r2, u, xi.w * xjt.w, C, mact, ljA, ljB, off, fs, x1, x2);
                             // The sums take the active lanes only (the others may hold any value).
                             if (act) {
-                                const float f = (float)fs;
-                                const float px = f * (float)dx, py = f * (float)dy, pz = f * (float)dz;
-                                fx[c] += px; fy[c] += py; fz[c] += pz;
-                                gx -= px; gy -= py; gz -= pz;
+                                const float f = (float)fs, px = (float)dx, py = (float)dy, pz = (float)dz;
+                                fx[c] = fmaf(f, px, (float)fx[c]);
+                                fy[c] = fmaf(f, py, (float)fy[c]);
+                                fz[c] = fmaf(f, pz, (float)fz[c]);
+                                gx = fmaf(f, px, (float)gx);
+                                gy = fmaf(f, py, (float)gy);
+                                gz = fmaf(f, pz, (float)gz);
                                 eel += x1;
                                 elj += x2;
                             }
@@ -564,12 +690,9 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                     }
                 }
             }
-            gx = sum8(gx);
-            gy = sum8(gy);
-            gz = sum8(gz);
-            const int el = e - w.first;
-            if (a < 3) sJF[el * 3 * NB_CL + 3 * b + a] = a == 0 ? gx : (a == 1 ? gy : gz);
-            if (lane == 0) sJ[el] = J;
+            const acc_t rec = j_record(gx, gy, gz, J, comp);
+            // Lanes a and 7 - a hold the same value.
+            sJ[(e - w.first) * 4 * NB_CL + 4 * b + comp] = rec;
             jc0 = jc1;
             lb0 = lb1;
             jc1 = jc2;
@@ -582,10 +705,12 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         wave_region_sync<WPG>();
         bool bad = false;
         if (!IMG) {
-            // j-forces of the whole item.
-            for (int k = lane; k < 3 * NB_CL * w.count; k += 64) {
-                const int el = k / (3 * NB_CL), r = k - el * 3 * NB_CL;
-                bad |= fx_atomic_add(facc, n_pad, sJ[el] * NB_CL + r / 3, r % 3, (double)sJF[k]);
+            // j-forces of the whole item: one record per lane.
+            for (int k = lane; k < NB_CL * w.count; k += 64) {
+                const acc_t *f = &sJ[4 * k];
+                const int sj = bits_j(f[3]) * NB_CL + (k & 7);
+                bad |= fx_atomic_add3(facc, n_pad, sj, -fscale * (double)f[0], -fscale * (double)f[1],
+                                      -fscale * (double)f[2]);
             }
         } else {
             // Image side: g'_j (scaled) is rotated back, g_j += R^T g'_j, and the
@@ -598,13 +723,13 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
 #pragma unroll
             for (int k = 0; k < 12; k++) G[k] = 0.0;
             for (int k = lane; k < NB_CL * w.count; k += 64) {
-                const int el = k >> 3, jb = k & 7;
-                const int sj = sJ[el] * NB_CL + jb;
-                const acc_t *f = &sJF[el * 3 * NB_CL + 3 * jb];
-                const double gx = isc * (double)f[0], gy = isc * (double)f[1], gz = isc * (double)f[2];
-                bad |= fx_atomic_add(facc, n_pad, sj, 0, fma(sX[0], gx, fma(sX[3], gy, sX[6] * gz)));
-                bad |= fx_atomic_add(facc, n_pad, sj, 1, fma(sX[1], gx, fma(sX[4], gy, sX[7] * gz)));
-                bad |= fx_atomic_add(facc, n_pad, sj, 2, fma(sX[2], gx, fma(sX[5], gy, sX[8] * gz)));
+                const acc_t *f = &sJ[4 * k];
+                const int sj = bits_j(f[3]) * NB_CL + (k & 7);
+                const double jsc = -fscale * isc;
+                const double gx = jsc * (double)f[0], gy = jsc * (double)f[1], gz = jsc * (double)f[2];
+                bad |= fx_atomic_add3(facc, n_pad, sj, fma(sX[0], gx, fma(sX[3], gy, sX[6] * gz)),
+                                      fma(sX[1], gx, fma(sX[4], gy, sX[7] * gz)),
+                                      fma(sX[2], gx, fma(sX[5], gy, sX[8] * gz)));
                 G[0] += gx; G[1] += gy; G[2] += gz;
                 if (moments) {
                     const double4 xr = load_slot(xq, sj);
@@ -624,34 +749,17 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                 }
             }
         }
-        // i-forces: transpose through LDS (over the records and the flushed
-        // j-force sums) so that lane 8b+a sums atom a of i-cluster c = b over
-        // the eight lanes that held its partials.
-        wave_region_sync<WPG>();
-#pragma unroll
-        for (int c = 0; c < NB_SCC; c++) {
-            sF[(3 * c + 0) * NB_SC + lane] = fx[c];
-            sF[(3 * c + 1) * NB_SC + lane] = fy[c];
-            sF[(3 * c + 2) * NB_SC + lane] = fz[c];
-        }
-        wave_region_sync<WPG>();
-        // Partials of (c, a) sit at lanes 8b' + a, b' = 0..7 (stride 8).
-        acc_t ig[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const acc_t *fr = &sF[(3 * b + k) * NB_SC + a];
-            ig[k] = ((fr[0] + fr[8]) + (fr[16] + fr[24])) + ((fr[32] + fr[40]) + (fr[48] + fr[56]));
-        }
-        const int si = (I0 + b) * NB_CL + a;
-#pragma unroll
-        for (int k = 0; k < 3; k++) bad |= fx_atomic_add(facc, n_pad, si, k, IMG ? isc * (double)ig[k] : (double)ig[k]);
-        eel = wave_sum_f64(eel);
-        elj = wave_sum_f64(elj);
-        if (lane < 2) {
+        // i-forces: lane 8b + a ends with atom a of i-cluster b.
+        const double iscale = IMG ? isc * fscale : fscale;
+        const acc_t ix = i_force(fx, lane), iy = i_force(fy, lane), iz = i_force(fz, lane);
+        bad |= fx_atomic_add3(facc, n_pad, I0 * NB_CL + lane, iscale * (double)ix, iscale * (double)iy,
+                              iscale * (double)iz);
+        // Energies: lane 0 holds the Coulomb total, lane 32 the Lennard-Jones one.
+        const double etot = wave_sum2_f64(eel, F64 ? elj : elj * (1.0 / 3.0));
+        if ((lane & 31) == 0) {
             const int slot = it & (NB_ESLOTS - 1);
-            const int kind = lane + (IMG ? 2 : 0);
-            const double v = lane == 0 ? eel : elj;
-            bad |= fx_add(eacc_word(D->eacc, kind, 0, slot), eacc_word(D->eacc, kind, 1, slot), IMG ? isc * v : v);
+            const int kind = (lane >> 5) + (IMG ? 2 : 0);
+            bad |= fx_add(eacc_word(D->eacc, kind, 0, slot), eacc_word(D->eacc, kind, 1, slot), IMG ? isc * etot : etot);
         }
         raise_error(D->err, bad, NB_ERR_RANGE);
     }

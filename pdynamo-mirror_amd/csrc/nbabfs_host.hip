@@ -202,6 +202,15 @@ static void make_factors(double damp, double inner, double outer, AbfsFactors &F
         F.bF0 = v - 0.5 * damp * g;
         F.bAlpha = -0.5 * g / damp;
     }
+    // The mixed kernel's forms: P(r2) - 1 expanded about r2On in u (r2 = r2On + (r2Off - r2On) u).
+    const long double w = (long double)r2off - r2on, on = r2on;
+    F.uScale = (double)(1.0L / w);
+    F.uShift = -(r2on * F.uScale);
+    F.sOn = 1.0 / inner;
+    F.p0 = (double)(((long double)F.a - 1.0L) - on * (F.b + on * (F.c + F.d * on)));
+    F.p1 = (double)(-w * (F.b + on * (2.0L * F.c + 3.0L * F.d * on)));
+    F.p2 = (double)(-w * w * (F.c + 3.0L * F.d * on));
+    F.p3 = (double)(-w * w * w * F.d);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2031,6 +2040,7 @@ extern "C" int nbabfs_state_create(const nbabfs_options *opt, int natoms, const 
             p[5] = -(2.0 * ak * F.aF6 + bk);
             p[6] = 2.0 * bk * F.bF3;
             p[7] = ak * F.aF6 * F.aF6 - bk * F.bF3 * F.bF3;
+            for (int q = 0; q < 8; q++) p[q] *= 3.0;     // the force's factor 3; the energy is divided by it once per item
         }
     }
     // Exclusions: symmetric CSR, ascending rows, no duplicates or self pairs

@@ -42,6 +42,9 @@ struct AbfsFactors {
     double a, b, c, d, qShift1, qShift2, qF0, qAlpha;
     double aF6, aK12, aShift12, aF0, aAlpha;
     double bF3, bK6, bShift6, bF0, bAlpha;
+    // Tiled mixed kernel: u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff and
+    // the Coulomb energy polynomial P - 1 = p0 + u (p1 + u (p2 + u p3)).
+    double uScale, uShift, sOn, p0, p1, p2, p3;
 };
 
 struct Entry {              // 80 bytes
@@ -177,6 +180,34 @@ __device__ __forceinline__ bool fx_add(long long *lo_word, long long *hi_word, d
 __device__ __forceinline__ bool fx_atomic_add(long long *facc, int n_pad, int slot, int comp, double v)
 {
     return fx_add(&facc[(size_t)comp * n_pad + slot], &facc[(size_t)(comp + 3) * n_pad + slot], v);
+}
+
+// The gradient components x, y, z of one slot.  A component below 2^15 has no
+// high word and rint(v 2^32) as its low word, the words fx_split gives, from one
+// multiply-add; the slot's words sit at 32-bit offsets from wave-uniform bases.
+// A wave with a larger (or non-finite) component takes the general split.  Slots
+// with three zero components (padding) are left alone.
+__device__ __forceinline__ bool fx_atomic_add3(long long *facc, int n_pad, int slot, double x, double y, double z)
+{
+    const double m = fabs(x) + fabs(y) + fabs(z);
+    if (__any(!(m < 32768.0))) {
+        bool bad = fx_atomic_add(facc, n_pad, slot, 0, x);
+        bad |= fx_atomic_add(facc, n_pad, slot, 1, y);
+        bad |= fx_atomic_add(facc, n_pad, slot, 2, z);
+        return bad;
+    }
+    if (m > 0.0) {
+        const double magic = 6755399441055744.0;
+        const unsigned off = (unsigned)slot * 8u;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double v = k == 0 ? x : (k == 1 ? y : z);
+            const long long lo = __double_as_longlong(fma(v, NB_FX_LO_SCALE, magic)) - __double_as_longlong(magic);
+            GAS char *base = (GAS char *)(facc + (size_t)k * n_pad);
+            __hip_atomic_fetch_add((GAS long long *)(base + off), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    return false;
 }
 
 // Error word of a system (SysDesc::err), raised by the per-call kernels and
