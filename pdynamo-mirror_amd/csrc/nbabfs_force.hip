@@ -83,7 +83,10 @@ __device__ __forceinline__ bool pair_fp64(const AbfsFactors &F, double r2, doubl
 //   * Coulomb energy: s + sc (P - 1) + qShift2 with sc = min(s, 1/inner) and
 //     P - 1 = (a - 1) - r2 (b + r2 (c + d r2)) as a cubic in u.  In the plain
 //     region sc (P - 1) + qShift2 is the constant qShift1 (the reference's
-//     energies meet at the inner cutoff), so no region is selected.
+//     energies meet at the inner cutoff), so no region is selected.  The cubic's
+//     leading coefficient is divided out of all of it (eel is E / eScale, scaled
+//     back with the item's total), so every step has at most one constant, which
+//     is all an instruction can take from scalar registers.
 //   * Lennard-Jones in both undamped regions is one polynomial in s = 1/r,
 //       E = C12 s^12 + C6 s^6 + C3 s^3 + C0,
 //     whose coefficients per type pair and region come from a row table (plain:
@@ -108,7 +111,7 @@ __device__ __forceinline__ double min_uniform(double x, double s)
     return r;
 }
 
-__device__ __forceinline__ void pair_rows(const AbfsFactors &F, double p3, double r2, double u, double qq, double4 C,
+__device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, double u, double qq, double4 C,
                                           unsigned long long mact, const GAS double *__restrict__ ljA,
                                           const GAS double *__restrict__ ljB, int off, double &fs, double &eel,
                                           double &elj)
@@ -119,23 +122,23 @@ __device__ __forceinline__ void pair_rows(const AbfsFactors &F, double p3, doubl
     const double s2 = s * s;
     const double s3 = s2 * s;
     const double s6 = s3 * s3;
-    const double Q = fma(u * u, fma(2.0, u, -3.0), 1.0);
+    const double Q = fma(u * u, fma(2.0, u, F.minus3), 1.0);
     const double sc = min_uniform(s, F.sOn);
-    const double pm1 = fma(fma(fma(p3, u, F.p2), u, F.p1), u, F.p0);
-    double e1 = qq * (s + fma(sc, pm1, F.qShift2));
+    const double pm1 = fma(fma(u + F.p2, u, F.p1), u, F.p0);
+    double e1 = qq * fma(s, F.eInv, fma(sc, pm1, F.qShift2e));
     // inner = s^3 (4 C12 s^6 + 2 C6) + C3 = 2 s^3 (C12 s^6 + t1) + C3, t1 = C12 s^6 + C6.
     const double t1 = fma(C.x, s6, C.y);
     double e2 = fma(t1, s6, fma(C.z, s3, C.w));
     const double inner = fma(s3 + s3, fma(C.x, s6, t1), C.z);
     // Minus twice dE/d(r^2): Coulomb qq s^3 Q, Lennard-Jones 3 s^5 inner (the rows' factor 3).
     double f = s3 * fma(s2, inner, qq * Q);
-    if (__builtin_amdgcn_ballot_w64(r2 < F.r2Damp) & mact) {
-        if (r2 < F.r2Damp) {
-            const double A = ljA[off >> 6], B = ljB[off >> 6];
-            e1 = qq * fma(-F.qAlpha, r2, F.qF0);
-            e2 = 3.0 * (A * fma(-F.aAlpha, r2, F.aF0) - B * fma(-F.bAlpha, r2, F.bF0));
-            f = 2.0 * (qq * F.qAlpha + (A * F.aAlpha - B * F.bAlpha));
-        }
+    // A branch of the whole wave (its lanes select), so the usual path has no execution-mask bookkeeping.
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(r2 < F.r2Damp) & mact) != 0ull, 0)) {
+        const bool damped = r2 < F.r2Damp;
+        const double A = ljA[off >> 6], B = ljB[off >> 6];
+        e1 = damped ? qq * fma(F.qAlphaE, r2, F.qF0e) : e1;
+        e2 = damped ? 3.0 * (A * fma(-F.aAlpha, r2, F.aF0) - B * fma(-F.bAlpha, r2, F.bF0)) : e2;
+        f = damped ? 2.0 * (qq * F.qAlpha + (A * F.aAlpha - B * F.bAlpha)) : f;
     }
     fs = f;
     eel = e1;
@@ -298,6 +301,16 @@ __device__ __forceinline__ void pairs14_block(const SysDesc &D, const AbfsFactor
 // fetched while the current one is evaluated.
 // ------------------------------------------------------------------------------------------------
 
+// A value read from LDS at an address the caller has made a 32-bit LDS one.
+#define LAS __attribute__((address_space(3)))
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ double4 lds_record(const LAS char *p)
+{
+    const f64x2 u = *(const LAS f64x2 *)p, v = *(const LAS f64x2 *)(p + 16);
+    return make_double4(u.x, u.y, v.x, v.y);
+}
+
 __device__ __forceinline__ double4 load_slot(const GAS double *__restrict__ xr, int k)
 {
     return make_double4(xr[4 * k], xr[4 * k + 1], xr[4 * k + 2], xr[4 * k + 3]);
@@ -306,8 +319,10 @@ __device__ __forceinline__ double4 load_slot(const GAS double *__restrict__ xr, 
 // The j-cluster's records and types: a wave-uniform base plus a 32-bit lane offset.
 __device__ __forceinline__ double4 load_j(const GAS double *__restrict__ xr, int J, unsigned off)
 {
+    // The uniform part of the address stays in scalar registers and the lane's 32-bit offset in one vector register
+    // (a 64-bit lane offset hoisted out of the entry loop would cost a register pair and an addition per load).
     unsigned long long base = (unsigned long long)(xr + (size_t)J * (4 * NB_CL));
-    asm("" : "+s"(base));      // keeps the uniform part of the address in scalar registers
+    asm volatile("" : "+s"(base), "+v"(off));
     const GAS double *p = (const GAS double *)((const GAS char *)base + off);
     return make_double4(p[0], p[1], p[2], p[3]);
 }
@@ -315,23 +330,28 @@ __device__ __forceinline__ double4 load_j(const GAS double *__restrict__ xr, int
 __device__ __forceinline__ int load_jtype(const GAS int *__restrict__ ty, int J, unsigned off)
 {
     unsigned long long base = (unsigned long long)(ty + (size_t)J * NB_CL);
-    asm("" : "+s"(base));
+    asm volatile("" : "+s"(base), "+v"(off));
     return *(const GAS int *)((const GAS char *)base + off);
 }
 
-// Entry fields through the vector memory path: J and cbits are read by every
-// lane from one address (one request) and made uniform; each lane reads its
-// own tile-mask byte (64 consecutive bytes per entry).
-__device__ __forceinline__ int2 entry_jc(const GAS unsigned char *__restrict__ eb, int e)
+// Entry fields through the vector memory path: one load brings the header's
+// words (lanes 8b .. 8b + 7 read word b, off = 4 b: the lane offset the j-atom
+// types use), of which J (word 0) and cbits (word 2) are read back from their
+// lanes; each lane reads its own tile-mask byte (64 consecutive bytes per entry).
+__device__ __forceinline__ int entry_header(const GAS unsigned char *__restrict__ eb, int e, unsigned off)
 {
-    const GAS int *p = (const GAS int *)(eb + (size_t)e * sizeof(Entry));
-    return make_int2(p[0], p[2]);
+    unsigned long long base = (unsigned long long)(eb + (size_t)e * sizeof(Entry));
+    asm volatile("" : "+s"(base), "+v"(off));
+    return *(const GAS int *)((const GAS char *)base + off);
 }
+
+__device__ __forceinline__ int header_j(int h) { return __builtin_amdgcn_readlane(h, 0); }
+__device__ __forceinline__ int header_cbits(int h) { return __builtin_amdgcn_readlane(h, 16); }
 
 __device__ __forceinline__ int entry_bits(const GAS unsigned char *__restrict__ eb, int e, unsigned lane)
 {
     unsigned long long base = (unsigned long long)(eb + (size_t)e * sizeof(Entry));
-    asm("" : "+s"(base));
+    asm volatile("" : "+s"(base), "+v"(lane));
     return ((const GAS unsigned char *)base + 16)[lane];
 }
 
@@ -452,7 +472,8 @@ __device__ __forceinline__ T i_force(T (&f)[NB_SCC], int lane)
 // wave: the item's i-cluster records and slot types, then one record per entry
 // and j-atom (the three j-force sums and the j-cluster), flushed to the
 // fixed-point accumulators once at the end of the item.
-#define NB_LDS_I_BYTES (NB_SC * 32 + NB_SC * 4)
+#define NB_LDS_IREC 48          // x, y, z, q and the type's row offset, padded
+#define NB_LDS_I_BYTES (NB_SC * NB_LDS_IREC)
 #define NB_LDS_ROW_LIMIT 16384
 #define NB_LDS_GROUP_LIMIT (160 * 1024 / 4)
 
@@ -478,11 +499,13 @@ __device__ __forceinline__ void wave_region_sync()
     }
 }
 
-// Four waves per SIMD: the register allocator fits the kernel in 128 VGPRs
-// without spilling (137 unconstrained, three waves), measured 2-3% faster.
-// IMG: the launch over the image lists' work items (the main list's items run
-// in an instance without any image code); it runs at three waves per SIMD,
-// whose register budget holds the transformation without spilling.
+// Waves per SIMD.  A tile is a chain of two LDS reads and about forty dependent FP64 instructions, so the issue slots
+// fill only with enough waves: five fit in 96 VGPRs, with no spill inside the entry loop, because the loop holds no
+// 64-bit lane offsets, one LDS address for all tiles (records at a 16-byte-aligned stride with the type beside the
+// charge), header words of one load, FP32 copies of dx, dy, dz across the pair terms and no polynomial factor in vector
+// registers.  16-image batch: 680 us per call with three waves, 620 with four, 603 with five (647 before, four waves).
+// IMG: the launch over the image lists' work items (the main list's items run in an instance without any image code);
+// it runs at three waves per SIMD, whose register budget holds the transformation without spilling.
 // F64: the full-FP64 instance (the NBABFS_TILED_FP64 comparison path): the same list, tiles, staging and
 // fixed-point sums, with the reference's FP64 pair arithmetic (pair_fp64: divide and square root, no FP32
 // seed, raw A and B per type pair) and FP64 force vectors; three waves per SIMD for its larger accumulators.
@@ -493,7 +516,7 @@ __device__ __forceinline__ void wave_region_sync()
 // with empty ones).  Image items and the persistent queues run one wave per
 // group.
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG || F64) ? 3 : 4))) void k_force_tiled(
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG || F64) ? 3 : 5))) void k_force_tiled(
     const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, AbfsFactors F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
@@ -526,8 +549,6 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
     using acc_t = typename std::conditional<F64, double, float>::type;
     double4 *sR = (double4 *)lds;
     unsigned char *region = lds + rows_bytes + (size_t)wave * wave_bytes;
-    double4 *sI = (double4 *)region;
-    int *sT = (int *)(region + NB_SC * 32);
     acc_t *sJ = (acc_t *)(region + NB_LDS_I_BYTES);   // [entry][j-atom] of (x, y, z, J)
     // The group's row table, staged once when the items are one per wave.
     int rows_sys = -1;
@@ -602,20 +623,26 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         const int e_last = w.first + w.count - 1;
         const double4 irec = load_slot(xq, I0 * NB_CL + lane);
         const int ityp = ty[I0 * NB_CL + lane];
-        int2 jc0 = entry_jc(eb, w.first);
-        int lb0 = entry_bits(eb, w.first, bl);
-        int2 jc1 = entry_jc(eb, min(w.first + 1, e_last));
-        int lb1 = entry_bits(eb, min(w.first + 1, e_last), bl);
+        const unsigned jrec = 32u * b, jtyp = 4u * b;      // byte offsets in a j-cluster's records and types
+        const int h0 = entry_header(eb, w.first, jtyp);
+        int lbn = entry_bits(eb, w.first, bl);
+        int hn = entry_header(eb, min(w.first + 1, e_last), jtyp);
 
         // A persistent wave's region still holds its previous item's data until every lane is past it.
         if (qp.heads != nullptr) wave_region_sync<WPG>();
         if (IMG && lane < 12) sX[lane] = X[lane];
         if (ROWS_LDS && rows_sys < 0)
             for (int k = lane; k < 2 * nt * nt; k += 64) sR[k] = load_slot(rows, k);
-        sI[lane] = irec;
-        sT[lane] = 64 * nt * ityp;   // byte offset of the type's first row pair
-        int J = __builtin_amdgcn_readfirstlane(jc0.x);
-        const unsigned jrec = 32u * b, jtyp = 4u * b;      // byte offsets in a j-cluster's records and types
+        {
+            double *r = (double *)(region + NB_LDS_IREC * lane);
+            r[0] = irec.x;
+            r[1] = irec.y;
+            r[2] = irec.z;
+            r[3] = irec.w;
+            *(int *)(r + 4) = 64 * nt * ityp;   // byte offset of the type's first row pair
+        }
+        int J = header_j(h0);
+        int cbn = header_cbits(h0);
         double4 xj = load_j(xq, J, jrec);
         int tj = 64 * load_jtype(ty, J, jtyp);
         const int comp = min(a, NB_CL - 1 - a);
@@ -626,17 +653,21 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
 #pragma unroll
         for (int c = 0; c < NB_SCC; c++) fx[c] = fy[c] = fz[c] = (acc_t)0;
         // Two factors kept in vector registers: their multiply-adds already read one scalar operand.
-        double uShift = F.uShift, p3 = F.p3;
-        asm("" : "+v"(uShift), "+v"(p3));
+        double uShift = F.uShift;
+        asm("" : "+v"(uShift));
         double eel = 0.0, elj = 0.0;
+        // The i-records are read at constant offsets from one address per lane (the compiler would keep one per tile).
+        const LAS char *ip = (const LAS char *)(region + NB_LDS_IREC * a);
+        asm("" : "+v"(ip));
         for (int e = w.first; e <= e_last; e++) {
-            const int Jn = __builtin_amdgcn_readfirstlane(jc1.x);
+            // Entry e + 1's cluster and mask were asked for one entry ago, its header two entries ago.
+            const int cb = cbn, lb = lbn;
+            const int Jn = header_j(hn);
+            cbn = header_cbits(hn);
             const double4 xjn = load_j(xq, Jn, jrec);
             const int tjn = 64 * load_jtype(ty, Jn, jtyp);
-            const int2 jc2 = entry_jc(eb, min(e + 2, e_last));
-            const int lb2 = entry_bits(eb, min(e + 2, e_last), bl);
-            const int cb = __builtin_amdgcn_readfirstlane(jc0.y);
-            const int lb = lb0;
+            hn = entry_header(eb, min(e + 2, e_last), jtyp);
+            lbn = entry_bits(eb, min(e + 1, e_last), bl);
             // Image items: the j-atom's image position (its load was issued one entry earlier).
             const double4 xjt = IMG ? image_slot(xj, sX) : xj;
             acc_t gx = (acc_t)0, gy = (acc_t)0, gz = (acc_t)0;
@@ -644,7 +675,10 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
             for (int c = 0; c < NB_SCC; c++) {
                 if (cb & (1 << c)) {
                     const bool inl = (lb & (1 << c)) != 0;
-                    const double4 xi = sI[c * NB_CL + a];
+                    double4 xi = lds_record(ip + c * NB_CL * NB_LDS_IREC);
+                    int ti = *(const LAS int *)(ip + c * NB_CL * NB_LDS_IREC + 32);
+                    // The charge and type are read with the position, not after the branch below: one LDS wait per tile.
+                    asm("" : "+v"(xi.w), "+v"(ti));
                     const double dx = xi.x - xjt.x, dy = xi.y - xjt.y, dz = xi.z - xjt.z;
                     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
                     const bool inr = r2 <= F.r2Off;
@@ -653,8 +687,8 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                     const unsigned long long mact = __builtin_amdgcn_ballot_w64(inl) & __builtin_amdgcn_ballot_w64(inr);
                     const bool act = __builtin_amdgcn_inverse_ballot_w64(mact);
                     if (mact != 0ull) {
-                        // Byte offset of the pair's plain row.
-                        const int ti = sT[c * NB_CL + a];
+                        float px = (float)dx, py = (float)dy, pz = (float)dz;
+                        if (!F64) asm("" : "+v"(px), "+v"(py), "+v"(pz));   // three registers across the pair terms, not six
                         if (F64) {
                             // PairwiseInteraction.h:72-119 in FP64 with the reference's operations.
                             if (act) {
@@ -673,10 +707,10 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                             const double4 C = ROWS_LDS ? *(const double4 *)((const unsigned char *)sR + off)
                                                        : load_slot(rows, off >> 5);
                             double fs, x1, x2;
-                            pair_rows(F, p3, r2, u, xi.w * xjt.w, C, mact, ljA, ljB, off, fs, x1, x2);
+                            pair_rows(F, r2, u, xi.w * xjt.w, C, mact, ljA, ljB, off, fs, x1, x2);
                             // The sums take the active lanes only (the others may hold any value).
                             if (act) {
-                                const float f = (float)fs, px = (float)dx, py = (float)dy, pz = (float)dz;
+                                const float f = (float)fs;
                                 fx[c] = fmaf(f, px, (float)fx[c]);
                                 fy[c] = fmaf(f, py, (float)fy[c]);
                                 fz[c] = fmaf(f, pz, (float)fz[c]);
@@ -693,10 +727,6 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
             const acc_t rec = j_record(gx, gy, gz, J, comp);
             // Lanes a and 7 - a hold the same value.
             sJ[(e - w.first) * 4 * NB_CL + 4 * b + comp] = rec;
-            jc0 = jc1;
-            lb0 = lb1;
-            jc1 = jc2;
-            lb1 = lb2;
             J = Jn;
             xj = xjn;
             tj = tjn;
@@ -755,7 +785,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         bad |= fx_atomic_add3(facc, n_pad, I0 * NB_CL + lane, iscale * (double)ix, iscale * (double)iy,
                               iscale * (double)iz);
         // Energies: lane 0 holds the Coulomb total, lane 32 the Lennard-Jones one.
-        const double etot = wave_sum2_f64(eel, F64 ? elj : elj * (1.0 / 3.0));
+        const double etot = wave_sum2_f64(F64 ? eel : eel * F.eScale, F64 ? elj : elj * (1.0 / 3.0));
         if ((lane & 31) == 0) {
             const int slot = it & (NB_ESLOTS - 1);
             const int kind = (lane >> 5) + (IMG ? 2 : 0);
@@ -1181,7 +1211,8 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
     const dim3 grid(ngroups + nblk(n14_blocks, wpg));
     const int acc = full_fp64 ? 8 : 4;
     const int wave_bytes = (int)tiled_lds_wave(max_count, acc);
-    // The row table goes to LDS when the group's LDS still lets four groups of four waves (or ten single waves) share a CU.
+    // The row table goes to LDS when the group's LDS still lets four groups of four waves (or ten single waves) share a CU
+    // (five groups do up to 32 KB: ten types with 16 entries per wave take 27 KB).
     const size_t limit = wpg == 1 ? NB_LDS_ROW_LIMIT : NB_LDS_GROUP_LIMIT;
     const bool rows_lds = !full_fp64 && tiled_lds_rows(max_ntypes, true) + (size_t)wpg * wave_bytes <= limit;
     const int rows_bytes = (int)tiled_lds_rows(max_ntypes, rows_lds);

@@ -207,10 +207,16 @@ static void make_factors(double damp, double inner, double outer, AbfsFactors &F
     F.uScale = (double)(1.0L / w);
     F.uShift = -(r2on * F.uScale);
     F.sOn = 1.0 / inner;
-    F.p0 = (double)(((long double)F.a - 1.0L) - on * (F.b + on * (F.c + F.d * on)));
-    F.p1 = (double)(-w * (F.b + on * (2.0L * F.c + 3.0L * F.d * on)));
-    F.p2 = (double)(-w * w * (F.c + 3.0L * F.d * on));
-    F.p3 = (double)(-w * w * w * F.d);
+    const long double p3 = -w * w * w * F.d;       // the leading coefficient, divided out of the others
+    F.p0 = (double)((((long double)F.a - 1.0L) - on * (F.b + on * (F.c + F.d * on))) / p3);
+    F.p1 = (double)(-w * (F.b + on * (2.0L * F.c + 3.0L * F.d * on)) / p3);
+    F.p2 = (double)(-w * w * (F.c + 3.0L * F.d * on) / p3);
+    F.eScale = (double)p3;
+    F.eInv = (double)(1.0L / p3);
+    F.qShift2e = (double)((long double)F.qShift2 / p3);
+    F.qF0e = (double)((long double)F.qF0 / p3);
+    F.qAlphaE = (double)(-(long double)F.qAlpha / p3);
+    F.minus3 = -3.0;
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -42,9 +42,10 @@ struct AbfsFactors {
     double a, b, c, d, qShift1, qShift2, qF0, qAlpha;
     double aF6, aK12, aShift12, aF0, aAlpha;
     double bF3, bK6, bShift6, bF0, bAlpha;
-    // Tiled mixed kernel: u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff and
-    // the Coulomb energy polynomial P - 1 = p0 + u (p1 + u (p2 + u p3)).
-    double uScale, uShift, sOn, p0, p1, p2, p3;
+    // Tiled mixed kernel: u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff, and the
+    // Coulomb energy divided by eScale, the leading coefficient of P - 1 = eScale (p0 + u (p1 + u (p2 + u))).
+    double uScale, uShift, sOn, p0, p1, p2, eScale, eInv, qShift2e, qF0e, qAlphaE;
+    double minus3;              // -3 (an operand in scalar registers, not a pair of vector registers)
 };
 
 struct Entry {              // 80 bytes
