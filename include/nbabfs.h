@@ -49,7 +49,7 @@ extern "C" {
                                  vectors: the mixed path without its FP32 parts
                                  (no image lists)                                    */
 
-/* Upper bound of nbabfs_options.entriesPerItem (per-item j-force staging in LDS). */
+/* Upper bound of nbabfs_options.entriesPerItem. */
 #define NBABFS_MAX_ENTRIES_PER_ITEM 128
 
 typedef struct nbabfs_state nbabfs_state;
@@ -70,7 +70,8 @@ typedef struct {
     int    minimumPoints;          /* 500  */
     int    precision;              /* NBABFS_MIXED, NBABFS_PLAIN_FP64 or NBABFS_TILED_FP64 */
     int    entriesPerItem;         /* cluster-pair entries per work item (0 = 16, at most
-                                      NBABFS_MAX_ENTRIES_PER_ITEM) */
+                                      NBABFS_MAX_ENTRIES_PER_ITEM): average entries of a dense
+                                      system; items are cut by cost, small lists finer */
     int    wavesPerCU;             /* persistent-kernel waves per CU; 0 = one workgroup per work item */
     int    imageEntriesPerItem;    /* entries per work item of the image lists (0 = 16) */
     int    useGridByCell;          /* 1 (the ABFS default): grid search cell by cell

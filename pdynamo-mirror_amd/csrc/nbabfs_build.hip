@@ -16,6 +16,8 @@
 
 #include <float.h>
 
+#include <algorithm>
+
 // ------------------------------------------------------------------------------------------------
 // Bounding box (Coordinates3_EnclosingOrthorhombicBox, pCore-1.9.0/extensions/csource/
 // Coordinates3.c:498-605).  Min/max are order independent, so a tree is exact.
@@ -433,10 +435,11 @@ __device__ __forceinline__ JAtom load_jatom_cross(int J, int b, const double *__
     return r;
 }
 
-// Write candidate k's entry (scratch slot base + k); returns 1 if it lists a pair.
+// Write candidate k's entry (scratch slot base + k); returns 1 if it lists a pair, and adds the entry's cost.
 __device__ __forceinline__ int search_store(Entry *__restrict__ scratch, size_t sbase, int slot, int scap, int lane,
-                                            int Jc, int sc, int img, int lbits, int cbits)
+                                            int Jc, int sc, int img, int lbits, int cbits, int &ncost)
 {
+    ncost += entry_cost(cbits);
     if (slot < scap) {
         Entry *en = &scratch[sbase + slot];
         en->bits[lane] = (unsigned char)lbits;
@@ -466,7 +469,8 @@ __device__ __forceinline__ int search_eval_cross(const SearchParams &P, int npen
                                                  const unsigned char *sCm, const int *sIatom, const int *sIfree,
                                                  const int4 *sIcell, const double *sIx, const double *sIy,
                                                  const double *sIz, const ImageGrid &G, const double *__restrict__ jxyz,
-                                                 const int *__restrict__ slot_atom, Entry *__restrict__ scratch)
+                                                 const int *__restrict__ slot_atom, Entry *__restrict__ scratch,
+                                                 int &ncost)
 {
     const int a = lane >> 3, b = lane & 7;
     const int wst = 2 * P.u + 1;
@@ -526,7 +530,7 @@ __device__ __forceinline__ int search_eval_cross(const SearchParams &P, int npen
             if (ok) lbits |= 1 << c;
             if (__ballot(ok)) cbits |= 1 << c;
         }
-        nvalid += search_store(scratch, sbase, base + k, scap, lane, Jc, sc, img, lbits, cbits);
+        nvalid += search_store(scratch, sbase, base + k, scap, lane, Jc, sc, img, lbits, cbits, ncost);
     }
     return nvalid;
 }
@@ -550,7 +554,7 @@ __device__ __forceinline__ int search_eval_self(const SearchParams &P, int npend
                                                 const unsigned char *sCm, const double4 *sIp, const int4 *sIc,
                                                 const int2 *sIxr, const int *sXoff, const int *sXcnt,
                                                 const int *sXpool, const unsigned char *sSten,
-                                                Entry *__restrict__ scratch)
+                                                Entry *__restrict__ scratch, int &ncost)
 {
     const int a = lane >> 3, b = lane & 7;
     const unsigned wst = 2 * P.u + 1, nst = wst * wst * wst;
@@ -626,7 +630,7 @@ __device__ __forceinline__ int search_eval_self(const SearchParams &P, int npend
             lbits |= ok ? (1 << c) : 0;
             if (__ballot(ok)) cbits |= 1 << c;
         }
-        nvalid += search_store(scratch, sbase, base + k, scap, lane, Jc, sc, -1, lbits, cbits);
+        nvalid += search_store(scratch, sbase, base + k, scap, lane, Jc, sc, -1, lbits, cbits, ncost);
     }
     return nvalid;
 }
@@ -646,7 +650,8 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
                                                               const float4 *__restrict__ bhi,
                                                               const int2 *__restrict__ colcl,
                                                               Entry *__restrict__ scratch, int *__restrict__ ncand,
-                                                              int *__restrict__ counts, int *__restrict__ overflow)
+                                                              int *__restrict__ counts, int *__restrict__ costs,
+                                                              int *__restrict__ overflow)
 {
     const int sc = blockIdx.x;
     const int img = CROSS ? (int)blockIdx.y : -1;
@@ -676,7 +681,7 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
     __shared__ int sCand[NB_CAND];
     __shared__ unsigned char sCm[NB_CAND];
     __shared__ int sColStart[NB_MAXCOL], sColPre[NB_MAXCOL + 1];
-    __shared__ int sWcnt[NB_SEARCH_WAVES];
+    __shared__ int sWcnt[NB_SEARCH_WAVES], sWcost[NB_SEARCH_WAVES];
 
     // Stage the super-cluster (wave 0) and the stencil (all waves).
     if (w == 0) {
@@ -734,7 +739,7 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
         lo.x = fminf(lo.x, sIlo[c].x); lo.y = fminf(lo.y, sIlo[c].y); lo.z = fminf(lo.z, sIlo[c].z);
         hi.x = fmaxf(hi.x, sIhi[c].x); hi.y = fmaxf(hi.y, sIhi[c].y); hi.z = fmaxf(hi.z, sIhi[c].z);
     }
-    int nvalid = 0;      // entries written by this wave
+    int nvalid = 0, ncost = 0;      // entries written by this wave, their cost
     int base = 0;        // candidates handed out before the current list
     if (lo.x <= hi.x) {  // super-cluster holds at least one atom (uniform over the block)
         const float reach = P.reach;
@@ -765,10 +770,10 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
         auto evaluate = [&](int npend) {
             if (CROSS)
                 nvalid += search_eval_cross<PC>(P, npend, w, lane, I0, sc, img, base, scap, sbase, sCand, sCm, sIatom,
-                                                sIfree, sIcell, sIx, sIy, sIz, G, jxyz, slot_atom, scratch);
+                                                sIfree, sIcell, sIx, sIy, sIz, G, jxyz, slot_atom, scratch, ncost);
             else
                 nvalid += search_eval_self<STEN, PC>(P, npend, w, lane, I0, sc, base, scap, sbase, sCand, sCm, sIp, sIc,
-                                                 sIxr, sXoff, sXcnt, sXpool, sSten, scratch);
+                                                 sIxr, sXoff, sXcnt, sXpool, sSten, scratch, ncost);
         };
 
         int npend = 0;
@@ -857,34 +862,37 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
         evaluate(npend);
         base += npend;
     }
-    if (lane == 0) sWcnt[w] = nvalid;
+    if (lane == 0) {
+        sWcnt[w] = nvalid;
+        sWcost[w] = ncost;
+    }
     __syncthreads();
     if (tid == 0) {
-        int tot = 0;
-        for (int v = 0; v < NB_SEARCH_WAVES; v++) tot += sWcnt[v];
+        int tot = 0, cost = 0;
+        for (int v = 0; v < NB_SEARCH_WAVES; v++) {
+            tot += sWcnt[v];
+            cost += sWcost[v];
+        }
         counts[blk] = tot;
+        costs[blk] = cost;
         ncand[blk] = base;
         if (base > scap) atomicMax(overflow, base);
     }
 }
 
 // Compact per-super-cluster entries (candidate slots with any listed pair, in
-// candidate order), count their pairs into *npairs (or per block), and cut
-// them into work items.  Block b compacts search block b, whose
-// super-cluster is b % nsc.
+// candidate order) and count their pairs per block.  Block b compacts search
+// block b, whose super-cluster is b % nsc.
 #define NB_COMPACT_THREADS 256
 __global__ __launch_bounds__(NB_COMPACT_THREADS) void k_compact(const Entry *__restrict__ scratch, int cap,
                                                                 const int *__restrict__ soff,
                                                                 const int *__restrict__ ncand,
-                                                                const int *__restrict__ counts,
                                                                 const int *__restrict__ eoff,
-                                                                const int *__restrict__ ioff, int nsc, int per_item,
-                                                                int sys, Entry *__restrict__ entries,
-                                                                WorkItem *__restrict__ items,
+                                                                Entry *__restrict__ entries,
                                                                 unsigned long long *__restrict__ npairs_block)
 {
     const int sc = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int nc = soff ? ncand[sc] : min(ncand[sc], cap), cnt = counts[sc], e0 = eoff[sc], i0 = ioff[sc];
+    const int nc = soff ? ncand[sc] : min(ncand[sc], cap), e0 = eoff[sc];
     const Entry *__restrict__ src = scratch + (soff ? (size_t)soff[sc] : (size_t)sc * cap);
     __shared__ int sW[NB_COMPACT_THREADS / 64];
     __shared__ unsigned long long sP[NB_COMPACT_THREADS / 64];
@@ -927,200 +935,133 @@ __global__ __launch_bounds__(NB_COMPACT_THREADS) void k_compact(const Entry *__r
         for (int v = 0; v < NB_COMPACT_THREADS / 64; v++) t += sP[v];
         npairs_block[sc] = t;
     }
-    const int nit = (cnt + per_item - 1) / per_item;
-    for (int k = tid; k < nit; k += NB_COMPACT_THREADS) {
-        WorkItem wi;
-        wi.sys = sys;
-        if (soff) wi.sys |= (sc / nsc + 1) << 16;   // image lists: image of the block, plus one
-        wi.sc = sc % nsc;
-        wi.first = e0 + k * per_item;
-        wi.count = min(per_item, cnt - k * per_item);
-        items[i0 + k] = wi;
-    }
 }
 
-// Longest-first order of the work items (by the number of i-cluster tiles of
-// their entries), so that the items still running when the GPU drains are the
-// short ones.  Results do not depend on the order: every sum is fixed point.
-__global__ __launch_bounds__(256) void k_item_cost(const WorkItem *__restrict__ items, int nitems,
-                                                   const Entry *__restrict__ entries, int maxcost,
-                                                   int *__restrict__ cost, int *__restrict__ hist)
+// Work items of a compacted list: the entries of block s (a super-cluster, or
+// an (image, super-cluster) block of the image lists: images != 0, each item's
+// sys field then carries (image + 1) << 16) are cut at equal steps of their
+// summed cost into the block's n items.  Entry i starts item q when its
+// exclusive cost prefix p reaches q's step, q = p n / C; a step is longer than
+// any entry's cost (NB_MIN_ITEM_COST), so no item is empty.
+__global__ __launch_bounds__(256) void k_cut_items(const int *__restrict__ counts, const int *__restrict__ costs,
+                                                   const int *__restrict__ eoff, const int *__restrict__ ioff,
+                                                   const int *__restrict__ nits, int nsc, int sys, int images,
+                                                   const Entry *__restrict__ entries, WorkItem *__restrict__ items)
 {
-    // One wavefront per item: its lanes read the entries' i-cluster masks.
-    const int k = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (k >= nitems) return;
-    const WorkItem w = items[k];
-    int c = 0;
-    for (int e = w.first + lane; e < w.first + w.count; e += 64) c += __popc(entries[e].cbits & 0xff);
-    for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o, 64);
-    c = min(c, maxcost);
-    if (lane == 0) {
-        cost[k] = c;
-        if (hist) atomicAdd(&hist[maxcost - c], 1);
-    }
-}
-
-// Rank r in the longest-first order goes to position r, or, for the
-// persistent queues (interleave != 0), to queue r % 8 at place r / 8, so every
-// per-XCD queue is itself longest-first and the queues are balanced.
-__device__ __forceinline__ int queue_start(int nitems, int q)
-{
-    int s = 0;
-    for (int v = 0; v < q; v++) s += (nitems - v + 7) / 8;
-    return s;
-}
-
-// Longest-first order in one workgroup: histogram of the costs, its scan and
-// the scatter all in LDS.  Most items share a few costs, so the histogram is
-// kept in NB_ORDER_COPIES copies (wave w adds into copy w % NB_ORDER_COPIES)
-// to spread the atomics on a hot bin; the scan runs over (bin, copy) in that
-// order.  Items of equal cost keep no particular order.
-#define NB_ORDER_THREADS 1024
-#define NB_ORDER_BINS 2048
-#define NB_ORDER_COPIES 4
-#define NB_ORDER_UNROLL 8
-__global__ __launch_bounds__(NB_ORDER_THREADS) void k_item_order(const WorkItem *__restrict__ items, int nitems,
-                                                                 const int *__restrict__ cost, int maxcost,
-                                                                 int interleave, WorkItem *__restrict__ out)
-{
-    __shared__ int sH[NB_ORDER_BINS * NB_ORDER_COPIES];    // [bin][copy]
-    __shared__ int sW[NB_ORDER_THREADS / 64];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, cp = w % NB_ORDER_COPIES;
-    for (int b = t; b < NB_ORDER_BINS * NB_ORDER_COPIES; b += NB_ORDER_THREADS) sH[b] = 0;
-    __syncthreads();
-    // The loads of a pass are issued together (indices clamped, so none is conditional).
-    for (int k0 = t; k0 < nitems; k0 += NB_ORDER_UNROLL * NB_ORDER_THREADS) {
-        int cc[NB_ORDER_UNROLL];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int cnt = counts[s], total = costs[s], e0 = eoff[s], n = nits[s];
+    if (cnt <= 0) return;
+    WorkItem *own = items + ioff[s];
+    __shared__ int sW[4];
+    int carry = 0;      // cost of the chunks before this one
+    for (int k0 = 0; k0 < cnt; k0 += 256) {
+        const int k = k0 + tid;
+        const int c = k < cnt ? entry_cost(entries[e0 + k].cbits) : 0;
+        int incl = c;
 #pragma unroll
-        for (int u = 0; u < NB_ORDER_UNROLL; u++) cc[u] = cost[min(k0 + u * NB_ORDER_THREADS, nitems - 1)];
-#pragma unroll
-        for (int u = 0; u < NB_ORDER_UNROLL; u++)
-            if (k0 + u * NB_ORDER_THREADS < nitems) atomicAdd(&sH[(maxcost - cc[u]) * NB_ORDER_COPIES + cp], 1);
-    }
-    __syncthreads();
-    // Exclusive scan over (bin, copy): eight consecutive counters per thread.
-    constexpr int PER = NB_ORDER_BINS * NB_ORDER_COPIES / NB_ORDER_THREADS;
-    int h[PER], sum = 0;
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-        h[q] = sH[PER * t + q];
-        sum += h[q];
-    }
-    int incl = sum;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += v;
-    }
-    if (lane == 63) sW[w] = incl;
-    __syncthreads();
-    int ex = incl - sum;
-    for (int v = 0; v < w; v++) ex += sW[v];
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-        sH[PER * t + q] = ex;
-        ex += h[q];
-    }
-    __syncthreads();
-    for (int k0 = t; k0 < nitems; k0 += NB_ORDER_UNROLL * NB_ORDER_THREADS) {
-        int cc[NB_ORDER_UNROLL];
-        int4 wi[NB_ORDER_UNROLL];
-#pragma unroll
-        for (int u = 0; u < NB_ORDER_UNROLL; u++) {
-            const int k = min(k0 + u * NB_ORDER_THREADS, nitems - 1);
-            cc[u] = cost[k];
-            wi[u] = ((const int4 *)items)[k];
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
         }
-        int r[NB_ORDER_UNROLL];
-#pragma unroll
-        for (int u = 0; u < NB_ORDER_UNROLL; u++)
-            r[u] = k0 + u * NB_ORDER_THREADS < nitems ? atomicAdd(&sH[(maxcost - cc[u]) * NB_ORDER_COPIES + cp], 1) : -1;
-#pragma unroll
-        for (int u = 0; u < NB_ORDER_UNROLL; u++)
-            if (r[u] >= 0) ((int4 *)out)[interleave ? queue_start(nitems, r[u] & 7) + (r[u] >> 3) : r[u]] = wi[u];
+        if (lane == 63) sW[w] = incl;
+        __syncthreads();
+        int before = carry;
+        for (int v = 0; v < 4; v++) {
+            if (v < w) before += sW[v];
+            carry += sW[v];
+        }
+        const int p = before + incl - c;
+        if (k < cnt) {
+            // q of this entry and of the one before it (whose prefix is p minus its own cost: only the step matters).
+            const int q = (int)((long long)p * n / total);
+            const int cp = k > 0 ? entry_cost(entries[e0 + k - 1].cbits) : 0;
+            const int qp = k > 0 ? (int)((long long)(p - cp) * n / total) : -1;
+            if (q != qp) {
+                WorkItem &o = own[q];
+                o.first = e0 + k;
+                o.J0 = entries[e0 + k].J;
+            }
+        }
+        __syncthreads();
     }
-}
-
-__global__ __launch_bounds__(256) void k_item_scatter(const WorkItem *__restrict__ items, int nitems,
-                                                      const int *__restrict__ cost, int maxcost, int interleave,
-                                                      int *__restrict__ cursor, WorkItem *__restrict__ out)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= nitems) return;
-    const int r = atomicAdd(&cursor[maxcost - cost[k]], 1);
-    out[interleave ? queue_start(nitems, r & 7) + (r >> 3) : r] = items[k];
-}
-
-// Work items of an already compacted list for another entries-per-item cut.
-// images != 0: the blocks are (image, super-cluster) blocks of the image
-// lists, and each item's sys field carries (image + 1) << 16.
-__global__ __launch_bounds__(256) void k_cut_items(const int *__restrict__ counts, const int *__restrict__ eoff,
-                                                   const int *__restrict__ ioff, int nblocks, int nsc, int per_item,
-                                                   int sys, int images, WorkItem *__restrict__ items)
-{
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= nblocks) return;
-    const int cnt = counts[s], e0 = eoff[s], i0 = ioff[s];
-    for (int k = 0; k * per_item < cnt; k++) {
-        WorkItem wi;
-        wi.sys = images ? (sys | ((s / nsc + 1) << 16)) : sys;
-        wi.sc = s % nsc;
-        wi.first = e0 + k * per_item;
-        wi.count = min(per_item, cnt - k * per_item);
-        items[i0 + k] = wi;
+    __threadfence_block();
+    __syncthreads();
+    const int tag = images ? (sys | ((s / nsc + 1) << 16)) : sys;
+    for (int q = tid; q < n; q += 256) {
+        WorkItem &o = own[q];
+        const int first = *(volatile int *)&o.first;
+        const int next = q + 1 < n ? *(volatile int *)&own[q + 1].first : e0 + cnt;
+        o.sys = tag;
+        o.sc = s % nsc;
+        o.count = next - first;
     }
 }
 
 // Entry and item offsets of the super-clusters from their entry counts, and
-// the totals (entries, items, search capacity needed) into out[0..2], in one
-// workgroup (each thread scans a contiguous chunk).
+// the totals (entries, items, search capacity needed, cost per item) into
+// out[0..3], in one workgroup (each thread scans a contiguous chunk).  The cut
+// follows the list's total cost (item_cost), so the entries come first.
 #define NB_OFFS_THREADS 1024
 #define NB_OFFS_MAX (64 * NB_OFFS_THREADS)
-__global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__restrict__ counts, int m, int per_item,
+__global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__restrict__ counts,
+                                                                  const int *__restrict__ costs, int m, ItemCut cut,
                                                                   int *__restrict__ eoff, int *__restrict__ nits,
                                                                   int *__restrict__ ioff, const int *__restrict__ need,
                                                                   int *__restrict__ out)
 {
     __shared__ int sE[NB_OFFS_THREADS / 64], sI[NB_OFFS_THREADS / 64];
+    __shared__ long long sC[NB_OFFS_THREADS / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int chunk = (m + NB_OFFS_THREADS - 1) / NB_OFFS_THREADS;
     const int lo = min(t * chunk, m), hi = min(lo + chunk, m);
-    int se = 0, si = 0;
+    int se = 0;
+    long long sc = 0;
     for (int k = lo; k < hi; k++) {
-        const int c = counts[k];
-        se += c;
-        si += (c + per_item - 1) / per_item;
+        se += counts[k];
+        sc += costs[k];
     }
-    int ie = se, ii = si;   // inclusive scans over the wave
+    int ie = se;            // inclusive scan over the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(ie, o, 64), u = __shfl_up(ii, o, 64);
-        if (lane >= o) {
-            ie += v;
-            ii += u;
-        }
+        const int v = __shfl_up(ie, o, 64);
+        if (lane >= o) ie += v;
+        sc += __shfl_xor(sc, o, 64);
     }
     if (lane == 63) {
         sE[w] = ie;
-        sI[w] = ii;
+        sC[w] = sc;
     }
     __syncthreads();
-    int be = 0, bi = 0, te = 0, ti = 0;
+    int be = 0, te = 0;
+    long long tc = 0;
     for (int v = 0; v < NB_OFFS_THREADS / 64; v++) {
-        if (v < w) {
-            be += sE[v];
-            bi += sI[v];
-        }
+        if (v < w) be += sE[v];
         te += sE[v];
+        tc += sC[v];
+    }
+    const int per_item = item_cost(cut, tc, m);
+    int si = 0;
+    for (int k = lo; k < hi; k++) si += (costs[k] + per_item - 1) / per_item;
+    int ii = si;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(ii, o, 64);
+        if (lane >= o) ii += v;
+    }
+    if (lane == 63) sI[w] = ii;
+    __syncthreads();
+    int bi = 0, ti = 0;
+    for (int v = 0; v < NB_OFFS_THREADS / 64; v++) {
+        if (v < w) bi += sI[v];
         ti += sI[v];
     }
     int e = be + ie - se, i = bi + ii - si;
     for (int k = lo; k < hi; k++) {
-        const int c = counts[k], ni = (c + per_item - 1) / per_item;
+        const int ni = (costs[k] + per_item - 1) / per_item;
         eoff[k] = e;
         ioff[k] = i;
         nits[k] = ni;
-        e += c;
+        e += counts[k];
         i += ni;
     }
     if (t == 0) {
@@ -1128,14 +1069,52 @@ __global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__r
         o[0] = te;
         o[1] = ti;
         o[2] = *need;
+        o[3] = per_item;
     }
 }
 
-__global__ __launch_bounds__(256) void k_items_per_sc(const int *__restrict__ counts, int nsc, int per_item,
+// Items per block for a cost per item of per_item.
+__global__ __launch_bounds__(256) void k_items_per_sc(const int *__restrict__ costs, int nsc, int per_item,
                                                       int *__restrict__ nitems)
 {
     int s = blockIdx.x * 256 + threadIdx.x;
-    if (s < nsc) nitems[s] = (counts[s] + per_item - 1) / per_item;
+    if (s < nsc) nitems[s] = (costs[s] + per_item - 1) / per_item;
+}
+
+// Items of the image lists' blocks and where each block's items go, in one workgroup; *out: their number.  A block cuts
+// into n items of cost C / n, and the blocks are laid out by falling item cost (NB_IORDER_BINS steps; the order within a
+// step is free: the items' sums are exact integers).  Blocks at an image's edge hold few entries, so the items differ
+// much more than the main list's, and a long one at the end of a launch is waited for: 23,559 atoms in a 50 A cell took
+// 150 us per call in block order and 139 us in this one.
+#define NB_IORDER_BINS 256
+__global__ __launch_bounds__(1024) void k_image_items(const int *__restrict__ costs, int m, int per_item,
+                                                      int *__restrict__ nits, int *__restrict__ ioff,
+                                                      int *__restrict__ out)
+{
+    __shared__ int sH[NB_IORDER_BINS];
+    const int t = threadIdx.x;
+    auto bin = [&](int c, int n) { return NB_IORDER_BINS - 1 - (int)((long long)(c / n) * (NB_IORDER_BINS - 1) / per_item); };
+    if (t < NB_IORDER_BINS) sH[t] = 0;
+    __syncthreads();
+    for (int k = t; k < m; k += 1024) {
+        const int c = costs[k], n = (c + per_item - 1) / per_item;
+        nits[k] = n;
+        if (n > 0) atomicAdd(&sH[bin(c, n)], n);
+    }
+    __syncthreads();
+    int own = 0, before = 0;
+    if (t < NB_IORDER_BINS) {
+        own = sH[t];
+        for (int v = 0; v < t; v++) before += sH[v];
+    }
+    __syncthreads();
+    if (t < NB_IORDER_BINS) sH[t] = before;
+    if (t == NB_IORDER_BINS - 1) *(volatile int *)out = before + own;
+    __syncthreads();
+    for (int k = t; k < m; k += 1024) {
+        const int c = costs[k], n = (c + per_item - 1) / per_item;
+        ioff[k] = n > 0 ? atomicAdd(&sH[bin(c, n)], n) : 0;
+    }
 }
 
 // Canonical pair keys max*n+min (for parity against the reference set).
@@ -1523,8 +1502,8 @@ void launch_slot_records(const double *xyz, const int *slot_atom, int n_pad, con
 }
 
 void launch_search(const SearchParams &P, int nsc, const double *xyz, const int *slot_atom, const float4 *blo,
-                   const float4 *bhi, const int2 *colcl, Entry *scratch, int *ncand, int *counts, int *overflow,
-                   hipStream_t s)
+                   const float4 *bhi, const int2 *colcl, Entry *scratch, int *ncand, int *counts, int *costs,
+                   int *overflow, hipStream_t s)
 {
     if (nsc <= 0) return;
     const int wst = 2 * P.u + 1;
@@ -1532,42 +1511,42 @@ void launch_search(const SearchParams &P, int nsc, const double *xyz, const int 
     if (sten != 0 && P.pointcell) {
         if (sten == 1)
             hipLaunchKernelGGL((k_search<false, 1, true>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom,
-                               blo, bhi, colcl, scratch, ncand, counts, overflow);
+                               blo, bhi, colcl, scratch, ncand, counts, costs, overflow);
         else
             hipLaunchKernelGGL((k_search<false, 2, true>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom,
-                               blo, bhi, colcl, scratch, ncand, counts, overflow);
+                               blo, bhi, colcl, scratch, ncand, counts, costs, overflow);
         return;
     }
     if (sten == 0)
         hipLaunchKernelGGL((k_search<false, 0>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, overflow);
+                           colcl, scratch, ncand, counts, costs, overflow);
     else if (sten == 1)
         hipLaunchKernelGGL((k_search<false, 1>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, overflow);
+                           colcl, scratch, ncand, counts, costs, overflow);
     else
         hipLaunchKernelGGL((k_search<false, 2>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, overflow);
+                           colcl, scratch, ncand, counts, costs, overflow);
 }
 
 void launch_search_images(const SearchParams &P, int nsc, int nimg, const double *xyz, const int *slot_atom,
-                          const float4 *blo, const float4 *bhi, Entry *scratch, int *ncand, int *counts, int *overflow,
-                          hipStream_t s)
+                          const float4 *blo, const float4 *bhi, Entry *scratch, int *ncand, int *counts, int *costs,
+                          int *overflow, hipStream_t s)
 {
     if (nsc <= 0 || nimg <= 0) return;
     if (P.use_grid && P.pointcell)
         hipLaunchKernelGGL((k_search<true, 0, true>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz,
-                           slot_atom, blo, bhi, (const int2 *)nullptr, scratch, ncand, counts, overflow);
+                           slot_atom, blo, bhi, (const int2 *)nullptr, scratch, ncand, counts, costs, overflow);
     else
         hipLaunchKernelGGL((k_search<true, 0>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo,
-                           bhi, (const int2 *)nullptr, scratch, ncand, counts, overflow);
+                           bhi, (const int2 *)nullptr, scratch, ncand, counts, costs, overflow);
 }
 
-void launch_cut_items(const int *counts, const int *eoff, const int *ioff, int nblocks, int nsc, int per_item,
-                      int sys, WorkItem *items, hipStream_t s, bool images)
+void launch_cut_items(const int *counts, const int *costs, const int *eoff, const int *ioff, const int *nits,
+                      int nblocks, int nsc, int sys, const Entry *entries, WorkItem *items, hipStream_t s, int images)
 {
     if (nblocks > 0)
-        hipLaunchKernelGGL(k_cut_items, dim3(nblk(nblocks, 256)), dim3(256), 0, s, counts, eoff, ioff, nblocks, nsc,
-                           per_item, sys, images ? 1 : 0, items);
+        hipLaunchKernelGGL(k_cut_items, dim3(nblocks), dim3(256), 0, s, counts, costs, eoff, ioff, nits, nsc, sys,
+                           images, entries, items);
 }
 
 void launch_image_transform(const double *xyz, int n, const double *rt, int ntrans, double *out, hipStream_t s)
@@ -1605,37 +1584,23 @@ void launch_export_image_pairs(const Entry *entries, int nent, const int *slot_a
                            cap, keys);
 }
 
-void launch_order_items(const WorkItem *items, int nitems, const Entry *entries, int maxcost, int interleave, int *cost,
-                        int *hist, int *cursor, int *scantmp, WorkItem *out, hipStream_t s)
-{
-    if (nitems <= 0) return;
-    if (maxcost + 1 <= NB_ORDER_BINS) {
-        hipLaunchKernelGGL(k_item_cost, dim3(nblk(nitems, 4)), dim3(256), 0, s, items, nitems, entries, maxcost, cost,
-                           (int *)nullptr);
-        hipLaunchKernelGGL(k_item_order, dim3(1), dim3(NB_ORDER_THREADS), 0, s, items, nitems, cost, maxcost,
-                           interleave, out);
-        return;
-    }
-    launch_fill_int(hist, (size_t)maxcost + 1, 0, s);
-    hipLaunchKernelGGL(k_item_cost, dim3(nblk(nitems, 4)), dim3(256), 0, s, items, nitems, entries, maxcost, cost,
-                       hist);
-    launch_scan(hist, cursor, maxcost + 1, scantmp, s);
-    hipLaunchKernelGGL(k_item_scatter, dim3(nblk(nitems, 256)), dim3(256), 0, s, items, nitems, cost, maxcost,
-                       interleave, cursor, out);
-}
-
-bool launch_list_offsets(const int *counts, int nsc, int per_item, int *eoff, int *nits, int *ioff, const int *need,
-                         int *out, hipStream_t s)
+bool launch_list_offsets(const int *counts, const int *costs, int nsc, const ItemCut &cut, int *eoff, int *nits,
+                         int *ioff, const int *need, int *out, hipStream_t s)
 {
     if (nsc <= 0 || nsc > NB_OFFS_MAX) return false;
-    hipLaunchKernelGGL(k_list_offsets, dim3(1), dim3(NB_OFFS_THREADS), 0, s, counts, nsc, per_item, eoff, nits, ioff,
+    hipLaunchKernelGGL(k_list_offsets, dim3(1), dim3(NB_OFFS_THREADS), 0, s, counts, costs, nsc, cut, eoff, nits, ioff,
                        need, out);
     return true;
 }
 
-void launch_items_per_sc(const int *counts, int nsc, int per_item, int *nitems, hipStream_t s)
+void launch_image_items(const int *costs, int m, int per_item, int *nits, int *ioff, int *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_items_per_sc, dim3(nblk(nsc, 256)), dim3(256), 0, s, counts, nsc, per_item, nitems);
+    hipLaunchKernelGGL(k_image_items, dim3(1), dim3(1024), 0, s, costs, m, per_item, nits, ioff, out);
+}
+
+void launch_items_per_sc(const int *costs, int nsc, int per_item, int *nitems, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_items_per_sc, dim3(nblk(nsc, 256)), dim3(256), 0, s, costs, nsc, per_item, nitems);
 }
 
 // Sum of the per-block pair counts into *out (one workgroup).
@@ -1651,13 +1616,12 @@ __global__ __launch_bounds__(256) void k_sum_u64(const unsigned long long *__res
     if (threadIdx.x == 0) *out = (sP[0] + sP[1]) + (sP[2] + sP[3]);
 }
 
-void launch_compact(const Entry *scratch, int cap, const int *soff, const int *ncand, const int *counts,
-                    const int *eoff, const int *ioff, int nblocks, int nsc, int per_item, int sys, Entry *entries,
-                    WorkItem *items, unsigned long long *npairs, unsigned long long *npairs_block, hipStream_t s)
+void launch_compact(const Entry *scratch, int cap, const int *soff, const int *ncand, const int *eoff, int nblocks,
+                    Entry *entries, unsigned long long *npairs, unsigned long long *npairs_block, hipStream_t s)
 {
     if (nblocks <= 0) return;
-    hipLaunchKernelGGL(k_compact, dim3(nblocks), dim3(NB_COMPACT_THREADS), 0, s, scratch, cap, soff, ncand, counts,
-                       eoff, ioff, nsc, per_item, sys, entries, items, npairs_block);
+    hipLaunchKernelGGL(k_compact, dim3(nblocks), dim3(NB_COMPACT_THREADS), 0, s, scratch, cap, soff, ncand, eoff, entries,
+                       npairs_block);
     if (npairs) hipLaunchKernelGGL(k_sum_u64, dim3(1), dim3(256), 0, s, npairs_block, nblocks, npairs);
 }
 

@@ -112,8 +112,7 @@ __device__ __forceinline__ double min_uniform(double x, double s)
 }
 
 __device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, double u, double qq, double4 C,
-                                          unsigned long long mact, const GAS double *__restrict__ ljA,
-                                          const GAS double *__restrict__ ljB, int off, double &fs, double &eel,
+                                          unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
                                           double &elj)
 {
     const double y = (double)__builtin_amdgcn_rsqf((float)r2);
@@ -132,13 +131,16 @@ __device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, doubl
     const double inner = fma(s3 + s3, fma(C.x, s6, t1), C.z);
     // Minus twice dE/d(r^2): Coulomb qq s^3 Q, Lennard-Jones 3 s^5 inner (the rows' factor 3).
     double f = s3 * fma(s2, inner, qq * Q);
-    // A branch of the whole wave (its lanes select), so the usual path has no execution-mask bookkeeping.
+    // A branch of the whole wave (its lanes select), so the usual path has no execution-mask bookkeeping.  Its factors and
+    // tables are read through the descriptor here: as kernel arguments they would hold (and spill) scalar registers over
+    // the whole entry loop.
     if (__builtin_expect((__builtin_amdgcn_ballot_w64(r2 < F.r2Damp) & mact) != 0ull, 0)) {
+        const GAS double *k = as_global(D->damp);
         const bool damped = r2 < F.r2Damp;
-        const double A = ljA[off >> 6], B = ljB[off >> 6];
-        e1 = damped ? qq * fma(F.qAlphaE, r2, F.qF0e) : e1;
-        e2 = damped ? 3.0 * (A * fma(-F.aAlpha, r2, F.aF0) - B * fma(-F.bAlpha, r2, F.bF0)) : e2;
-        f = damped ? 2.0 * (qq * F.qAlpha + (A * F.aAlpha - B * F.bAlpha)) : f;
+        const double A = as_global(D->ljA)[off >> 6], B = as_global(D->ljB)[off >> 6];
+        e1 = damped ? qq * fma(k[1], r2, k[0]) : e1;
+        e2 = damped ? 3.0 * (A * fma(-k[3], r2, k[2]) - B * fma(-k[5], r2, k[4])) : e2;
+        f = damped ? 2.0 * (qq * k[6] + (A * k[3] - B * k[5])) : f;
     }
     fs = f;
     eel = e1;
@@ -231,12 +233,12 @@ __global__ __launch_bounds__(256) void k_prepare(const SysDesc *__restrict__ des
     }
 }
 
-// A wave-uniform FP64 value moved into scalar registers.
-__device__ __forceinline__ double uniform_f64(double v)
+// One lane's FP64 value in scalar registers.
+__device__ __forceinline__ double lane_f64(double v, int lane)
 {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
-    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
@@ -334,19 +336,15 @@ __device__ __forceinline__ int load_jtype(const GAS int *__restrict__ ty, int J,
     return *(const GAS int *)((const GAS char *)base + off);
 }
 
-// Entry fields through the vector memory path: one load brings the header's
-// words (lanes 8b .. 8b + 7 read word b, off = 4 b: the lane offset the j-atom
-// types use), of which J (word 0) and cbits (word 2) are read back from their
-// lanes; each lane reads its own tile-mask byte (64 consecutive bytes per entry).
-__device__ __forceinline__ int entry_header(const GAS unsigned char *__restrict__ eb, int e, unsigned off)
+// Entry fields through the vector memory path.  Headers: lane k reads (J, cbits)
+// of entry first + k, so one load brings a whole item's headers (64 entries) and
+// the entry loop takes them from its lanes; each lane reads its own tile-mask
+// byte of an entry (64 consecutive bytes).
+__device__ __forceinline__ int2 entry_headers(const GAS unsigned char *__restrict__ eb, int first, int count, int lane)
 {
-    unsigned long long base = (unsigned long long)(eb + (size_t)e * sizeof(Entry));
-    asm volatile("" : "+s"(base), "+v"(off));
-    return *(const GAS int *)((const GAS char *)base + off);
+    const GAS int *p = (const GAS int *)(eb + (size_t)(first + min(lane, max(count - 1, 0))) * sizeof(Entry));
+    return make_int2(p[0], p[1]);
 }
-
-__device__ __forceinline__ int header_j(int h) { return __builtin_amdgcn_readlane(h, 0); }
-__device__ __forceinline__ int header_cbits(int h) { return __builtin_amdgcn_readlane(h, 16); }
 
 __device__ __forceinline__ int entry_bits(const GAS unsigned char *__restrict__ eb, int e, unsigned lane)
 {
@@ -471,7 +469,8 @@ __device__ __forceinline__ T i_force(T (&f)[NB_SCC], int lane)
 // system when it fits (ROWS_LDS: staged once per group), then one region per
 // wave: the item's i-cluster records and slot types, then one record per entry
 // and j-atom (the three j-force sums and the j-cluster), flushed to the
-// fixed-point accumulators once at the end of the item.
+// fixed-point accumulators every NB_JCHUNK entries.
+#define NB_JCHUNK 16
 #define NB_LDS_IREC 48          // x, y, z, q and the type's row offset, padded
 #define NB_LDS_I_BYTES (NB_SC * NB_LDS_IREC)
 #define NB_LDS_ROW_LIMIT 16384
@@ -480,10 +479,7 @@ __device__ __forceinline__ T i_force(T (&f)[NB_SCC], int lane)
 static inline size_t tiled_lds_rows(int ntypes, bool rows_lds) { return rows_lds ? (size_t)2 * ntypes * ntypes * 32 : 0; }
 
 // acc: bytes of a force accumulator (4: FP32, the mixed kernel; 8: FP64, the full-FP64 kernel).
-static inline size_t tiled_lds_wave(int max_count, int acc)
-{
-    return NB_LDS_I_BYTES + (size_t)max_count * 4 * NB_CL * acc;
-}
+static inline size_t tiled_lds_wave(int acc) { return NB_LDS_I_BYTES + (size_t)NB_JCHUNK * 4 * NB_CL * acc; }
 
 // Wave-scope synchronisation of a wave's own LDS region (workgroups of several
 // independent waves); a workgroup barrier when the workgroup is one wave.
@@ -499,24 +495,77 @@ __device__ __forceinline__ void wave_region_sync()
     }
 }
 
+// Wave sums of three values into the fixed-point words ga[0..5].
+__device__ __forceinline__ bool add_sums3(long long *ga, double x, double y, double z, int lane)
+{
+    const double sx = wave_sum_f64(x), sy = wave_sum_f64(y), sz = wave_sum_f64(z);
+    const double v = lane == 0 ? sx : (lane == 1 ? sy : sz);
+    return lane < 3 && fx_add(&ga[2 * lane], &ga[2 * lane + 1], v);
+}
+
+// What a wave needs before its first tile: its lane's i-record and type, the
+// item's entry headers, the first entry's mask byte and j-record.  All of it is
+// asked for at once; a group asks before it stages its row table, so that the
+// two latencies overlap.
+struct ItemStart {
+    double4 rec, xj;
+    double xf;            // image items: lane k holds word k of the image transform
+    int2 head;
+    int typ, tj, bits;
+};
+
+template <bool IMG>
+__device__ __forceinline__ ItemStart item_start(const SysDesc *D, const WorkItem &w, int lane)
+{
+    const unsigned a = lane & 7, b = lane >> 3;
+    const GAS double *xq = (const GAS double *)D->xyzq;
+    const GAS int *ty = as_global(D->styp);
+    const GAS unsigned char *eb = (const GAS unsigned char *)D->entries;
+    ItemStart t;
+    t.head = entry_headers(eb, w.first, w.count, lane);
+    t.bits = entry_bits(eb, w.first, 8 * a + b);
+    t.xf = IMG ? ((const GAS double *)&D->imgxf[max((w.sys >> 16) - 1, 0)])[min(lane, 13)] : 0.0;
+    t.rec = load_slot(xq, w.sc * NB_SC + lane);
+    t.typ = ty[w.sc * NB_SC + lane];
+    t.xj = load_j(xq, w.J0, 32u * b);
+    t.tj = load_jtype(ty, w.J0, 4u * b);
+    return t;
+}
+
+// An item whose fields are the same on every lane, in scalar registers.
+__device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
+{
+    WorkItem u = {};
+    u.sys = __builtin_amdgcn_readfirstlane(w.sys);
+    u.sc = __builtin_amdgcn_readfirstlane(w.sc);
+    u.first = __builtin_amdgcn_readfirstlane(w.first);
+    u.count = __builtin_amdgcn_readfirstlane(w.count);
+    u.J0 = __builtin_amdgcn_readfirstlane(w.J0);
+    return u;
+}
+
 // Waves per SIMD.  A tile is a chain of two LDS reads and about forty dependent FP64 instructions, so the issue slots
 // fill only with enough waves: five fit in 96 VGPRs, with no spill inside the entry loop, because the loop holds no
 // 64-bit lane offsets, one LDS address for all tiles (records at a 16-byte-aligned stride with the type beside the
-// charge), header words of one load, FP32 copies of dx, dy, dz across the pair terms and no polynomial factor in vector
-// registers.  16-image batch: 680 us per call with three waves, 620 with four, 603 with five (647 before, four waves).
-// IMG: the launch over the image lists' work items (the main list's items run in an instance without any image code);
-// it runs at three waves per SIMD, whose register budget holds the transformation without spilling.
+// charge), FP32 copies of dx, dy, dz across the pair terms and no polynomial factor in vector registers.  16-image batch:
+// 680 us per call with three waves, 620 with four, 603 with five.
+// A wave costs about 5 us beside its entries, and an entry's loads are a chain as long as its tiles: what a wave needs
+// first is asked for at once (ItemStart), and an item's entry headers come with one load.
+// IMG: the launch holds image items too (sys >> 16: the image plus one), beside the main list's or alone.  The j-record
+// is transformed once per entry; the image's part of the item's end takes four waves per SIMD (107 VGPRs, no spill).  One
+// launch, because a second stream's launch starts 15 us after its fork and joins 11 us after its end, and because the
+// image items fill the GPU as the main items drain: 23,559 atoms in a 50 A cell, 139 us per call with two launches,
+// 126 us with one.
 // F64: the full-FP64 instance (the NBABFS_TILED_FP64 comparison path): the same list, tiles, staging and
 // fixed-point sums, with the reference's FP64 pair arithmetic (pair_fp64: divide and square root, no FP32
 // seed, raw A and B per type pair) and FP64 force vectors; three waves per SIMD for its larger accumulators.
-// WPG: wavefronts per workgroup.  With 4 (the one-item-per-wave launches of
-// the main list), the row table is staged once for four items and a group's
-// LDS stays small enough for four waves per SIMD; the four items of a group
-// belong to one system (batches pad each system's items to a multiple of 4
-// with empty ones).  Image items and the persistent queues run one wave per
-// group.
+// WPG: wavefronts per workgroup.  With 4 (the one-item-per-wave launches),
+// the row table is staged once for four items and a group's LDS stays small
+// enough for five waves per SIMD; the four items of a group belong to one
+// system (batches pad each system's items to a multiple of 4 with empty
+// ones).  The persistent queues run one wave per group.
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG || F64) ? 3 : 5))) void k_force_tiled(
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 3 : (IMG ? 4 : 5)))) void k_force_tiled(
     const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, AbfsFactors F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
@@ -525,9 +574,10 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
     // A group's start is a chain of dependent loads (its work item, the system's descriptor, the records the item
     // names).  The loads that depend on nothing go out together with the guard's flag: the work item of a wave
     // with one item, and (sys1 >= 0: every item belongs to system sys1) the descriptor and its row table.
-    WorkItem w0 = {0, 0, 0, 0};
-    const bool one_item = qp.heads == nullptr && (IMG || (int)blockIdx.x < nforce_groups);
-    if (one_item && nitems > 0) w0 = items[min((int)blockIdx.x * WPG + wave, nitems - 1)];
+    constexpr bool QUEUE = WPG == 1 && !IMG;       // a persistent launch: items come from the per-XCD queues
+    WorkItem w0 = {};
+    if (!QUEUE && (int)blockIdx.x < nforce_groups && nitems > 0)
+        w0 = items[min((int)blockIdx.x * WPG + wave, nitems - 1)];
     // guard_skip with both loads issued here unconditionally (a null pointer reads the descriptor instead) and
     // their values compared only where the answer is needed.
     const int *gfp = guard.flag ? guard.flag : (const int *)descs;
@@ -535,7 +585,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
     const int gflag = __hip_atomic_load(gfp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int gepoch = __hip_atomic_load(gep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // Groups past the pair blocks evaluate the 1-4 list of system 0 (single-state launches), one block per wave.
-    if (!IMG && (int)blockIdx.x >= nforce_groups) {
+    if ((int)blockIdx.x >= nforce_groups) {
         const int blk = ((int)blockIdx.x - nforce_groups) * WPG + wave;
         if (!guard_skip(guard) && blk < descs[0].n14_blocks) pairs14_block(descs[0], F, blk, lane);
         return;
@@ -545,36 +595,37 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
     const int a = lane & 7, b = lane >> 3;
     const int bl = 8 * a + b;
     extern __shared__ __align__(32) unsigned char lds[];
-    __shared__ __align__(16) double sX[12];     // image items: R then T of the item's image
+    __shared__ __align__(16) double sXs[IMG ? WPG : 1][12];     // image items: R then T of the item's image
+    double *sX = sXs[IMG ? wave : 0];
     using acc_t = typename std::conditional<F64, double, float>::type;
     double4 *sR = (double4 *)lds;
     unsigned char *region = lds + rows_bytes + (size_t)wave * wave_bytes;
     acc_t *sJ = (acc_t *)(region + NB_LDS_I_BYTES);   // [entry][j-atom] of (x, y, z, J)
-    // The group's row table, staged once when the items are one per wave.
-    int rows_sys = -1;
-    if (ROWS_LDS && qp.heads == nullptr && WPG > 1) {
-        rows_sys = sys1 >= 0 ? sys1 : items[(int)blockIdx.x * WPG].sys;
-        const SysDesc *D0 = &descs[rows_sys];
-        const GAS double *__restrict__ rows0 = as_global(D0->ljrow);
-        const int nr = 2 * D0->ntypes * D0->ntypes;
-        for (int k = threadIdx.x; k < nr; k += 64 * WPG) sR[k] = load_slot(rows0, k);
-        __syncthreads();
+    // One item per wave: ask for all it needs, then stage the group's row table (the items of a group belong to one
+    // system).
+    ItemStart st = {};
+    if (!QUEUE) {
+        w0 = uniform_item(w0);
+        const SysDesc *D0 = &descs[sys1 >= 0 ? sys1 : (IMG ? (w0.sys & 0xffff) : w0.sys)];
+        st = item_start<IMG>(D0, w0, lane);
+        if (ROWS_LDS) {
+            const GAS double *__restrict__ rows0 = as_global(D0->ljrow);
+            const int nr = 2 * D0->ntypes * D0->ntypes;
+            for (int k = threadIdx.x; k < nr; k += 64 * WPG) sR[k] = load_slot(rows0, k);
+            if (WPG > 1) __syncthreads();
+        }
     }
     // The guard's answer is needed only now (the loads above are reads; the flag is uniform over the launch).
     if (guard.flag != nullptr && gflag == (guard.epoch_ptr ? gepoch : guard.epoch)) return;
+    // One work item per wave (the hardware dispatcher balances the load), or a persistent loop over per-XCD queues whose
+    // counters sit on separate 128-byte lines.
     int q = blockIdx.x & 7;
     int tries = 0;
-    // heads == null: one work item per wave (the hardware dispatcher
-    // balances the load); otherwise a persistent loop over per-XCD queues whose
-    // counters sit on separate 128-byte lines (one wave per group).
-    bool done = false;
-    while (!done && tries < 8) {
+    for (;;) {
         int it;
-        if (qp.heads == nullptr) {
-            it = (int)blockIdx.x * WPG + wave;
-            done = true;
-            if (it >= nitems) break;
-        } else {
+        WorkItem w = w0;
+        if (QUEUE) {
+            if (tries >= 8) break;
             int local = 0;
             if (lane == 0) local = atomicAdd(&qp.heads[32 * q], 1);
             local = __builtin_amdgcn_readfirstlane(local);
@@ -585,14 +636,12 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                 continue;
             }
             it = qs + local;
-        }
-        const WorkItem w = qp.heads == nullptr ? w0 : items[it];
-        // Empty items pad a batch's systems to whole groups; an item of another system than the staged rows
-        // would be a layout error (reported, never evaluated with the wrong rows).
-        if (w.count <= 0) continue;
-        if (rows_sys >= 0 && w.sys != rows_sys) {
-            raise_error(descs[rows_sys].err, true, NB_ERR_RANGE);
-            continue;
+            w = uniform_item(items[it]);
+            if (w.count <= 0) continue;
+        } else {
+            it = (int)blockIdx.x * WPG + wave;
+            // Empty items pad a batch's systems to whole groups.
+            if (it >= nitems || w.count <= 0) break;
         }
         const SysDesc *D = &descs[sys1 >= 0 ? sys1 : (IMG ? (w.sys & 0xffff) : w.sys)];
         const GAS double *__restrict__ xq = (const GAS double *)D->xyzq;
@@ -608,46 +657,44 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         // The item's image (-1: main list); all of its entries share it.
         int img = -1;
         double isc = 1.0;
-        const GAS double *X = nullptr;
-        if (IMG) {
-            img = __builtin_amdgcn_readfirstlane((w.sys >> 16) - 1);
-            X = (const GAS double *)&D->imgxf[img];
-            isc = uniform_f64(X[12]);
+        bool moments = false;
+        if (IMG) img = (w.sys >> 16) - 1;
+        if (IMG && img >= 0) {
+            isc = lane_f64(st.xf, 12);
+            moments = lane_f64(st.xf, 13) == 0.0;
         }
 
-        // The item's independent loads go out together: its super-cluster's records and types and its first two
-        // entries' headers and mask bytes; then the first j-cluster's records, which need the first header.
-        // Pipeline of the entry loop: while entry e is evaluated, entry e+1's j-cluster record and entry e+2's
-        // header and mask byte are in flight.  The indices are clamped, so every iteration issues the same loads
-        // and no atomic is pending inside the loop.
+        // Pipeline of the entry loop: while entry e is evaluated, entry e+1's j-cluster record and mask byte are in
+        // flight.  The indices are clamped, so every iteration issues the same loads and no atomic is pending inside
+        // the loop.
         const int e_last = w.first + w.count - 1;
-        const double4 irec = load_slot(xq, I0 * NB_CL + lane);
-        const int ityp = ty[I0 * NB_CL + lane];
+        if (QUEUE) st = item_start<IMG>(D, w, lane);
         const unsigned jrec = 32u * b, jtyp = 4u * b;      // byte offsets in a j-cluster's records and types
-        const int h0 = entry_header(eb, w.first, jtyp);
-        int lbn = entry_bits(eb, w.first, bl);
-        int hn = entry_header(eb, min(w.first + 1, e_last), jtyp);
 
         // A persistent wave's region still holds its previous item's data until every lane is past it.
-        if (qp.heads != nullptr) wave_region_sync<WPG>();
-        if (IMG && lane < 12) sX[lane] = X[lane];
-        if (ROWS_LDS && rows_sys < 0)
+        if (QUEUE) wave_region_sync<WPG>();
+        if (IMG && img >= 0 && lane < 12) sX[lane] = st.xf;
+        if (ROWS_LDS && QUEUE)
             for (int k = lane; k < 2 * nt * nt; k += 64) sR[k] = load_slot(rows, k);
         {
             double *r = (double *)(region + NB_LDS_IREC * lane);
-            r[0] = irec.x;
-            r[1] = irec.y;
-            r[2] = irec.z;
-            r[3] = irec.w;
-            *(int *)(r + 4) = 64 * nt * ityp;   // byte offset of the type's first row pair
+            r[0] = st.rec.x;
+            r[1] = st.rec.y;
+            r[2] = st.rec.z;
+            r[3] = st.rec.w;
+            *(int *)(r + 4) = 64 * nt * st.typ;   // byte offset of the type's first row pair
         }
-        int J = header_j(h0);
-        int cbn = header_cbits(h0);
-        double4 xj = load_j(xq, J, jrec);
-        int tj = 64 * load_jtype(ty, J, jtyp);
+        int hbase = w.first;                       // entry whose header lane 0 holds
+        int2 head = st.head;
+        int J = w.J0;
+        int cbn = __builtin_amdgcn_readlane(head.y, 0);
+        int lbn = st.bits;
+        double4 xj = st.xj;
+        int tj = 64 * st.tj;
         const int comp = min(a, NB_CL - 1 - a);
         const double fscale = F64 ? 1.0 : -1.0;            // i-force = fscale times the sum over j
         wave_region_sync<WPG>();
+        if (IMG && img >= 0) xj = image_slot(xj, sX);
 
         acc_t fx[NB_SCC], fy[NB_SCC], fz[NB_SCC];
 #pragma unroll
@@ -659,17 +706,22 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         // The i-records are read at constant offsets from one address per lane (the compiler would keep one per tile).
         const LAS char *ip = (const LAS char *)(region + NB_LDS_IREC * a);
         asm("" : "+v"(ip));
-        for (int e = w.first; e <= e_last; e++) {
-            // Entry e + 1's cluster and mask were asked for one entry ago, its header two entries ago.
+        bool bad = false;
+        for (int e0 = w.first; e0 <= e_last; e0 += NB_JCHUNK) {
+        const int e1 = min(e0 + NB_JCHUNK - 1, e_last);
+        for (int e = e0; e <= e1; e++) {
+            // The next entry's header is on lane en - hbase; an item of more than 64 entries reads the next 64.
             const int cb = cbn, lb = lbn;
-            const int Jn = header_j(hn);
-            cbn = header_cbits(hn);
+            const int en = min(e + 1, e_last);
+            if (en - hbase >= 64) {
+                hbase = en;
+                head = entry_headers(eb, hbase, e_last - hbase + 1, lane);
+            }
+            const int Jn = __builtin_amdgcn_readlane(head.x, en - hbase);
+            cbn = __builtin_amdgcn_readlane(head.y, en - hbase);
             const double4 xjn = load_j(xq, Jn, jrec);
             const int tjn = 64 * load_jtype(ty, Jn, jtyp);
-            hn = entry_header(eb, min(e + 2, e_last), jtyp);
-            lbn = entry_bits(eb, min(e + 1, e_last), bl);
-            // Image items: the j-atom's image position (its load was issued one entry earlier).
-            const double4 xjt = IMG ? image_slot(xj, sX) : xj;
+            lbn = entry_bits(eb, en, bl);
             acc_t gx = (acc_t)0, gy = (acc_t)0, gz = (acc_t)0;
 #pragma unroll
             for (int c = 0; c < NB_SCC; c++) {
@@ -679,7 +731,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                     int ti = *(const LAS int *)(ip + c * NB_CL * NB_LDS_IREC + 32);
                     // The charge and type are read with the position, not after the branch below: one LDS wait per tile.
                     asm("" : "+v"(xi.w), "+v"(ti));
-                    const double dx = xi.x - xjt.x, dy = xi.y - xjt.y, dz = xi.z - xjt.z;
+                    const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
                     const bool inr = r2 <= F.r2Off;
                     // Ballots of the two compares (lane masks as they stand), combined in scalar registers; the
@@ -694,7 +746,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                             if (act) {
                                 const int tij = (ti + tj) >> 6;
                                 double x1, x2, dF;
-                                pair_fp64(F, r2, xi.w * xjt.w, ljA[tij], ljB[tij], x1, x2, dF);
+                                pair_fp64(F, r2, xi.w * xj.w, ljA[tij], ljB[tij], x1, x2, dF);
                                 const double f = 2.0 * dF;
                                 fx[c] = fma(f, dx, fx[c]); fy[c] = fma(f, dy, fy[c]); fz[c] = fma(f, dz, fz[c]);
                                 gx = fma(f, dx, gx); gy = fma(f, dy, gy); gz = fma(f, dz, gz);
@@ -707,7 +759,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
                             const double4 C = ROWS_LDS ? *(const double4 *)((const unsigned char *)sR + off)
                                                        : load_slot(rows, off >> 5);
                             double fs, x1, x2;
-                            pair_rows(F, r2, u, xi.w * xjt.w, C, mact, ljA, ljB, off, fs, x1, x2);
+                            pair_rows(F, r2, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
                             // The sums take the active lanes only (the others may hold any value).
                             if (act) {
                                 const float f = (float)fs;
@@ -726,17 +778,17 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
             }
             const acc_t rec = j_record(gx, gy, gz, J, comp);
             // Lanes a and 7 - a hold the same value.
-            sJ[(e - w.first) * 4 * NB_CL + 4 * b + comp] = rec;
+            sJ[(e - e0) * 4 * NB_CL + 4 * b + comp] = rec;
             J = Jn;
             xj = xjn;
+            if (IMG && img >= 0) xj = image_slot(xj, sX);      // the j-atom's image position
             tj = tjn;
         }
-        // The entries' j-force sums (written by other lanes) are complete.
+        // The chunk's j-force sums (written by other lanes) are complete.
         wave_region_sync<WPG>();
-        bool bad = false;
-        if (!IMG) {
-            // j-forces of the whole item: one record per lane.
-            for (int k = lane; k < NB_CL * w.count; k += 64) {
+        if (!IMG || img < 0) {
+            // One record per lane.
+            for (int k = lane; k < NB_CL * (e1 - e0 + 1); k += 64) {
                 const acc_t *f = &sJ[4 * k];
                 const int sj = bits_j(f[3]) * NB_CL + (k & 7);
                 bad |= fx_atomic_add3(facc, n_pad, sj, -fscale * (double)f[0], -fscale * (double)f[1],
@@ -748,36 +800,37 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
             // for the lattice derivatives (SymmetryParameterGradients_ImageDerivatives,
             // pMolecule-1.9.0/extensions/csource/SymmetryParameterGradients.c:142-216).
             // A pure translation needs only h (the moments' derivative term vanishes).
-            const bool moments = __builtin_amdgcn_readfirstlane(X[13] == 0.0 ? 1 : 0) != 0;
-            double G[12];
-#pragma unroll
-            for (int k = 0; k < 12; k++) G[k] = 0.0;
-            for (int k = lane; k < NB_CL * w.count; k += 64) {
+            const double jsc = -fscale * isc;
+            const int nrec = NB_CL * (e1 - e0 + 1);
+            long long *ga = D->gacc + (size_t)img * NB_GACC_WORDS_PER_IMAGE +
+                            (size_t)(it & (NB_GSLOTS - 1)) * NB_GACC_WORDS_PER_SLOT;
+            double hx = 0.0, hy = 0.0, hz = 0.0;
+            for (int k = lane; k < nrec; k += 64) {
                 const acc_t *f = &sJ[4 * k];
                 const int sj = bits_j(f[3]) * NB_CL + (k & 7);
-                const double jsc = -fscale * isc;
                 const double gx = jsc * (double)f[0], gy = jsc * (double)f[1], gz = jsc * (double)f[2];
                 bad |= fx_atomic_add3(facc, n_pad, sj, fma(sX[0], gx, fma(sX[3], gy, sX[6] * gz)),
                                       fma(sX[1], gx, fma(sX[4], gy, sX[7] * gz)),
                                       fma(sX[2], gx, fma(sX[5], gy, sX[8] * gz)));
-                G[0] += gx; G[1] += gy; G[2] += gz;
-                if (moments) {
-                    const double4 xr = load_slot(xq, sj);
-                    G[3] = fma(gx, xr.x, G[3]); G[4] = fma(gx, xr.y, G[4]); G[5] = fma(gx, xr.z, G[5]);
-                    G[6] = fma(gy, xr.x, G[6]); G[7] = fma(gy, xr.y, G[7]); G[8] = fma(gy, xr.z, G[8]);
-                    G[9] = fma(gz, xr.x, G[9]); G[10] = fma(gz, xr.y, G[10]); G[11] = fma(gz, xr.z, G[11]);
+                hx += gx; hy += gy; hz += gz;
+            }
+            bad |= add_sums3(ga, hx, hy, hz, lane);
+            // Row a of the moments, one after the other (nine sums at once would not leave the entry loop its registers).
+            if (moments) {
+#pragma nounroll
+                for (int r = 0; r < 3; r++) {
+                    hx = hy = hz = 0.0;
+                    for (int k = lane; k < nrec; k += 64) {
+                        const acc_t *f = &sJ[4 * k];
+                        const double4 xr = load_slot(xq, bits_j(f[3]) * NB_CL + (k & 7));
+                        const double g = jsc * (double)f[r];
+                        hx = fma(g, xr.x, hx); hy = fma(g, xr.y, hy); hz = fma(g, xr.z, hz);
+                    }
+                    bad |= add_sums3(ga + 6 * (r + 1), hx, hy, hz, lane);
                 }
             }
-            long long *ga = D->gacc + (size_t)img * NB_GACC_WORDS_PER_IMAGE +
-                            (size_t)(it & (NB_GSLOTS - 1)) * NB_GACC_WORDS_PER_SLOT;
-            const int ncomp = moments ? 12 : 3;
-#pragma unroll
-            for (int k = 0; k < 12; k++) {
-                if (k < ncomp) {
-                    const double v = wave_sum_f64(G[k]);
-                    if (lane == k) bad |= fx_add(&ga[2 * k], &ga[2 * k + 1], v);
-                }
-            }
+        }
+        wave_region_sync<WPG>();
         }
         // i-forces: lane 8b + a ends with atom a of i-cluster b.
         const double iscale = IMG ? isc * fscale : fscale;
@@ -788,10 +841,12 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((IMG |
         const double etot = wave_sum2_f64(F64 ? eel : eel * F.eScale, F64 ? elj : elj * (1.0 / 3.0));
         if ((lane & 31) == 0) {
             const int slot = it & (NB_ESLOTS - 1);
-            const int kind = (lane >> 5) + (IMG ? 2 : 0);
-            bad |= fx_add(eacc_word(D->eacc, kind, 0, slot), eacc_word(D->eacc, kind, 1, slot), IMG ? isc * etot : etot);
+            const int kind = (lane >> 5) + (img >= 0 ? 2 : 0);
+            bad |= fx_add(eacc_word(D->eacc, kind, 0, slot), eacc_word(D->eacc, kind, 1, slot),
+                          2.0 * (IMG ? isc * etot : etot), 0x1p67);
         }
         raise_error(D->err, bad, NB_ERR_RANGE);
+        if (!QUEUE) break;
     }
 }
 
@@ -1071,7 +1126,7 @@ __global__ __launch_bounds__(256) void k_finalize(const SysDesc *__restrict__ de
                 // Canonical words of the total (0 <= low < 2^48), then one rounding.
                 h += l >> 48;
                 l &= (1ll << 48) - 1;
-                sE[kind] = (double)h * NB_FX_HI_UNIT + (double)l / NB_FX_LO_SCALE;
+                sE[kind] = 0.5 * ((double)h * NB_FX_HI_UNIT + (double)l / NB_FX_LO_SCALE);
             }
         }
         __syncthreads();
@@ -1200,17 +1255,16 @@ static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEve
 }
 
 void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const AbfsFactors &F,
-                        int nblocks, int max_ntypes, int max_count, ForceGuard g, hipStream_t s, bool images,
+                        int nblocks, int max_ntypes, ForceGuard g, hipStream_t s, bool images,
                         hipEvent_t ev_start, hipEvent_t ev_stop, int n14_blocks, bool full_fp64, int sys1)
 {
-    if (images) n14_blocks = 0;
     if (nblocks + n14_blocks <= 0) return;
     // One item per wave, four waves per group, unless the items come from the persistent queues or the images.
-    const int wpg = (images || q.heads != nullptr) ? 1 : NB_TILED_WPG;
+    const int wpg = q.heads != nullptr ? 1 : NB_TILED_WPG;
     const int ngroups = nblk(nblocks, wpg);
     const dim3 grid(ngroups + nblk(n14_blocks, wpg));
     const int acc = full_fp64 ? 8 : 4;
-    const int wave_bytes = (int)tiled_lds_wave(max_count, acc);
+    const int wave_bytes = (int)tiled_lds_wave(acc);
     // The row table goes to LDS when the group's LDS still lets four groups of four waves (or ten single waves) share a CU
     // (five groups do up to 32 KB: ten types with 16 entries per wave take 27 KB).
     const size_t limit = wpg == 1 ? NB_LDS_ROW_LIMIT : NB_LDS_GROUP_LIMIT;
@@ -1227,9 +1281,9 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
             launch_tiled_instance<false, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
     } else if (images) {
         if (rows_lds)
-            launch_tiled_instance<true, true, false, 1>(NB_TILED_ARGS);
+            launch_tiled_instance<true, true, false, NB_TILED_WPG>(NB_TILED_ARGS);
         else
-            launch_tiled_instance<false, true, false, 1>(NB_TILED_ARGS);
+            launch_tiled_instance<false, true, false, NB_TILED_WPG>(NB_TILED_ARGS);
     } else if (wpg == 1) {
         if (rows_lds)
             launch_tiled_instance<true, false, false, 1>(NB_TILED_ARGS);

@@ -214,8 +214,6 @@ static void make_factors(double damp, double inner, double outer, AbfsFactors &F
     F.eScale = (double)p3;
     F.eInv = (double)(1.0L / p3);
     F.qShift2e = (double)((long double)F.qShift2 / p3);
-    F.qF0e = (double)((long double)F.qF0 / p3);
-    F.qAlphaE = (double)(-(long double)F.qAlpha / p3);
     F.minus3 = -3.0;
 }
 
@@ -277,7 +275,7 @@ __global__ void k_remap_items(const WorkItem *__restrict__ src, int count, int p
         w.sys = sys;
         dst[k] = w;
     } else if (k < padded) {
-        dst[k] = WorkItem{sys, 0, 0, 0};
+        dst[k] = WorkItem{sys, 0, 0, 0, 0, {0, 0, 0}};
     }
 }
 
@@ -404,6 +402,7 @@ struct nbabfs_state {
     int u = 0;
     DBuf<unsigned char> stencil;
     int n_pad = 0, ncl = 0, nsc = 0, nent = 0, nitems = 0, cap = 512;
+    int item_units = NB_MIN_ITEM_COST;   // cost per item of the current cut of the main list
     DBuf<int> slot_atom, atom_slot;
     DBuf<int4> cellv;
     DBuf<float4> blo, bhi, centre;
@@ -412,8 +411,7 @@ struct nbabfs_state {
     DBuf<double4> srec;      // slot-ordered search records (self-list search)
     DBuf<int4> scell;
     DBuf<Entry> entries, scratch;
-    DBuf<WorkItem> items, items2;
-    DBuf<int> icost, ihist, icur;
+    DBuf<WorkItem> items;
     DBuf<int> rowptr, cols;
 
     // Per call.
@@ -443,7 +441,7 @@ struct nbabfs_state {
     int epoch = 0;
 
     // Build temporaries.
-    DBuf<int> key, count, off, cursor, sorted, padded, colstart, scantmp, counts, ncand, eoff, nits, ioff, flag;
+    DBuf<int> key, count, off, cursor, sorted, padded, colstart, scantmp, counts, costs, icosts, ncand, eoff, nits, ioff, flag;
     DBuf<int2> colcl;
     DBuf<double> bbpart, bbox;
     DBuf<unsigned long long> u64;
@@ -857,10 +855,6 @@ static void inverse_derivative(const double *m, int i, int j, double *o)
     for (int k = 0; k < 9; k++) o[k] *= sc;
 }
 
-// Work items longest-first (and, for the persistent queues, interleaved over
-// the eight per-XCD queues), then the queue bounds.  The main list's items
-// [0, nitems_main) and the image lists' items after them are ordered apart:
-// they run in two launches.
 // The pair count of the last build (synchronises the stream when it is still pending).
 static int resolve_npairs(nbabfs_state *S)
 {
@@ -895,34 +889,33 @@ static int staging_done(hipEvent_t *ev, hipStream_t st)
     return NBABFS_STATUS_CONTINUE;
 }
 
-static int order_items(nbabfs_state *S)
+// Cost of a work item of the image lists (23,559 atoms in a 50 A cell: 137 us per call at the main list's cost per entry,
+// 126 at the image lists' own).
+static int image_item_cost(const nbabfs_options &o)
+{
+    const int per = std::max(1, std::min(o.imageEntriesPerItem > 0 ? o.imageEntriesPerItem : 16, NBABFS_MAX_ENTRIES_PER_ITEM));
+    return std::max(NB_MIN_ITEM_COST, NB_IMAGE_ENTRY_COST * per);
+}
+
+// The cut of the main list for entriesPerItem; the waves the GPU holds at once are five per SIMD (mixed) or three (full
+// FP64).  The persistent queues cut every list alike.
+static ItemCut item_cut(const nbabfs_options &o, int per_item)
+{
+    const int cu = g_cu_count > 0 ? g_cu_count : 256;
+    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 3 : 5);
+    return ItemCut{NB_ENTRY_COST * std::max(1, per_item > 0 ? per_item : 16), o.wavesPerCU > 0 ? 0 : held};
+}
+
+// The queue bounds of the persistent launches: the main list's items [0, nitems_main) in eight runs.
+static int queue_bounds(nbabfs_state *S)
 {
     hipStream_t st = S->stream;
-    const int n = S->nitems_main, ni = S->nitems - S->nitems_main;
-    const int interleave = S->opt.wavesPerCU > 0 ? 1 : 0;
-    std::vector<int> qs(9);
-    if (n + ni > 0) {
-        const int maxcost = NB_SCC * std::max(1, S->opt.entriesPerItem);
-        CHK(S->icost.ensure(std::max(n, ni)));
-        CHK(S->ihist.ensure(maxcost + 1));
-        CHK(S->icur.ensure(maxcost + 1));
-        CHK(S->items2.ensure(n + ni));
-        CHK(S->scantmp.ensure(scan_tmp_size(maxcost + 1)));
-        launch_order_items(S->items.p, n, S->entries.p, maxcost, interleave, S->icost.p, S->ihist.p, S->icur.p,
-                           S->scantmp.p, S->items2.p, st);
-        launch_order_items(S->items.p + n, ni, S->entries.p, maxcost, 0, S->icost.p, S->ihist.p, S->icur.p,
-                           S->scantmp.p, S->items2.p + n, st);
-        HIPCHK(hipGetLastError());
-        S->items.swap(S->items2);
-    }
     S->items_version++;
-    qs[0] = 0;
-    for (int q = 0; q < 8; q++) qs[q + 1] = interleave ? qs[q] + (n - q + 7) / 8 * (n > q) : (int)((long long)n * (q + 1) / 8);
     // Pinned staging: the copy is asynchronous; the staging is rewritten only after it completed.
     CHK(S->h_qs.ensure(9));
     CHK(S->qstarts.ensure(9));
     CHK(staging_free(S->ev_qs));
-    std::memcpy(S->h_qs.p, qs.data(), 9 * sizeof(int));
+    for (int q = 0; q <= 8; q++) S->h_qs.p[q] = (int)((long long)S->nitems_main * q / 8);
     HIPCHK(hipMemcpyAsync(S->qstarts.p, S->h_qs.p, 9 * sizeof(int), hipMemcpyHostToDevice, st));
     CHK(staging_done(&S->ev_qs, st));
     return NBABFS_STATUS_CONTINUE;
@@ -1105,7 +1098,8 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->ncand.ensure(S->nsc));
     // Search, then the entry and item offsets; the totals and the capacity
     // check reach the host through mapped memory in one synchronisation.
-    const int per_item = std::max(1, o.entriesPerItem > 0 ? o.entriesPerItem : 16);
+    const ItemCut cut = item_cut(o, o.entriesPerItem);
+    CHK(S->costs.ensure(S->nsc));
     CHK(S->eoff.ensure(S->nsc + 1));
     CHK(S->nits.ensure(S->nsc));
     CHK(S->ioff.ensure(S->nsc + 1));
@@ -1116,12 +1110,15 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
         CHK(S->flag.ensure(1));
         launch_fill_int(S->flag.p, 1, 0, st);
         launch_search(P, S->nsc, d_xyz, S->slot_atom.p, S->blo.p, S->bhi.p, S->colcl.p, S->scratch.p, S->ncand.p,
-                      S->counts.p, S->flag.p, st);
-        if (!launch_list_offsets(S->counts.p, S->nsc, per_item, S->eoff.p, S->nits.p, S->ioff.p, S->flag.p, S->tail.d,
-                                 st)) {
+                      S->counts.p, S->costs.p, S->flag.p, st);
+        if (!launch_list_offsets(S->counts.p, S->costs.p, S->nsc, cut, S->eoff.p, S->nits.p, S->ioff.p, S->flag.p,
+                                 S->tail.d, st)) {
             launch_scan(S->counts.p, S->eoff.p, S->nsc, S->scantmp.p, st);
-            launch_items_per_sc(S->counts.p, S->nsc, per_item, S->nits.p, st);
+            // A list this long is cut at the nominal cost (the rule's total would have to come to the host first).
+            S->item_units = std::max(NB_MIN_ITEM_COST, cut.most);
+            launch_items_per_sc(S->costs.p, S->nsc, S->item_units, S->nits.p, st);
             launch_scan(S->nits.p, S->ioff.p, S->nsc, S->scantmp.p, st);
+            ((volatile int *)S->tail.h)[3] = S->item_units;
             hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->eoff.p, S->counts.p, S->ioff.p, S->nits.p,
                                S->nsc, S->flag.p, S->tail.d);
         }
@@ -1134,6 +1131,7 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     }
     S->nent = ((volatile int *)S->tail.h)[0];
     S->nitems = ((volatile int *)S->tail.h)[1];
+    S->item_units = ((volatile int *)S->tail.h)[3];
     S->nent_main = S->nent;
     S->nitems_main = S->nitems;
     S->desc_valid = false;
@@ -1144,8 +1142,9 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->items.ensure(S->nitems));
     CHK(S->u64.ensure(2));
     CHK(S->npblock.ensure(S->nsc));
-    launch_compact(S->scratch.p, S->cap, nullptr, S->ncand.p, S->counts.p, S->eoff.p, S->ioff.p, S->nsc, S->nsc,
-                   per_item, 0, S->entries.p, S->items.p, S->u64.p, S->npblock.p, st);
+    launch_compact(S->scratch.p, S->cap, nullptr, S->ncand.p, S->eoff.p, S->nsc, S->entries.p, S->u64.p, S->npblock.p, st);
+    launch_cut_items(S->counts.p, S->costs.p, S->eoff.p, S->ioff.p, S->nits.p, S->nsc, S->nsc, 0, S->entries.p,
+                     S->items.p, st);
     CHK(S->h_np.ensure(1));
     HIPCHK(hipMemcpyAsync(S->h_np.p, S->u64.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     S->np_pending = true;
@@ -1157,7 +1156,7 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->eacc.ensure(NB_EACC_WORDS));
     CHK(S->vacc.ensure(NB_VACC_WORDS));
     CHK(S->energies.ensure(NB_NENERGIES));
-    CHK(order_items(S));
+    CHK(queue_bounds(S));
     CHK(S->heads.ensure(8 * 32));
 
     // Plain path: full CSR rows (both directions).
@@ -1360,6 +1359,9 @@ static void fill_desc(nbabfs_state *S, SysDesc &D, const double *d_xyz, double *
     D.escale = S->escale;
     D.escale14 = S->escale14;
     D.qscale = std::sqrt(S->escale);
+    const AbfsFactors &F = S->F;
+    const double damp[7] = {F.qF0 / F.eScale, -F.qAlpha / F.eScale, F.aF0, F.aAlpha, F.bF0, F.bAlpha, F.qAlpha};
+    std::memcpy(D.damp, damp, sizeof(damp));
     D.n = S->n;
     D.n_pad = S->n_pad;
     D.ncl = S->ncl;
@@ -1381,13 +1383,6 @@ static void fill_desc(nbabfs_state *S, SysDesc &D, const double *d_xyz, double *
     D.eimgpart = (S->opt.precision == NBABFS_PLAIN_FP64 && D.n_img_items > 0) ? S->eimgpart.p : nullptr;
 }
 
-// Entries per work item of the image lists (they run in a launch of their own,
-// one workgroup per item, so smaller items balance the launch).
-static int image_per_item(const nbabfs_options &o)
-{
-    return std::max(1, std::min(o.imageEntriesPerItem > 0 ? o.imageEntriesPerItem : 16, NBABFS_MAX_ENTRIES_PER_ITEM));
-}
-
 // wavesPerCU > 0: persistent grid of that many waves per CU; otherwise one
 // workgroup per work item.
 static int n_persistent_blocks(const nbabfs_options &o, int nitems)
@@ -1407,39 +1402,46 @@ static int launch_force(nbabfs_state *S, ForceGuard g)
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     if (S->opt.precision != NBABFS_PLAIN_FP64) {
         const int nm = S->nitems_main, ni = S->nitems - S->nitems_main;
-        // The image launch runs on the second stream, overlapping the main one.
-        hipStream_t sti = st;
-        if (ni > 0 && nm > 0) {
-            if (!S->stream2) {
-                HIPCHK(hipStreamCreateWithFlags(&S->stream2, hipStreamNonBlocking));
-                HIPCHK(hipEventCreateWithFlags(&S->ev_fork, hipEventDisableTiming));
-                HIPCHK(hipEventCreateWithFlags(&S->ev_join, hipEventDisableTiming));
+        // The image lists' items follow the main list's, and the mixed kernel takes both in one launch.  The full-FP64
+        // and the persistent kernels take main items only: the images' launch then runs beside theirs, on the second
+        // stream.
+        const bool fp64 = S->opt.precision == NBABFS_TILED_FP64;
+        const int n14 = nblk(S->n14, NB_P14_BLOCK);
+        const QueueParams direct{nullptr, S->qstarts.p};
+        if (!fp64 && S->opt.wavesPerCU <= 0) {
+            if (S->timing && nm + ni > 0) CHK(timing_events(S, 2, ev));
+            launch_force_tiled(S->d_desc.p, S->items.p, direct, S->F, nm + ni, S->ntypes, g, st, ni > 0, ev[0], ev[1],
+                               n14, false, 0);
+        } else {
+            const bool fork = ni > 0 && nm > 0;
+            if (fork) {
+                if (!S->stream2) {
+                    HIPCHK(hipStreamCreateWithFlags(&S->stream2, hipStreamNonBlocking));
+                    HIPCHK(hipEventCreateWithFlags(&S->ev_fork, hipEventDisableTiming));
+                    HIPCHK(hipEventCreateWithFlags(&S->ev_join, hipEventDisableTiming));
+                }
+                HIPCHK(hipEventRecord(S->ev_fork, st));
+                HIPCHK(hipStreamWaitEvent(S->stream2, S->ev_fork, 0));
             }
-            HIPCHK(hipEventRecord(S->ev_fork, st));
-            HIPCHK(hipStreamWaitEvent(S->stream2, S->ev_fork, 0));
-            sti = S->stream2;
-        }
-        if (S->timing && nm + ni > 0) CHK(timing_events(S, (ni > 0 && nm > 0) ? 4 : 2, ev));
-        if (ni > 0) {
-            QueueParams q{nullptr, S->qstarts.p};
-            const int o = nm > 0 ? 2 : 0;
-            launch_force_tiled(S->d_desc.p, S->items.p + nm, q, S->F, ni, S->ntypes, image_per_item(S->opt), g, sti,
-                               true, ev[o], ev[o + 1], 0, false, 0);
-        }
-        if (nm > 0) {
-            QueueParams q{S->opt.wavesPerCU > 0 ? S->heads.p : nullptr, S->qstarts.p};
-            launch_force_tiled(S->d_desc.p, S->items.p, q, S->F, n_persistent_blocks(S->opt, nm), S->ntypes,
-                               S->opt.entriesPerItem, g, st, false, ev[0], ev[1], nblk(S->n14, NB_P14_BLOCK),
-                               S->opt.precision == NBABFS_TILED_FP64, 0);
-        } else if (S->n14 > 0) {
-            QueueParams q{nullptr, S->qstarts.p};
-            launch_force_tiled(S->d_desc.p, S->items.p, q, S->F, 0, S->ntypes, S->opt.entriesPerItem, g, st, false,
-                               ni > 0 ? nullptr : ev[0], ni > 0 ? nullptr : ev[1], nblk(S->n14, NB_P14_BLOCK),
-                               S->opt.precision == NBABFS_TILED_FP64, 0);
-        }
-        if (sti != st) {
-            HIPCHK(hipEventRecord(S->ev_join, sti));
-            HIPCHK(hipStreamWaitEvent(st, S->ev_join, 0));
+            const hipStream_t sti = fork ? S->stream2 : st;
+            if (S->timing && nm + ni > 0) CHK(timing_events(S, fork ? 4 : 2, ev));
+            if (ni > 0) {
+                const int o = nm > 0 ? 2 : 0;
+                launch_force_tiled(S->d_desc.p, S->items.p + nm, direct, S->F, ni, S->ntypes, g, sti, true, ev[o],
+                                   ev[o + 1], 0, false, 0);
+            }
+            if (nm > 0) {
+                const QueueParams q{S->opt.wavesPerCU > 0 ? S->heads.p : nullptr, S->qstarts.p};
+                launch_force_tiled(S->d_desc.p, S->items.p, q, S->F, n_persistent_blocks(S->opt, nm), S->ntypes, g, st,
+                                   false, ev[0], ev[1], n14, fp64, 0);
+            } else if (S->n14 > 0) {
+                launch_force_tiled(S->d_desc.p, S->items.p, direct, S->F, 0, S->ntypes, g, st, false,
+                                   ni > 0 ? nullptr : ev[0], ni > 0 ? nullptr : ev[1], n14, fp64, 0);
+            }
+            if (fork) {
+                HIPCHK(hipEventRecord(S->ev_join, sti));
+                HIPCHK(hipStreamWaitEvent(st, S->ev_join, 0));
+            }
         }
     } else {
         const int nm = S->nitems_main, ni = S->nitems - S->nitems_main;
@@ -1482,39 +1484,44 @@ static int mmmm_async(nbabfs_state *S, const double *d_xyz, double *d_grad)
 }
 
 // Cut the compacted entries of the current lists (main, then images) into
-// work items of per_item entries (the entries and their order are unchanged)
-// and order them longest-first.
+// work items for per_item entries per item (the entries and their order are
+// unchanged).
 static int recut_items(nbabfs_state *S, int per_item)
 {
     hipStream_t st = S->stream;
-    per_item = std::max(1, per_item > 0 ? per_item : 16);
-    const int ipi = image_per_item(S->opt);
     if (S->nsc <= 0) return NBABFS_STATUS_CONTINUE;
     const int nb = (int)S->slots.size() * S->nsc;
-    launch_items_per_sc(S->counts.p, S->nsc, per_item, S->nits.p, st);
-    launch_scan(S->nits.p, S->ioff.p, S->nsc, S->scantmp.p, st);
-    hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->eoff.p, S->counts.p, S->ioff.p, S->nits.p, S->nsc,
-                       S->flag.p, S->tail.d);
+    CHK(S->tail.ensure(16));
+    const ItemCut cut = item_cut(S->opt, per_item);
+    if (!launch_list_offsets(S->counts.p, S->costs.p, S->nsc, cut, S->eoff.p, S->nits.p, S->ioff.p, S->flag.p, S->tail.d,
+                             st)) {
+        const int units = std::max(NB_MIN_ITEM_COST, cut.most);
+        launch_items_per_sc(S->costs.p, S->nsc, units, S->nits.p, st);
+        launch_scan(S->nits.p, S->ioff.p, S->nsc, S->scantmp.p, st);
+        ((volatile int *)S->tail.h)[3] = units;
+        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->eoff.p, S->counts.p, S->ioff.p, S->nits.p, S->nsc,
+                           S->flag.p, S->tail.d);
+    }
     if (nb > 0) {
-        launch_items_per_sc(S->icounts.p, nb, ipi, S->inits.p, st);
-        launch_scan(S->inits.p, S->iioff.p, nb, S->scantmp.p, st);
-        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->ieoff.p, S->icounts.p, S->iioff.p, S->inits.p,
-                           nb, S->flag.p, S->tail.d + 4);
+        CHK(S->inits.ensure(nb));
+        CHK(S->iioff.ensure(nb));
+        launch_image_items(S->icosts.p, nb, image_item_cost(S->opt), S->inits.p, S->iioff.p, S->tail.d + 4, st);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     S->nitems_main = ((volatile int *)S->tail.h)[1];
-    const int nimg_items = nb > 0 ? ((volatile int *)S->tail.h)[5] : 0;
+    S->item_units = ((volatile int *)S->tail.h)[3];
+    const int nimg_items = nb > 0 ? ((volatile int *)S->tail.h)[4] : 0;
     S->nitems = S->nitems_main + nimg_items;
     CHK(S->items.ensure(std::max(S->nitems, 1)));
-    launch_cut_items(S->counts.p, S->eoff.p, S->ioff.p, S->nsc, S->nsc, per_item, 0, S->items.p, st);
-    if (nb > 0) {
-        launch_add_int(S->iioff.p, nb, S->nitems_main, st);
-        launch_cut_items(S->icounts.p, S->ieoff.p, S->iioff.p, nb, S->nsc, ipi, 0, S->items.p, st, true);
-    }
+    launch_cut_items(S->counts.p, S->costs.p, S->eoff.p, S->ioff.p, S->nits.p, S->nsc, S->nsc, 0, S->entries.p,
+                     S->items.p, st);
+    if (nb > 0)
+        launch_cut_items(S->icounts.p, S->icosts.p, S->ieoff.p, S->iioff.p, S->inits.p, nb, S->nsc, 0, S->entries.p,
+                         S->items.p + S->nitems_main, st, 1);
     HIPCHK(hipGetLastError());
     S->desc_valid = false;   // the descriptor carries the image item count
-    return order_items(S);
+    return queue_bounds(S);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1712,10 +1719,9 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
             CHK(S->flag.ensure(1));
             launch_fill_int(S->flag.p, 1, 0, st);
             CHK(S->icounts.ensure(nb));
+            CHK(S->icosts.ensure(nb));
             CHK(S->incand.ensure(nb));
             CHK(S->ieoff.ensure(nb + 1));
-            CHK(S->inits.ensure(nb));
-            CHK(S->iioff.ensure(nb + 1));
             hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->isoff.p, S->ibound.p, S->isoff.p,
                                S->ibound.p, nb, S->flag.p, S->tail.d);
             HIPCHK(hipGetLastError());
@@ -1725,27 +1731,21 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
             P.soff = S->isoff.p;
             P.scap = S->ibound.p;
             launch_search_images(P, nsc, ns, d_xyz, S->slot_atom.p, S->blo.p, S->bhi.p, S->iscratch.p, S->incand.p,
-                                 S->icounts.p, S->flag.p, st);
+                                 S->icounts.p, S->icosts.p, S->flag.p, st);
             launch_scan(S->icounts.p, S->ieoff.p, nb, S->scantmp.p, st);
-            const int per_item = image_per_item(o);
-            launch_items_per_sc(S->icounts.p, nb, per_item, S->inits.p, st);
-            launch_scan(S->inits.p, S->iioff.p, nb, S->scantmp.p, st);
-            hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->ieoff.p, S->icounts.p, S->iioff.p,
-                               S->inits.p, nb, S->flag.p, S->tail.d);
+            hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->ieoff.p, S->icounts.p, S->ieoff.p,
+                               S->icounts.p, nb, S->flag.p, S->tail.d);
             HIPCHK(hipGetLastError());
             HIPCHK(hipStreamSynchronize(st));
             if (((volatile int *)S->tail.h)[2] > 0)
                 return fail(NBABFS_STATUS_LOGIC_ERROR, "image search exceeded its candidate bound");
             const int nent_img = ((volatile int *)S->tail.h)[0];
-            const int nit_img = ((volatile int *)S->tail.h)[1];
             launch_add_int(S->ieoff.p, nb, S->nent_main, st);
-            launch_add_int(S->iioff.p, nb, S->nitems_main, st);
             CHK(ensure_entries_keep(S, (size_t)S->nent_main + nent_img, (size_t)S->nent_main));
-            CHK(S->items.ensure((size_t)S->nitems_main + nit_img + 1));
             CHK(S->inpairs.ensure(nb));
             CHK(S->h_inpairs.ensure(nb));
-            launch_compact(S->iscratch.p, 0, S->isoff.p, S->incand.p, S->icounts.p, S->ieoff.p, S->iioff.p, nb, nsc,
-                           per_item, 0, S->entries.p, S->items.p, nullptr, S->inpairs.p, st);
+            launch_compact(S->iscratch.p, 0, S->isoff.p, S->incand.p, S->ieoff.p, nb, S->entries.p, nullptr, S->inpairs.p,
+                           st);
             HIPCHK(hipMemcpyAsync(S->h_inpairs.p, S->inpairs.p, nb * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
             HIPCHK(hipGetLastError());
             HIPCHK(hipStreamSynchronize(st));
@@ -2730,13 +2730,9 @@ static int batch_enqueue(nbabfs_batch *B, hipEvent_t ev_start = nullptr, hipEven
     if (B->mixed) {
         if (B->nitems > 0) {
             QueueParams q{s0->opt.wavesPerCU > 0 ? B->heads.p : nullptr, B->qstarts.p};
-            int maxnt = 0, maxcount = 0;
-            for (auto *s : B->st) {
-                maxnt = std::max(maxnt, s->ntypes);
-                maxcount = std::max(maxcount, s->opt.entriesPerItem);
-            }
-            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt,
-                               maxcount, g, st, false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64);
+            int maxnt = 0;
+            for (auto *s : B->st) maxnt = std::max(maxnt, s->ntypes);
+            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt, g, st, false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64);
         }
     } else {
         launch_force_plain(B->d_desc.p, ns, B->max_n, s0->F, g, st, ev_start, ev_stop);

@@ -44,14 +44,14 @@ struct AbfsFactors {
     double bF3, bK6, bShift6, bF0, bAlpha;
     // Tiled mixed kernel: u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff, and the
     // Coulomb energy divided by eScale, the leading coefficient of P - 1 = eScale (p0 + u (p1 + u (p2 + u))).
-    double uScale, uShift, sOn, p0, p1, p2, eScale, eInv, qShift2e, qF0e, qAlphaE;
+    double uScale, uShift, sOn, p0, p1, p2, eScale, eInv, qShift2e;
     double minus3;              // -3 (an operand in scalar registers, not a pair of vector registers)
 };
 
 struct Entry {              // 80 bytes
     int J;                  // j-cluster (local index)
-    int sc;                 // owning super-cluster
     int cbits;              // bit c set if i-cluster c has any pair with J
+    int sc;                 // owning super-cluster
     int img;                // -1: main list; else the image whose copy of J is paired
     unsigned char bits[NB_SC];  // per lane l = 8a+b: bit c = pair (c,a)-(J,b) listed
 };
@@ -77,13 +77,15 @@ struct ImageXf {            // 160 bytes
 #define NB_GACC_WORDS_PER_SLOT 24
 #define NB_GACC_WORDS_PER_IMAGE (NB_GSLOTS * NB_GACC_WORDS_PER_SLOT)
 
-struct WorkItem {           // 16 bytes
+struct WorkItem {           // 32 bytes
     int sys;                // system index in the batch; image-list items: | (image + 1) << 16
     int sc;                 // super-cluster
     int first;              // first entry
     int count;              // entries
+    int J0;                 // the first entry's j-cluster: its records are asked for without waiting for the entry
+    int pad[3];
 };
-static_assert(sizeof(WorkItem) == 16, "work items are moved as one 16-byte word");
+static_assert(sizeof(WorkItem) == 32, "work items are read as two 16-byte words");
 
 // Everything a per-call kernel needs to know about one system.
 struct SysDesc {
@@ -114,6 +116,7 @@ struct SysDesc {
     double escale;              // Coulomb factor / dielectric
     double escale14;            // times electrostaticScale14
     double qscale;              // sqrt(escale): charges are stored pre-scaled
+    double damp[7];             // mixed kernel, damped region: Coulomb qF0, -qAlpha (over eScale), aF0, aAlpha, bF0, bAlpha, qAlpha
     int n, n_pad, ncl, ntypes, n14;
     int item_first, item_count; // range of this system's items in the batch
     int n_plain_blocks, n14_blocks;
@@ -157,11 +160,11 @@ __device__ __forceinline__ long long rint_i64(double x)
 // integer sums stay defined; the return value says that v was outside
 // (-2^66, 2^66) or NaN, and the callers raise the system's error word
 // (NB_ERR_RANGE) so that the energy call reports it instead of a wrong value.
-__device__ __forceinline__ bool fx_split(double v, long long &hi, long long &lo)
+__device__ __forceinline__ bool fx_split(double v, long long &hi, long long &lo, double limit = 0x1p66)
 {
     const double magic = 6755399441055744.0;
-    const bool bad = !(fabs(v) < 0x1p66);
-    v = fmin(fmax(v, -0x1p66), 0x1p66);
+    const bool bad = !(fabs(v) < limit);
+    v = fmin(fmax(v, -limit), limit);
     const double t = v * (1.0 / NB_FX_HI_UNIT) + magic;
     hi = __double_as_longlong(t) - __double_as_longlong(magic);
     const double r = fma(-(t - magic), NB_FX_HI_UNIT, v);
@@ -169,10 +172,10 @@ __device__ __forceinline__ bool fx_split(double v, long long &hi, long long &lo)
     return bad;
 }
 
-__device__ __forceinline__ bool fx_add(long long *lo_word, long long *hi_word, double v)
+__device__ __forceinline__ bool fx_add(long long *lo_word, long long *hi_word, double v, double limit = 0x1p66)
 {
     long long hi, lo;
-    const bool bad = fx_split(v, hi, lo);
+    const bool bad = fx_split(v, hi, lo, limit);
     if (lo != 0) __hip_atomic_fetch_add(as_global(lo_word), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (hi != 0) __hip_atomic_fetch_add(as_global(hi_word), hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return bad;
@@ -239,7 +242,9 @@ __device__ __forceinline__ double fx_value(const long long *facc, int n_pad, int
 
 // Energy accumulators: [kind][lo word, hi word][slot], kinds 0 = Coulomb and
 // 1 = LJ of the main list, 2 and 3 of the image lists; a work item adds into
-// slot (item % NB_ESLOTS).
+// slot (item % NB_ESLOTS).  The words hold twice the energy (the split's range
+// is 2^67 for it): small lists are cut into up to four times as many items as
+// the nominal cut, and each item is rounded once, at 2^-34 kJ/mol.
 #define NB_ESLOTS 64
 #define NB_EKINDS 4
 #define NB_EACC_WORDS (2 * NB_EKINDS * NB_ESLOTS)

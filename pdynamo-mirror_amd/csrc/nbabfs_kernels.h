@@ -78,6 +78,54 @@ struct ImageStep {
     int pad;
 };
 
+// Work items are runs of one super-cluster's entries of about the same cost.  An entry costs the pair kernel about 205
+// issue cycles per tile (i-cluster of its mask) and 110 of its own: two units per tile and one per entry, 11 for the
+// average entry of a dense system (4.9 tiles).  With equal numbers of entries the longest items had 2.1 times the tiles
+// of the average one, and a launch of one round of waves took as long as they did.
+__host__ __device__ inline int entry_cost(int cbits)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const int tiles = __popc(cbits & 0xff);
+#else
+    const int tiles = __builtin_popcount(cbits & 0xff);
+#endif
+    return tiles ? 2 * tiles + 1 : 0;
+}
+#define NB_ENTRY_COST 11
+#define NB_IMAGE_ENTRY_COST 6  // the average entry of the image lists (a cell's faces)
+#define NB_MIN_ITEM_COST 34     // twice the largest entry's cost: a block's equal steps are then longer than any entry
+
+// The cut of a list: `most` is the nominal cost of an item, `held` the waves the GPU holds at once (0: always the nominal
+// cost).
+struct ItemCut {
+    int most, held;
+};
+
+// Cost per item of a list of nsc blocks with this total cost.  A wave costs about 5 us beside its entries (its start, its
+// sums), so short items lose throughput: 64 droplets of 500 to 20,000 atoms in one call take 422 us with 16 average
+// entries per item, 462 with 8 and 600 with 4, and a state's cut has to serve single calls and batches alike (they give
+// the same bits).  Two rules leave the nominal cost:
+//   * A list of less than held / 16 nominal items (3,500 atoms of water) is one wave's chain long whatever the GPU could
+//     hold: it is cut into held / 16 items, down to a quarter of the nominal cost (648 atoms: 56 -> 42 us per call; such
+//     lists are a few percent of an uneven batch).
+//   * A list of about a whole number of rounds of waves is cut to fill them (20,001 atoms in full FP64: 144 -> 127 us).
+__host__ __device__ inline int item_cost(const ItemCut &c, long long total, int nsc)
+{
+    long long t = c.most;
+    if (c.held > 0) {
+        const long long round = t * c.held, few = c.held / 16;
+        if (total < t * few) {
+            t = total / few > t / 4 ? total / few : t / 4;
+        } else if (total >= round / 2) {
+            // Every block's last item is short: half an item per block.
+            const long long rounds = (total + round / 2) / round, slots = rounds * c.held - nsc / 2;
+            const long long fit = slots > 0 ? total / slots + 1 : t;
+            if (slots > c.held / 2 && (fit > t || rounds > 1)) t = fit;
+        }
+    }
+    return (int)(t > NB_MIN_ITEM_COST ? t : NB_MIN_ITEM_COST);
+}
+
 // List construction (nbabfs_build.hip).
 void launch_bbox(const double *xyz, int n, double *part, int nparts, double *out, hipStream_t s);
 void launch_bin(const double *xyz, int n, const BuildGrid &g, int4 *cellv, int *key, int *count, hipStream_t s);
@@ -97,10 +145,12 @@ void launch_slot_records(const double *xyz, const int *slot_atom, int n_pad, con
                          int4 *scell, hipStream_t s);
 // Self-list search (the records of P.srec / P.scell must describe the current coordinates and cells).
 void launch_search(const SearchParams &P, int nsc, const double *xyz, const int *slot_atom, const float4 *blo,
-                   const float4 *bhi, const int2 *colcl, Entry *scratch, int *ncand, int *counts, int *overflow,
-                   hipStream_t s);
-void launch_cut_items(const int *counts, const int *eoff, const int *ioff, int nblocks, int nsc, int per_item,
-                      int sys, WorkItem *items, hipStream_t s, bool images = false);
+                   const float4 *bhi, const int2 *colcl, Entry *scratch, int *ncand, int *counts, int *costs,
+                   int *overflow, hipStream_t s);
+// images: the number of image items when the blocks are those of the image lists (else 0).
+void launch_cut_items(const int *counts, const int *costs, const int *eoff, const int *ioff, const int *nits,
+                      int nblocks, int nsc, int sys, const Entry *entries, WorkItem *items, hipStream_t s,
+                      int images = 0);
 // Image lists: R'x + T' per transformation (12 doubles each), the stepped image
 // coordinates, the on-grid flags of the current coordinates, the cross search.
 void launch_image_transform(const double *xyz, int n, const double *rt, int ntrans, double *out, hipStream_t s);
@@ -110,27 +160,26 @@ void launch_image_cells(const double *xyz, int n, const BuildGrid &g, int pointc
                         const unsigned char *free_flags, int4 *icell, hipStream_t s);
 void launch_image_grid(const double *ixyz, int n, int nimg, const BuildGrid &g, ImageGrid *igrid, hipStream_t s);
 void launch_search_images(const SearchParams &P, int nsc, int nimg, const double *xyz, const int *slot_atom,
-                          const float4 *blo, const float4 *bhi, Entry *scratch, int *ncand, int *counts, int *overflow,
-                          hipStream_t s);
+                          const float4 *blo, const float4 *bhi, Entry *scratch, int *ncand, int *counts, int *costs,
+                          int *overflow, hipStream_t s);
 // Upper bound of each (image, super-cluster) block's candidates (its scratch capacity).
 void launch_image_bounds(const SearchParams &P, int nsc, int nimg, const float4 *blo, const float4 *bhi, int *bound,
                          hipStream_t s);
 void launch_add_int(int *p, int m, int v, hipStream_t s);
 void launch_export_image_pairs(const Entry *entries, int nent, const int *slot_atom, long long n, int img,
                                unsigned long long *cursor, long long cap, long long *keys, hipStream_t s);
-void launch_order_items(const WorkItem *items, int nitems, const Entry *entries, int maxcost, int interleave, int *cost,
-                        int *hist, int *cursor, int *scantmp, WorkItem *out, hipStream_t s);
-void launch_items_per_sc(const int *counts, int nsc, int per_item, int *nitems, hipStream_t s);
-// Entry and item offsets (exclusive scans of counts and of ceil(counts / per_item)) and the totals
-// {entries, items, *need} into out, in one launch; false (nothing launched) when nsc is beyond its single workgroup.
-bool launch_list_offsets(const int *counts, int nsc, int per_item, int *eoff, int *nits, int *ioff, const int *need,
-                         int *out, hipStream_t s);
-// nblocks compaction blocks (super-cluster = block % nsc); the pairs of each
-// block are stored into npairs_block and, when npairs is given, their sum into *npairs.
-// soff (or null: block * cap) gives each block's scratch offset.
-void launch_compact(const Entry *scratch, int cap, const int *soff, const int *ncand, const int *counts,
-                    const int *eoff, const int *ioff, int nblocks, int nsc, int per_item, int sys, Entry *entries,
-                    WorkItem *items, unsigned long long *npairs, unsigned long long *npairs_block, hipStream_t s);
+// Items per block (ceil(costs / per_item)); the sum of the block costs into mapped host memory.
+void launch_items_per_sc(const int *costs, int nsc, int per_item, int *nitems, hipStream_t s);
+void launch_image_items(const int *costs, int m, int per_item, int *nits, int *ioff, int *out, hipStream_t s);
+// Entry and item offsets (exclusive scans of counts and of ceil(costs / per_item), per_item from the cut and the total
+// cost) and {entries, items, *need, per_item} into out, in one launch; false (nothing launched) when nsc is beyond its
+// single workgroup.
+bool launch_list_offsets(const int *counts, const int *costs, int nsc, const ItemCut &cut, int *eoff, int *nits,
+                         int *ioff, const int *need, int *out, hipStream_t s);
+// nblocks compaction blocks; the pairs of each block are stored into npairs_block and, when npairs is given, their
+// sum into *npairs.  soff (or null: block * cap) gives each block's scratch offset.
+void launch_compact(const Entry *scratch, int cap, const int *soff, const int *ncand, const int *eoff, int nblocks,
+                    Entry *entries, unsigned long long *npairs, unsigned long long *npairs_block, hipStream_t s);
 void launch_export_pairs(const Entry *entries, int nent, const int *slot_atom, long long n,
                          unsigned long long *cursor, long long cap, long long *keys, hipStream_t s);
 void launch_csr_degree(const Entry *entries, int nent, const int *slot_atom, int *deg, hipStream_t s);
@@ -177,7 +226,7 @@ void launch_prepare(const SysDesc *d_desc, int nsys, int max_npad, int tiled, in
 // sys1 >= 0: every item belongs to system sys1 (a single-state launch), so the kernel reads its descriptor without
 // waiting for the items.
 void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const AbfsFactors &F,
-                        int nblocks, int max_ntypes, int max_count, ForceGuard g, hipStream_t s, bool images = false,
+                        int nblocks, int max_ntypes, ForceGuard g, hipStream_t s, bool images = false,
                         hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr, int n14_blocks = 0,
                         bool full_fp64 = false, int sys1 = -1);
 // The 1-4 list in blocks of NB_P14_BLOCK pairs (k_pairs14, or extra waves of a single-state pair launch).

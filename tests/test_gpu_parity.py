@@ -127,6 +127,23 @@ def test_options_14_dielectric(oracle_mod):
     _check(terms, grad, rterms, rgrad, 1e-6, 1e-5, "", o.abs_sums(mm.coordinates3))
 
 
+# Work items of 1 to 128 average entries: one entry per item, an item that ends inside a chunk of 16 entries, items of more
+# than one chunk, and items of more than 64 entries (their headers are read in two parts), from the direct launch
+# (a list large enough to keep the nominal cut) and from the persistent queues.
+@pytest.mark.parametrize("nwater,box,entries,waves", [(216, 18.6, 1, 0), (216, 18.6, 16, 0), (1000, 31.0, 17, 0),
+                                                      (1000, 31.0, 33, 12), (1000, 31.0, 128, 12), (6667, 58.4, 128, 0)])
+@pytest.mark.parametrize("precision,etol,gtol", PATHS[:2])
+def test_work_item_cuts(oracle_mod, nwater, box, entries, waves, precision, etol, gtol):
+    from pdynamo_amd import synthetic
+    mm = synthetic.water_lattice(nwater, box, seed=77)
+    s = _system(mm, precision=precision, entriesPerItem=entries, wavesPerCU=waves)
+    _, terms, grad = _run(s)
+    o = oracle_mod.OracleABFS(mm, nthreads=8)
+    rterms, rgrad, _ = o.energy(mm.coordinates3)
+    assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
+    _check(terms, grad, rterms, rgrad, etol, gtol, "", o.abs_sums(mm.coordinates3))
+
+
 def _water_with_14(nwater, box, seed):
     """Waters on a jittered lattice (no overlapping atoms: the Coulomb and 1-4 terms are not small beside the
     LJ term) plus intermolecular "1-4" pairs between atoms 2.5-5 A apart, excluded from the main list as a
