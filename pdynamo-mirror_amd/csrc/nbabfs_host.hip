@@ -435,7 +435,7 @@ struct nbabfs_state {
     // Coordinates for which the last update already queued the prepare pass
     // and the pair kernel (the energy call on the same array only finalizes).
     const double *forced_xyz = nullptr;
-    MappedInts upflag, tail, prepdone;
+    MappedInts tail, prepdone;
     DBuf<int> dflag;
     DBuf<unsigned long long> prepcount;
     int epoch = 0;
@@ -1252,7 +1252,6 @@ static int update(nbabfs_state *S, const double *d_xyz, int *rebuilt)
     if (!doUpdate && S->has_sym && std::memcmp(S->M, S->Mxf, sizeof(S->M)) != 0) CHK(upload_image_xf(S));
     if (!doUpdate) {
         const double buf = 0.5 * (S->opt.listCutoff - S->opt.outerCutoff);
-        CHK(S->upflag.ensure(1));
         if (!S->dflag.p) {
             CHK(S->dflag.ensure(1));
             CHK(S->prepcount.ensure(1));
@@ -1264,7 +1263,7 @@ static int update(nbabfs_state *S, const double *d_xyz, int *rebuilt)
         CHK(ensure_desc(S, d_xyz, S->last_grad));
         S->epoch = next_epoch(S->epoch);
         const bool plain = S->opt.precision == NBABFS_PLAIN_FP64;
-        PrepareCheck chk{d_xyz, S->xyz_ref.p, S->has_fixed ? S->freef.p : nullptr, buf * buf, S->upflag.d,
+        PrepareCheck chk{d_xyz, S->xyz_ref.p, S->has_fixed ? S->freef.p : nullptr, buf * buf,
                          S->dflag.p, S->epoch, S->prepcount.p, S->prepdone.d};
         errw_before_prepare(S);
         launch_prepare(S->d_desc.p, 1, S->n_pad, plain ? 0 : 1, S->heads.p, chk, st);
@@ -1277,15 +1276,15 @@ static int update(nbabfs_state *S, const double *d_xyz, int *rebuilt)
         // Wait for the test through the mapped completion marker (no event in
         // the stream between the two kernels); the stream is checked as well,
         // so a failed launch cannot leave the host waiting.
-        for (long spin = 0; *(volatile int *)S->prepdone.h != S->epoch; spin++) {
+        for (long spin = 0; std::abs(*(volatile int *)S->prepdone.h) != S->epoch; spin++) {
             if ((spin & 1023) == 1023) {
                 const hipError_t q = hipStreamQuery(st);
                 if (q != hipSuccess && q != hipErrorNotReady) return fail(NBABFS_STATUS_LOGIC_ERROR, "%s", hipGetErrorString(q));
-                if (q == hipSuccess && *(volatile int *)S->prepdone.h != S->epoch)
+                if (q == hipSuccess && std::abs(*(volatile int *)S->prepdone.h) != S->epoch)
                     return fail(NBABFS_STATUS_LOGIC_ERROR, "update test finished without its completion marker");
             }
         }
-        doUpdate = *(volatile int *)S->upflag.h == S->epoch;
+        doUpdate = *(volatile int *)S->prepdone.h < 0;
         if (doUpdate && S->forced_xyz) {
             // The guarded launch returns at once; keep it out of the timing.
             if (S->timing && !S->ev_group.empty()) {
@@ -1468,7 +1467,7 @@ static int mmmm_async(nbabfs_state *S, const double *d_xyz, double *d_grad)
         return NBABFS_STATUS_CONTINUE;
     }
     if (S->forced_xyz != d_xyz) {
-        PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, nullptr, 0, nullptr, nullptr};
+        PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, 0, nullptr, nullptr};
         errw_before_prepare(S);
         launch_prepare(S->d_desc.p, 1, S->n_pad, plain ? 0 : 1, S->heads.p, none, st);
         CHK(launch_force(S, ForceGuard{nullptr, 0}));
@@ -1847,7 +1846,7 @@ static int autotune(nbabfs_state *S, const double *d_xyz, int *best_epi, int *be
     }
     CHK(ensure_call_buffers(S));
     CHK(ensure_desc(S, d_xyz, S->last_grad));
-    PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, nullptr, 0, nullptr, nullptr};
+    PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, 0, nullptr, nullptr};
     errw_before_prepare(S);
     launch_prepare(S->d_desc.p, 1, S->n_pad, 1, S->heads.p, none, st);
     hipEvent_t ev[2 * reps];
@@ -2725,7 +2724,7 @@ static int batch_enqueue(nbabfs_batch *B, hipEvent_t ev_start = nullptr, hipEven
     if (B->max_n > 0)
         hipLaunchKernelGGL(k_check_batch, dim3(nblk(B->max_n, 256), ns), dim3(256), 0, st, B->d_check.p, B->flags.d,
                            B->gguard.p);
-    PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, nullptr, 0, nullptr, nullptr};
+    PrepareCheck none{nullptr, nullptr, nullptr, 0.0, nullptr, 0, nullptr, nullptr};
     launch_prepare(B->d_desc.p, ns, B->max_npad, B->mixed ? 1 : 0, B->heads.p, none, st);
     if (B->mixed) {
         if (B->nitems > 0) {

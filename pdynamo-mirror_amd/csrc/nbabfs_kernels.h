@@ -200,11 +200,11 @@ struct PrepareCheck {
     const double *ref;                 // coordinates of the last list build (null: no test)
     const unsigned char *free_flags;   // null: every atom is free
     double bufsq;                      // (half the list buffer)^2
-    int *flag;                         // host-mapped: receives epoch when some free atom moved too far
-    int *dflag;                        // device copy of the same flag (read by ForceGuard)
+    int *dflag;                        // device: receives epoch when some free atom moved too far (read by ForceGuard)
     int epoch;
     unsigned long long *counter;       // device: blocks finished << 32 | blocks with a moved atom (reset by the last)
-    int *done;                         // host-mapped: receives epoch once every block has finished
+    int *done;                         // host-mapped: once every block has finished, receives epoch, negative when some
+                                       // free atom moved too far
 };
 
 // A force launch queued before the update decision is known: every
