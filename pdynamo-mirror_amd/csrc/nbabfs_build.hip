@@ -396,18 +396,13 @@ __device__ __forceinline__ float box_gap2(float4 alo, float4 ahi, float4 blo, fl
 // 1020-1150): both atoms in the MM selection, not excluded, OR selection (free atoms), and either the grid
 // rule (both on grid; stencil flag 2 = whole cell pair within the cutoff,
 // 1 = FP64 distance test, 0 = out of range) or, for the direct method, the
-// FP64 distance test alone.  The self-list evaluation computes every part of
-// it without branches (a tile's lanes all take the same path); only the
-// exclusion scan, needed when j falls inside i's excluded index range, is a
-// branch.
-//
-// STEN (self lists): 0 direct method, 1 grid with the stencil in LDS, 2 grid
-// with the stencil read from global memory (more than NB_STENCIL_LDS cells).
+// FP64 distance test alone (search_eval_self says when that decides for the
+// grid too).  GRID (self lists): the grid method.
 // ------------------------------------------------------------------------------------------------
+#define NB_STENCIL_LDS 4096  // point/cell search: stencil bytes held in LDS (u <= 7)
 #define NB_SEARCH_WAVES 8
 #define NB_SEARCH_THREADS (64 * NB_SEARCH_WAVES)
 #define NB_XPOOL 1024        // exclusion indices of one super-cluster held in LDS
-#define NB_STENCIL_LDS 4096  // stencil bytes held in LDS (u <= 7)
 #define NB_CAND 1024         // candidate list: flushed once it holds more than NB_CAND - NB_SEARCH_THREADS
 #define NB_MAXCOL 256        // x-y columns handled per flattened scan
 
@@ -535,89 +530,94 @@ __device__ __forceinline__ int search_eval_cross(const SearchParams &P, int npen
     return nvalid;
 }
 
+// One pair's full rule (self lists): both atoms real, in the MM selection and (grid) on the grid, one of them free; the
+// cell offset + u per axis (ic holds the cell - u) in [0, 2u] within the stencil; near: the FP64 distance test.
+// PC (point/cell grid search, PairListGenerator.c:1155-1218): the atom with the higher index is the point and the other
+// atom's cell is searched.  The pair is listed when that cell is in the stencil around the point's search cell, the
+// point/cell smallest squared distance is below cutoff^2, and either the largest is at most cutoff^2 (the cell is taken
+// whole) or the FP64 distance test passes.  The lower-index atom must be on the grid; the point may be off it (its
+// record then holds its search cell, see k_slot_records).
+template <bool GRID, bool PC>
+__device__ __forceinline__ bool pair_rule(const SearchParams &P, const unsigned char *sSten, const double4 &ip, const int4 &ic, const double4 &jp,
+                                          const int4 &jc, bool near)
+{
+    const unsigned wst = 2 * P.u + 1, nst = wst * wst * wst;
+    const int jatom = __double2loint(jp.w), jfl = __double2hiint(jp.w);
+    bool ok;
+    if (PC) {
+        const bool ipt = __double2loint(ip.w) > jatom;      // i is the point
+        ok = (((ic.w | jfl) & (NB_SF_FREE | NB_SF_QC | NB_SF_EMPTY)) == NB_SF_FREE) & !((ipt ? jfl : ic.w) & NB_SF_OFFGRID);
+    } else {
+        ok = ((ic.w | jfl) & (NB_SF_FREE | NB_SF_QC | NB_SF_OFFGRID | NB_SF_EMPTY)) == NB_SF_FREE;
+    }
+    if (!GRID) return ok & near;
+    const unsigned ux = (unsigned)(jc.x - ic.x), uy = (unsigned)(jc.y - ic.y), uz = (unsigned)(jc.z - ic.z);
+    const bool inb = max(max(ux, uy), uz) < wst;
+    const unsigned si = min((ux * wst + uy) * wst + uz, nst - 1u);
+    const int flag = PC && nst <= NB_STENCIL_LDS ? (int)sSten[si] : (int)P.stencil[si];
+    if (PC) {
+        // The stencil is symmetric, so the offset between the two search cells decides membership in either direction.
+        const bool ipt = __double2loint(ip.w) > jatom;
+        double minR2, maxR2;
+        point_cell_r2(P.glower, P.gh, ipt ? ip.x : jp.x, ipt ? ip.y : jp.y, ipt ? ip.z : jp.z, ipt ? jc.x : ic.x + P.u,
+                      ipt ? jc.y : ic.y + P.u, ipt ? jc.z : ic.z + P.u, minR2, maxR2);
+        return ok & inb & (flag != 0) & (minR2 < P.cutoff2) & ((maxR2 <= P.cutoff2) | near);
+    }
+    return ok & inb & ((flag == 2) | ((flag == 1) & near));
+}
+
 // Self lists: the candidates sCand[0..npend) of one wave.  Lane 8a + b
 // evaluates i-atom (c, a) of each listed tile c against j-atom b; lanes with
-// b < a hold the lower triangle of the self tile (J = I0 + c).  Every part of
-// the rule is computed without branches; only the exclusion scan (j inside
-// i's excluded index range) branches.
+// b < a hold the lower triangle of the self tile (J = I0 + c).
 //
-// PC (point/cell grid search, PairListGenerator.c:1155-1218): the atom with
-// the higher index is the point and the other atom's cell is searched.  The
-// pair is listed when that cell is in the stencil around the point's search
-// cell, the point/cell smallest squared distance is below cutoff^2, and either
-// the largest is at most cutoff^2 (the cell is taken whole) or the FP64
-// distance test passes.  The lower-index atom must be on the grid; the point
-// may be off it (its record then holds its search cell, see k_slot_records).
-template <int STEN, bool PC>
+// Bound by the instructions of the tile test: about 1.5 million tiles for 100,002 atoms at some 45 vector instructions
+// each for the full rule, 160 us.  The cell rule differs from the plain distance test only where a distance equals the
+// cutoff to rounding: cells hold their atoms, so flag 2 (the whole cell pair in reach) has no pair beyond the cutoff and
+// flag 0 none within it, but for the rounding of the cell an atom is put in (at most 1e-11 A for the spans check_box
+// takes).  So a tile is decided by the distance test alone (145 us) unless one of its lanes lies within the band
+// [P.inner2, P.outer2] around the cutoff, 1e-9 of it wide or more; such a tile takes the full rule.  An atom that is in
+// no pair (QC, off the grid, an empty slot) has an infinite x, which fails the test.
+template <bool GRID, bool PC>
 __device__ __forceinline__ int search_eval_self(const SearchParams &P, int npend, int w, int lane, int I0, int sc,
                                                 int base, int scap, size_t sbase, const int *sCand,
                                                 const unsigned char *sCm, const double4 *sIp, const int4 *sIc,
                                                 const int2 *sIxr, const int *sXoff, const int *sXcnt,
-                                                const int *sXpool, const unsigned char *sSten,
+                                                const int *sXpool, const unsigned char *sSten, bool fixed,
                                                 Entry *__restrict__ scratch, int &ncost)
 {
     const int a = lane >> 3, b = lane & 7;
-    const unsigned wst = 2 * P.u + 1, nst = wst * wst * wst;
+    const bool lower = b < a;
     int nvalid = 0;
     double4 jpn = make_double4(0.0, 0.0, 0.0, 0.0);
-    int4 jcn = make_int4(0, 0, 0, 0);
-    if (w < npend) {
-        const int Jn = sCand[w];
-        jpn = P.srec[Jn * NB_CL + b];
-        if (STEN) jcn = P.scell[Jn * NB_CL + b];
-    }
+    if (w < npend) jpn = P.srec[sCand[w] * NB_CL + b];
     for (int k = w; k < npend; k += NB_SEARCH_WAVES) {
-        const double4 jp = jpn;
-        const int4 jc = jcn;
+        double4 jp = jpn;
         const int Jc = __builtin_amdgcn_readfirstlane(sCand[k]);
         const int cmc = __builtin_amdgcn_readfirstlane(sCm[k]);
-        if (k + NB_SEARCH_WAVES < npend) {
-            const int Jn = sCand[k + NB_SEARCH_WAVES];
-            jpn = P.srec[Jn * NB_CL + b];
-            if (STEN) jcn = P.scell[Jn * NB_CL + b];
-        }
+        if (k + NB_SEARCH_WAVES < npend) jpn = P.srec[sCand[k + NB_SEARCH_WAVES] * NB_CL + b];
         const int jatom = __double2loint(jp.w), jfl = __double2hiint(jp.w);
+        int4 jc = make_int4(0, 0, 0, 0);
+        if (PC) jc = P.scell[Jc * NB_CL + b];
+        const double jx = (!PC && (jfl & (NB_SF_QC | NB_SF_OFFGRID | NB_SF_EMPTY))) ? __builtin_inf() : jp.x;
         int lbits = 0, cbits = 0;
 #pragma unroll
         for (int c = 0; c < NB_SCC; c++) {
             if (!(cmc & (1 << c))) continue;
             const int li = c * NB_CL + a;
             const double4 ip = sIp[li];
-            const int4 ic = sIc[li];
             const int2 xr = sIxr[li];
-            // Both atoms real, in the MM selection and (grid) on the grid, one of them free.
             bool ok;
             if (PC) {
-                const bool ipt = __double2loint(ip.w) > jatom;      // i is the point
-                ok = (((ic.w | jfl) & (NB_SF_FREE | NB_SF_QC | NB_SF_EMPTY)) == NB_SF_FREE) &
-                     !((ipt ? jfl : ic.w) & NB_SF_OFFGRID);
+                ok = pair_rule<true, true>(P, sSten, ip, sIc[li], jp, jc,
+                                           ref_dist2(ip.x, ip.y, ip.z, jp.x, jp.y, jp.z) <= P.cutoff2);
             } else {
-                ok = ((ic.w | jfl) & (NB_SF_FREE | NB_SF_QC | NB_SF_OFFGRID | NB_SF_EMPTY)) == NB_SF_FREE;
+                const double r2 = ref_dist2(ip.x, ip.y, ip.z, jx, jp.y, jp.z);
+                ok = r2 <= (GRID ? P.inner2 : P.cutoff2);
+                if (GRID && __ballot(ok) != __ballot(r2 <= P.outer2))
+                    ok = pair_rule<true, false>(P, sSten, ip, sIc[li], jp, P.scell[Jc * NB_CL + b], r2 <= P.cutoff2);
+                if (fixed) ok = ok & (((__double2hiint(ip.w) | jfl) & NB_SF_FREE) != 0);
             }
-            ok = ok & ((Jc < I0 + c) | (b < a));
-            const bool near = ref_dist2(ip.x, ip.y, ip.z, jp.x, jp.y, jp.z) <= P.cutoff2;
-            if (PC) {
-                // The stencil is symmetric, so the offset between the two search cells decides membership in
-                // either direction.
-                const unsigned ux = (unsigned)(jc.x - ic.x), uy = (unsigned)(jc.y - ic.y), uz = (unsigned)(jc.z - ic.z);
-                const bool inb = max(max(ux, uy), uz) < wst;
-                const unsigned si = min((ux * wst + uy) * wst + uz, nst - 1u);
-                const int flag = STEN == 1 ? (int)sSten[si] : (int)P.stencil[si];
-                const bool ipt = __double2loint(ip.w) > jatom;
-                double minR2, maxR2;
-                point_cell_r2(P.glower, P.gh, ipt ? ip.x : jp.x, ipt ? ip.y : jp.y, ipt ? ip.z : jp.z, ipt ? jc.x : ic.x + P.u,
-                              ipt ? jc.y : ic.y + P.u, ipt ? jc.z : ic.z + P.u, minR2, maxR2);
-                ok = ok & inb & (flag != 0) & (minR2 < P.cutoff2) & ((maxR2 <= P.cutoff2) | near);
-            } else if (STEN) {
-                // Cell offset + u per axis (sIc holds the cell - u), in [0, 2u] within the stencil.
-                const unsigned ux = (unsigned)(jc.x - ic.x), uy = (unsigned)(jc.y - ic.y), uz = (unsigned)(jc.z - ic.z);
-                const bool inb = max(max(ux, uy), uz) < wst;
-                const unsigned si = min((ux * wst + uy) * wst + uz, nst - 1u);
-                const int flag = STEN == 1 ? (int)sSten[si] : (int)P.stencil[si];
-                ok = ok & inb & ((flag == 2) | ((flag == 1) & near));
-            } else {
-                ok = ok & near;
-            }
+            if (Jc >= I0 + c) ok = ok & lower;      // the self tile (a later cluster is never listed)
             const bool inx = ok & (jatom >= xr.x) & (jatom <= xr.y);
             if (__ballot(inx)) {
                 if (inx) {
@@ -643,7 +643,7 @@ __device__ __forceinline__ int search_eval_self(const SearchParams &P, int npend
 // no exclusions, every (i, j) pair including an atom with its own image, the
 // OR selection, i on the reference grid (grid method), and the FP64 distance
 // test against the image coordinates GenerateImageLists produced.
-template <bool CROSS, int STEN, bool PC = false>
+template <bool CROSS, bool GRID, bool PC = false>
 __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_eu((CROSS || PC) ? 1 : 8))) void k_search(SearchParams P, const double *__restrict__ xyz,
                                                               const int *__restrict__ slot_atom,
                                                               const float4 *__restrict__ blo,
@@ -677,13 +677,15 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
     __shared__ int2 sIxr[CROSS ? 1 : NB_SC];
     __shared__ int sXoff[CROSS ? 1 : NB_SC], sXcnt[CROSS ? 1 : NB_SC];
     __shared__ int sXpool[CROSS ? 1 : NB_XPOOL];
-    __shared__ unsigned char sSten[STEN == 1 ? NB_STENCIL_LDS : 1];
+    constexpr bool STENCIL = PC && !CROSS;
+    __shared__ unsigned char sSten[STENCIL ? NB_STENCIL_LDS : 1];
+    __shared__ int sFixed;
     __shared__ int sCand[NB_CAND];
     __shared__ unsigned char sCm[NB_CAND];
     __shared__ int sColStart[NB_MAXCOL], sColPre[NB_MAXCOL + 1];
     __shared__ int sWcnt[NB_SEARCH_WAVES], sWcost[NB_SEARCH_WAVES];
 
-    // Stage the super-cluster (wave 0) and the stencil (all waves).
+    // Stage the super-cluster (wave 0).
     if (w == 0) {
         if (lane < NB_SCC) {
             sIlo[lane] = blo[I0 + lane];
@@ -703,7 +705,11 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
             const double4 ip = P.srec[I0 * NB_CL + lane];
             const int4 ic = P.scell[I0 * NB_CL + lane];
             const int ia = __double2loint(ip.w);
+            const int ifl = __double2hiint(ip.w);
             sIp[lane] = ip;
+            if (!PC && (ifl & (NB_SF_QC | NB_SF_OFFGRID | NB_SF_EMPTY))) sIp[lane].x = __builtin_inf();
+            const unsigned long long fixed = __ballot(!(ifl & (NB_SF_FREE | NB_SF_EMPTY)));
+            if (lane == 0) sFixed = fixed != 0ull ? 1 : 0;
             sIc[lane] = make_int4(ic.x - P.u, ic.y - P.u, ic.z - P.u, __double2hiint(ip.w));
             int xs = 0, xc = 0;
             if (ia >= 0) {
@@ -728,10 +734,11 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
             sIxr[lane] = xc > 0 ? make_int2(P.xidx[xs], P.xidx[xs + xc - 1]) : make_int2(0, -1);
         }
     }
-    const int wst = 2 * P.u + 1;
-    const int nst = wst * wst * wst;
-    if (STEN == 1)
-        for (int k = tid; k < nst; k += NB_SEARCH_THREADS) sSten[k] = P.stencil[k];
+    if (STENCIL) {
+        const int wst = 2 * P.u + 1, nst = wst * wst * wst;
+        if (nst <= NB_STENCIL_LDS)
+            for (int k = tid; k < nst; k += NB_SEARCH_THREADS) sSten[k] = P.stencil[k];
+    }
     __syncthreads();
 
     float4 lo = sIlo[0], hi = sIhi[0];
@@ -772,8 +779,8 @@ __global__ __launch_bounds__(NB_SEARCH_THREADS) __attribute__((amdgpu_waves_per_
                 nvalid += search_eval_cross<PC>(P, npend, w, lane, I0, sc, img, base, scap, sbase, sCand, sCm, sIatom,
                                                 sIfree, sIcell, sIx, sIy, sIz, G, jxyz, slot_atom, scratch, ncost);
             else
-                nvalid += search_eval_self<STEN, PC>(P, npend, w, lane, I0, sc, base, scap, sbase, sCand, sCm, sIp, sIc,
-                                                 sIxr, sXoff, sXcnt, sXpool, sSten, scratch, ncost);
+                nvalid += search_eval_self<GRID, PC>(P, npend, w, lane, I0, sc, base, scap, sbase, sCand, sCm, sIp, sIc, sIxr,
+                                                     sXoff, sXcnt, sXpool, sSten, sFixed != 0, scratch, ncost);
         };
 
         int npend = 0;
@@ -1506,26 +1513,16 @@ void launch_search(const SearchParams &P, int nsc, const double *xyz, const int 
                    int *overflow, hipStream_t s)
 {
     if (nsc <= 0) return;
-    const int wst = 2 * P.u + 1;
-    const int sten = !P.use_grid ? 0 : (wst * wst * wst <= NB_STENCIL_LDS ? 1 : 2);
-    if (sten != 0 && P.pointcell) {
-        if (sten == 1)
-            hipLaunchKernelGGL((k_search<false, 1, true>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom,
-                               blo, bhi, colcl, scratch, ncand, counts, costs, overflow);
-        else
-            hipLaunchKernelGGL((k_search<false, 2, true>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom,
-                               blo, bhi, colcl, scratch, ncand, counts, costs, overflow);
-        return;
-    }
-    if (sten == 0)
-        hipLaunchKernelGGL((k_search<false, 0>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, costs, overflow);
-    else if (sten == 1)
-        hipLaunchKernelGGL((k_search<false, 1>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, costs, overflow);
+    const dim3 grid(nsc), block(NB_SEARCH_THREADS);
+    if (!P.use_grid)
+        hipLaunchKernelGGL((k_search<false, false>), grid, block, 0, s, P, xyz, slot_atom, blo, bhi, colcl, scratch, ncand,
+                           counts, costs, overflow);
+    else if (P.pointcell)
+        hipLaunchKernelGGL((k_search<false, true, true>), grid, block, 0, s, P, xyz, slot_atom, blo, bhi, colcl, scratch,
+                           ncand, counts, costs, overflow);
     else
-        hipLaunchKernelGGL((k_search<false, 2>), dim3(nsc), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo, bhi,
-                           colcl, scratch, ncand, counts, costs, overflow);
+        hipLaunchKernelGGL((k_search<false, true>), grid, block, 0, s, P, xyz, slot_atom, blo, bhi, colcl, scratch, ncand,
+                           counts, costs, overflow);
 }
 
 void launch_search_images(const SearchParams &P, int nsc, int nimg, const double *xyz, const int *slot_atom,
@@ -1534,10 +1531,10 @@ void launch_search_images(const SearchParams &P, int nsc, int nimg, const double
 {
     if (nsc <= 0 || nimg <= 0) return;
     if (P.use_grid && P.pointcell)
-        hipLaunchKernelGGL((k_search<true, 0, true>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz,
+        hipLaunchKernelGGL((k_search<true, false, true>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz,
                            slot_atom, blo, bhi, (const int2 *)nullptr, scratch, ncand, counts, costs, overflow);
     else
-        hipLaunchKernelGGL((k_search<true, 0>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo,
+        hipLaunchKernelGGL((k_search<true, false>), dim3(nsc, nimg), dim3(NB_SEARCH_THREADS), 0, s, P, xyz, slot_atom, blo,
                            bhi, (const int2 *)nullptr, scratch, ncand, counts, costs, overflow);
 }
 

@@ -1074,6 +1074,9 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     SearchParams P;
     std::memset(&P, 0, sizeof(P));
     P.cutoff2 = o.listCutoff * o.listCutoff;
+    const double band = 1.0e-9 * P.cutoff2 + 1.0e-9 * o.listCutoff + 1.0e-15;
+    P.inner2 = P.cutoff2 - band;
+    P.outer2 = P.cutoff2 + band;
     P.stencil = S->stencil.p;
     P.u = S->u;
     P.use_grid = g.use_grid;

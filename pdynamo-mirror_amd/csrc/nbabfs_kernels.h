@@ -27,6 +27,7 @@ struct ImageGrid {
 
 struct SearchParams {
     double cutoff2;                       // listCutoff^2 (FP64 test)
+    double inner2, outer2;                // grid method: the distance test decides outside [inner2, outer2]
     const unsigned char *stencil;         // (2u+1)^3 flags
     int u;
     int use_grid;

@@ -144,6 +144,28 @@ def test_work_item_cuts(oracle_mod, nwater, box, entries, waves, precision, etol
     _check(terms, grad, rterms, rgrad, etol, gtol, "", o.abs_sums(mm.coordinates3))
 
 
+# Distances equal to the list cutoff, exactly or to rounding: a lattice of 9/4 A has its 6 0 0 and 4 4 2 neighbours at
+# 13.5 A, on cell boundaries too; and atoms moved by 1e-13 to 1e-7 A, inside and outside the band in which the search takes
+# the whole cell rule.
+@pytest.mark.parametrize("factor", [0.5, 0.37, 1.0])
+@pytest.mark.parametrize("shift", [0.0, 1.0e-13, 1.0e-10, 1.0e-8, 1.0e-7])
+def test_pairs_at_the_list_cutoff(oracle_mod, shift, factor):
+    from pdynamo_amd import NBModelABFS, PairListGenerator, System, synthetic
+    n = 19
+    mm = synthetic.random_small_system(n ** 3, 40.0, 5)
+    grid = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    rng = np.random.default_rng(6)
+    mm.coordinates3 = 2.25 * grid + shift * rng.uniform(-1.0, 1.0, (n ** 3, 3))
+    gen = PairListGenerator(cutoff=13.5, cutoffCellSizeFactor=factor, useGridByCell=True, sortIndices=False,
+                            minimumPoints=500, minimumCellExtent=2)
+    s = System.FromSynthetic(mm)
+    s.DefineNBModel(NBModelABFS(generator=gen))
+    _run(s)
+    o = oracle_mod.OracleABFS(mm, cell_factor=factor)
+    o.energy(mm.coordinates3)
+    assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
+
+
 def _water_with_14(nwater, box, seed):
     """Waters on a jittered lattice (no overlapping atoms: the Coulomb and 1-4 terms are not small beside the
     LJ term) plus intermolecular "1-4" pairs between atoms 2.5-5 A apart, excluded from the main list as a
