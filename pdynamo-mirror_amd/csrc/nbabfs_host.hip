@@ -121,24 +121,25 @@ struct PinBuf {
     ~PinBuf() { release(); }
 };
 
-// Coherent pinned host memory that kernels write directly (rebuild flags):
-// the host reads it after the stream has synchronised, with no copy.
-struct MappedInts {
-    int *h = nullptr;
-    int *d = nullptr;
+// Coherent pinned host memory that kernels write directly (rebuild flags,
+// energies): the host reads it after the stream has synchronised, with no copy.
+template <typename T>
+struct MappedBuf {
+    T *h = nullptr;
+    T *d = nullptr;
     size_t cap = 0;
     int ensure(size_t m)
     {
         if (h && m <= cap) return NBABFS_STATUS_CONTINUE;
         release();
         size_t mm = std::max<size_t>(m, 16);
-        if (hipHostMalloc((void **)&h, mm * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        if (hipHostMalloc((void **)&h, mm * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
             hipHostGetDevicePointer((void **)&d, h, 0) != hipSuccess) {
             (void)hipGetLastError();
             release();
-            return fail(NBABFS_STATUS_OUT_OF_MEMORY, "mapped host allocation of %zu bytes failed", mm * sizeof(int));
+            return fail(NBABFS_STATUS_OUT_OF_MEMORY, "mapped host allocation of %zu bytes failed", mm * sizeof(T));
         }
-        std::memset(h, 0, mm * sizeof(int));
+        std::memset(h, 0, mm * sizeof(T));
         cap = mm;
         return NBABFS_STATUS_CONTINUE;
     }
@@ -148,7 +149,7 @@ struct MappedInts {
         h = d = nullptr;
         cap = 0;
     }
-    ~MappedInts() { release(); }
+    ~MappedBuf() { release(); }
 };
 
 // Epochs written by the update test; never 0, the initial flag value.
@@ -418,14 +419,14 @@ struct nbabfs_state {
     DBuf<double4> xyzq;
     DBuf<int> styp;
     DBuf<long long> facc;
-    DBuf<double> epart14, eplain, gplain, energies, eimgpart;
+    DBuf<double> epart14, eplain, gplain, eimgpart;
     DBuf<long long> eacc, vacc;
     DBuf<int> errw;                // error word of the per-call kernels (NB_ERR_* bits)
     bool err_dirty = false;        // a prepare pass ran since the last finalize pass read errw
     DBuf<SysDesc> d_desc;
     DBuf<int> heads, qstarts;
     PinBuf<SysDesc> h_desc;
-    PinBuf<double> h_energies, h_grad;
+    PinBuf<double> h_grad;
     SysDesc desc_shadow;           // the descriptor last uploaded to d_desc (valid when desc_valid)
     bool desc_valid = false;
     long items_version = 0;        // bumped whenever the work items are cut or ordered anew
@@ -435,7 +436,10 @@ struct nbabfs_state {
     // Coordinates for which the last update already queued the prepare pass
     // and the pair kernel (the energy call on the same array only finalizes).
     const double *forced_xyz = nullptr;
-    MappedInts tail, prepdone;
+    MappedBuf<int> tail, prepdone;
+    // Outputs of the last call (NB_NENERGIES), written by the finalize pass: a copy back after the kernels cost a launch
+    // and 4 us of each call (648 atoms: 42 us per call with the copy, 37 us without).
+    MappedBuf<double> energies;
     DBuf<int> dflag;
     DBuf<unsigned long long> prepcount;
     int epoch = 0;
@@ -1353,7 +1357,7 @@ static void fill_desc(nbabfs_state *S, SysDesc &D, const double *d_xyz, double *
     D.vacc = S->vacc.p;
     D.epart14 = S->epart14.p;
     D.eplain = S->eplain.p;
-    D.energies = S->energies.p;
+    D.energies = S->energies.d;
     D.err = S->errw.p;
     D.rowptr = S->csrValid ? S->rowptr.p : nullptr;
     D.cols = S->csrValid ? S->cols.p : nullptr;
@@ -1465,7 +1469,7 @@ static int mmmm_async(nbabfs_state *S, const double *d_xyz, double *d_grad)
     // finalize pass, which reads the descriptor after the pair kernel.
     CHK(ensure_desc(S, d_xyz, d_grad));
     if (S->n == 0) {
-        launch_fill_int((int *)S->energies.p, 2 * NB_NENERGIES, 0, st);
+        launch_fill_int((int *)S->energies.d, 2 * NB_NENERGIES, 0, st);
         HIPCHK(hipGetLastError());
         return NBABFS_STATUS_CONTINUE;
     }
@@ -2167,18 +2171,15 @@ extern "C" int nbabfs_mmmm_energy_async(nbabfs_state *S, const double *d_xyz, do
 extern "C" int nbabfs_energies(nbabfs_state *S, double *energies, int *present)
 {
     if (!S || !energies) return fail(NBABFS_STATUS_INVALID_ARGUMENT, "null argument");
-    CHK(S->h_energies.ensure(NB_NENERGIES));
     CHK(S->energies.ensure(NB_NENERGIES));
-    HIPCHK(hipMemcpyAsync(S->h_energies.p, S->energies.p, NB_NENERGIES * sizeof(double), hipMemcpyDeviceToHost,
-                          S->stream));
     HIPCHK(hipStreamSynchronize(S->stream));
-    std::memcpy(energies, S->h_energies.p, 4 * sizeof(double));
+    std::memcpy(energies, S->energies.h, 4 * sizeof(double));
     CHK(resolve_npairs(S));
     if (present) {
         present[0] = S->npairs > 0;
         present[1] = S->n14 > 0;
     }
-    return call_status((int)S->h_energies.p[NB_ESTATUS], "energy call");
+    return call_status((int)S->energies.h[NB_ESTATUS], "energy call");
 }
 
 extern "C" int nbabfs_energy_host(nbabfs_state *S, const double *xyz, double *grad_inout, double *energies,
@@ -2357,9 +2358,7 @@ extern "C" int nbabfs_image_terms(nbabfs_state *S, double *energies, double *dEd
     if (!S) return fail(NBABFS_STATUS_INVALID_ARGUMENT, "state is NULL");
     hipStream_t st = S->stream;
     const int ns = (int)S->slots.size();
-    CHK(S->h_energies.ensure(NB_NENERGIES));
     CHK(S->energies.ensure(NB_NENERGIES));
-    HIPCHK(hipMemcpyAsync(S->h_energies.p, S->energies.p, NB_NENERGIES * sizeof(double), hipMemcpyDeviceToHost, st));
     if (dEdM && ns > 0) {
         CHK(S->h_gacc.ensure((size_t)NB_GACC_WORDS_PER_IMAGE * ns));
         HIPCHK(hipMemcpyAsync(S->h_gacc.p, S->gacc.p, (size_t)NB_GACC_WORDS_PER_IMAGE * ns * sizeof(long long),
@@ -2367,11 +2366,11 @@ extern "C" int nbabfs_image_terms(nbabfs_state *S, double *energies, double *dEd
     }
     HIPCHK(hipStreamSynchronize(st));
     if (energies) {
-        energies[0] = S->h_energies.p[4];
-        energies[1] = S->h_energies.p[5];
+        energies[0] = S->energies.h[4];
+        energies[1] = S->energies.h[5];
     }
     if (present) *present = S->nimages > 0;
-    CHK(call_status((int)S->h_energies.p[NB_ESTATUS], "energy call"));
+    CHK(call_status((int)S->energies.h[NB_ESTATUS], "energy call"));
     if (!dEdM || ns == 0) return NBABFS_STATUS_CONTINUE;
     const double *o = S->grid.corg;
     for (int k = 0; k < ns; k++) {
@@ -2590,14 +2589,13 @@ struct nbabfs_batch {
     PinBuf<SysDesc> h_desc;
     DBuf<WorkItem> items;
     DBuf<int> heads, qstarts;
-    MappedInts flags;               // [k]: epoch when system k must be rebuilt; [nsys]: epoch of the last test
+    MappedBuf<int> flags;               // [k]: epoch when system k must be rebuilt; [nsys]: epoch of the last test
     // Guard words of the batch's passes: [0] the epoch when some system must be rebuilt, [1] the test's epoch.
     DBuf<int> gguard;
     std::vector<CheckDesc> check_shadow;   // the test's descriptors on the device
     DBuf<CheckDesc> d_check;
     PinBuf<CheckDesc> h_check;
-    PinBuf<double> h_energies;
-    DBuf<double> energies;
+    MappedBuf<double> energies;     // NB_NENERGIES per system
     int nitems = 0, max_npad = 0, max_n = 0, max_n14b = 0;
     std::vector<SysDesc> shadow;   // the descriptors of the current layout (graph_valid implies they are current)
     bool layout_valid = false;
@@ -2693,7 +2691,7 @@ static int batch_layout(nbabfs_batch *B, const double *const *d_xyz, double *con
         CHK(ensure_call_buffers(s));
         SysDesc &D = B->h_desc.p[k];
         fill_desc(s, D, d_xyz[k], d_grad ? d_grad[k] : nullptr);
-        D.energies = B->energies.p + NB_NENERGIES * (size_t)k;
+        D.energies = B->energies.d + NB_NENERGIES * (size_t)k;
         const int padded = nblk(s->nitems, NB_TILED_WPG) * NB_TILED_WPG;
         if (padded > 0)
             hipLaunchKernelGGL(k_remap_items, dim3(nblk(padded, 256)), dim3(256), 0, st, s->items.p, s->nitems, padded,
@@ -2741,8 +2739,6 @@ static int batch_enqueue(nbabfs_batch *B, hipEvent_t ev_start = nullptr, hipEven
     }
     launch_pairs14(B->d_desc.p, ns, B->max_n14b, s0->F, st, g);
     launch_finalize(B->d_desc.p, ns, B->max_npad, B->mixed ? 0 : 1, st, g);
-    HIPCHK(hipMemcpyAsync(B->h_energies.p, B->energies.p, NB_NENERGIES * (size_t)ns * sizeof(double),
-                          hipMemcpyDeviceToHost, st));
     return NBABFS_STATUS_CONTINUE;
 }
 
@@ -2755,7 +2751,7 @@ static int batch_relayout_if_needed(nbabfs_batch *B, const double *const *d_xyz,
     for (int k = 0; k < ns && !relayout; k++) {
         SysDesc D;
         fill_desc(B->st[k], D, d_xyz[k], d_grad ? d_grad[k] : nullptr);
-        D.energies = B->energies.p + NB_NENERGIES * (size_t)k;
+        D.energies = B->energies.d + NB_NENERGIES * (size_t)k;
         relayout = B->last_items[k] != B->st[k]->items_version || std::memcmp(&D, &B->shadow[k], sizeof(SysDesc)) != 0;
     }
     if (relayout) CHK(batch_layout(B, d_xyz, d_grad));
@@ -2858,7 +2854,6 @@ extern "C" int nbabfs_batch_energy(nbabfs_batch *B, const double *const *d_xyz, 
     CHK(B->d_check.ensure(ns));
     CHK(B->h_check.ensure(ns));
     CHK(B->flags.ensure(ns + 1));
-    CHK(B->h_energies.ensure(NB_NENERGIES * (size_t)ns));
     if (!B->gguard.p) {
         CHK(B->gguard.ensure(2));
         launch_fill_int(B->gguard.p, 2, 0, st);
@@ -2896,13 +2891,13 @@ extern "C" int nbabfs_batch_energy(nbabfs_batch *B, const double *const *d_xyz, 
     CHK(batch_collect_timing(B));
     int bad = -1;
     for (int k = 0; k < ns; k++) {
-        std::memcpy(energies + 4 * (size_t)k, B->h_energies.p + NB_NENERGIES * (size_t)k, 4 * sizeof(double));
-        if (bad < 0 && B->h_energies.p[NB_NENERGIES * (size_t)k + NB_ESTATUS] != 0.0) bad = k;
+        std::memcpy(energies + 4 * (size_t)k, B->energies.h + NB_NENERGIES * (size_t)k, 4 * sizeof(double));
+        if (bad < 0 && B->energies.h[NB_NENERGIES * (size_t)k + NB_ESTATUS] != 0.0) bad = k;
     }
     if (bad >= 0) {
         char what[64];
         std::snprintf(what, sizeof(what), "batch system %d", bad);
-        return call_status((int)B->h_energies.p[NB_NENERGIES * (size_t)bad + NB_ESTATUS], what);
+        return call_status((int)B->energies.h[NB_NENERGIES * (size_t)bad + NB_ESTATUS], what);
     }
     return NBABFS_STATUS_CONTINUE;
 }
@@ -3385,13 +3380,10 @@ extern "C" int nbabfs_qcmm_terms(nbabfs_state *S, double *energies, int *present
 {
     if (!S || !energies) return fail(NBABFS_STATUS_INVALID_ARGUMENT, "null argument");
     if (!S->has_qc) return fail(NBABFS_STATUS_LOGIC_ERROR, "the state has no QC atoms");
-    CHK(S->h_energies.ensure(NB_NENERGIES));
     CHK(S->energies.ensure(NB_NENERGIES));
-    HIPCHK(hipMemcpyAsync(S->h_energies.p, S->energies.p, NB_NENERGIES * sizeof(double), hipMemcpyDeviceToHost,
-                          S->stream));
     HIPCHK(hipStreamSynchronize(S->stream));
-    energies[0] = S->h_energies.p[6];
-    energies[1] = S->h_energies.p[7];
+    energies[0] = S->energies.h[6];
+    energies[1] = S->energies.h[7];
     if (present) {
         present[0] = S->n_lj > 0;
         present[1] = S->n_lj14 > 0;
