@@ -111,13 +111,16 @@ __device__ __forceinline__ double min_uniform(double x, double s)
     return r;
 }
 
+// F64 (the full-FP64 instance): the seed is v_rsq_f64 (2^-23 or better), and one third-order step leaves rounding alone,
+// 2 ulp of 1/r.
+template <bool F64>
 __device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, double u, double qq, double4 C,
                                           unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
                                           double &elj)
 {
-    const double y = (double)__builtin_amdgcn_rsqf((float)r2);
+    const double y = F64 ? __builtin_amdgcn_rsq(r2) : (double)__builtin_amdgcn_rsqf((float)r2);
     const double h = fma(-(r2 * y), y, 1.0);
-    const double s = fma(0.5 * y, h, y);
+    const double s = F64 ? fma(y * h, fma(0.375, h, 0.5), y) : fma(0.5 * y, h, y);
     const double s2 = s * s;
     const double s3 = s2 * s;
     const double s6 = s3 * s3;
@@ -552,16 +555,18 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // launch, because a second stream's launch starts 15 us after its fork and joins 11 us after its end, and because the
 // image items fill the GPU as the main items drain: 23,559 atoms in a 50 A cell, 139 us per call with two launches,
 // 126 us with one.
-// F64: the full-FP64 instance (the NBABFS_TILED_FP64 comparison path): the same list, tiles, staging and
-// fixed-point sums, with the reference's FP64 pair arithmetic (pair_fp64: divide and square root, no FP32
-// seed, raw A and B per type pair) and FP64 force vectors; three waves per SIMD for its larger accumulators.
+// F64: the full-FP64 instance (NBABFS_TILED_FP64): the same list, tiles, staging, polynomial rows and fixed-point sums
+// with 1/r to rounding and FP64 force vectors, at four waves per SIMD (128 VGPRs) for its larger accumulators.  With the
+// reference's own expressions (seven divides and a square root per tile, both regions for a wave that holds both) a tile
+// took 790 issue cycles and 20,001 atoms 126 us per call; with the rows it takes 227 and 69 us, and the gradients' error
+// against exact sums (7e-12 of their RMS, the fixed-point rounding) stays as it was.
 // WPG: wavefronts per workgroup.  With 4 (the one-item-per-wave launches),
 // the row table is staged once for four items and a group's LDS stays small
 // enough for five waves per SIMD; the four items of a group belong to one
 // system (batches pad each system's items to a multiple of 4 with empty
 // ones).  The persistent queues run one wave per group.
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 3 : (IMG ? 4 : 5)))) void k_force_tiled(
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((F64 || IMG) ? 4 : 5))) void k_force_tiled(
     const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, AbfsFactors F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
@@ -642,8 +647,6 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
         const SysDesc *D = &descs[sys1 >= 0 ? sys1 : (IMG ? (w.sys & 0xffff) : w.sys)];
         const GAS double *__restrict__ xq = (const GAS double *)D->xyzq;
         const GAS int *__restrict__ ty = as_global(D->styp);
-        const GAS double *__restrict__ ljA = as_global(D->ljA);
-        const GAS double *__restrict__ ljB = as_global(D->ljB);
         const GAS double *__restrict__ rows = as_global(D->ljrow);
         const GAS unsigned char *__restrict__ eb = (const GAS unsigned char *)D->entries;
         long long *facc = D->facc;
@@ -688,7 +691,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
         double4 xj = st.xj;
         int tj = 64 * st.tj;
         const int comp = min(a, NB_CL - 1 - a);
-        const double fscale = F64 ? 1.0 : -1.0;            // i-force = fscale times the sum over j
+        const double fscale = -1.0;            // i-force = fscale times the sum over j
         wave_region_sync<WPG>();
         if (IMG && img >= 0) xj = image_slot(xj, sX);
 
@@ -737,34 +740,24 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
                     if (mact != 0ull) {
                         float px = (float)dx, py = (float)dy, pz = (float)dz;
                         if (!F64) asm("" : "+v"(px), "+v"(py), "+v"(pz));   // three registers across the pair terms, not six
-                        if (F64) {
-                            // PairwiseInteraction.h:72-119 in FP64 with the reference's operations.
-                            if (act) {
-                                const int tij = (ti + tj) >> 6;
-                                double x1, x2, dF;
-                                pair_fp64(F, r2, xi.w * xj.w, ljA[tij], ljB[tij], x1, x2, dF);
-                                const double f = 2.0 * dF;
-                                fx[c] = fma(f, dx, fx[c]); fy[c] = fma(f, dy, fy[c]); fz[c] = fma(f, dz, fz[c]);
-                                gx = fma(f, dx, gx); gy = fma(f, dy, gy); gz = fma(f, dz, gz);
-                                eel += x1;
-                                elj += x2;
-                            }
-                        } else {
+                        {
                             const double u = switch_coordinate(F, uShift, r2);
                             const int off = ti + tj + (int)min((unsigned)__double2hiint(u), 32u);
                             const double4 C = ROWS_LDS ? *(const double4 *)((const unsigned char *)sR + off)
                                                        : load_slot(rows, off >> 5);
                             double fs, x1, x2;
-                            pair_rows(F, r2, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
+                            pair_rows<F64>(F, r2, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
                             // The sums take the active lanes only (the others may hold any value).
                             if (act) {
-                                const float f = (float)fs;
-                                fx[c] = fmaf(f, px, (float)fx[c]);
-                                fy[c] = fmaf(f, py, (float)fy[c]);
-                                fz[c] = fmaf(f, pz, (float)fz[c]);
-                                gx = fmaf(f, px, (float)gx);
-                                gy = fmaf(f, py, (float)gy);
-                                gz = fmaf(f, pz, (float)gz);
+                                const acc_t f = (acc_t)fs;
+                                const acc_t vx = F64 ? (acc_t)dx : (acc_t)px, vy = F64 ? (acc_t)dy : (acc_t)py,
+                                            vz = F64 ? (acc_t)dz : (acc_t)pz;
+                                fx[c] = fma(f, vx, fx[c]);
+                                fy[c] = fma(f, vy, fy[c]);
+                                fz[c] = fma(f, vz, fz[c]);
+                                gx = fma(f, vx, gx);
+                                gy = fma(f, vy, gy);
+                                gz = fma(f, vz, gz);
                                 eel += x1;
                                 elj += x2;
                             }
@@ -834,7 +827,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
         bad |= fx_atomic_add3(facc, n_pad, I0 * NB_CL + lane, iscale * (double)ix, iscale * (double)iy,
                               iscale * (double)iz);
         // Energies: lane 0 holds the Coulomb total, lane 32 the Lennard-Jones one.
-        const double etot = wave_sum2_f64(F64 ? eel : eel * F.eScale, F64 ? elj : elj * (1.0 / 3.0));
+        const double etot = wave_sum2_f64(eel * F.eScale, elj * (1.0 / 3.0));
         if ((lane & 31) == 0) {
             const int slot = it & (NB_ESLOTS - 1);
             const int kind = (lane >> 5) + (img >= 0 ? 2 : 0);
@@ -1264,17 +1257,23 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
     // The row table goes to LDS when the group's LDS still lets four groups of four waves (or ten single waves) share a CU
     // (five groups do up to 32 KB: ten types with 16 entries per wave take 27 KB).
     const size_t limit = wpg == 1 ? NB_LDS_ROW_LIMIT : NB_LDS_GROUP_LIMIT;
-    const bool rows_lds = !full_fp64 && tiled_lds_rows(max_ntypes, true) + (size_t)wpg * wave_bytes <= limit;
+    const bool rows_lds = tiled_lds_rows(max_ntypes, true) + (size_t)wpg * wave_bytes <= limit;
     const int rows_bytes = (int)tiled_lds_rows(max_ntypes, rows_lds);
     const size_t bytes = rows_bytes + (size_t)wpg * wave_bytes;
 #define NB_TILED_ARGS grid, bytes, s, ev_start, ev_stop, d_desc, items, q, F, rows_bytes, wave_bytes, g, nblocks, ngroups, \
                       sys1
     if (full_fp64) {
-        // No row table: the FP64 pair terms read the raw A and B of the type pair.
-        if (wpg == 1)
-            launch_tiled_instance<false, false, true, 1>(NB_TILED_ARGS);
-        else
-            launch_tiled_instance<false, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
+        if (wpg == 1) {
+            if (rows_lds)
+                launch_tiled_instance<true, false, true, 1>(NB_TILED_ARGS);
+            else
+                launch_tiled_instance<false, false, true, 1>(NB_TILED_ARGS);
+        } else {
+            if (rows_lds)
+                launch_tiled_instance<true, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
+            else
+                launch_tiled_instance<false, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
+        }
     } else if (images) {
         if (rows_lds)
             launch_tiled_instance<true, true, false, NB_TILED_WPG>(NB_TILED_ARGS);

@@ -906,7 +906,7 @@ static int image_item_cost(const nbabfs_options &o)
 static ItemCut item_cut(const nbabfs_options &o, int per_item)
 {
     const int cu = g_cu_count > 0 ? g_cu_count : 256;
-    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 3 : 5);
+    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 4 : 5);
     return ItemCut{NB_ENTRY_COST * std::max(1, per_item > 0 ? per_item : 16), o.wavesPerCU > 0 ? 0 : held};
 }
 
