@@ -391,7 +391,7 @@ struct nbabfs_state {
     long long calls = 0, updates = 0, npairs = 0;
     // The pair count of the last build reaches h_np without a synchronisation; it is read (and added to the
     // statistics when np_stat) at the next synchronisation that needs it.
-    PinBuf<unsigned long long> h_np;
+    MappedBuf<unsigned long long> h_np;
     bool np_pending = false, np_stat = false;
     std::vector<unsigned char> stencil_h;   // stencil flags last uploaded
     PinBuf<int> h_qs;                       // staging of the queue starts
@@ -447,9 +447,9 @@ struct nbabfs_state {
     // Build temporaries.
     DBuf<int> key, count, off, cursor, sorted, padded, colstart, scantmp, counts, costs, icosts, ncand, eoff, nits, ioff, flag;
     DBuf<int2> colcl;
-    DBuf<double> bbpart, bbox;
+    DBuf<double> bbpart;
     DBuf<unsigned long long> u64;
-    PinBuf<double> h_bbox;
+    MappedBuf<double> h_bbox;
     PinBuf<int> h_int;
 
     // Crystal symmetry: the transformations given at set-up (fractional, 9 + 3
@@ -864,7 +864,7 @@ static int resolve_npairs(nbabfs_state *S)
 {
     if (!S->np_pending) return NBABFS_STATUS_CONTINUE;
     HIPCHK(hipStreamSynchronize(S->stream));
-    S->npairs = (long long)S->h_np.p[0];
+    S->npairs = (long long)S->h_np.h[0];
     S->np_pending = false;
     if (S->np_stat) S->sumPairs += (double)S->npairs;
     S->np_stat = false;
@@ -915,6 +915,7 @@ static int queue_bounds(nbabfs_state *S)
 {
     hipStream_t st = S->stream;
     S->items_version++;
+    if (S->opt.wavesPerCU <= 0) return NBABFS_STATUS_CONTINUE;      // no queues
     // Pinned staging: the copy is asynchronous; the staging is rewritten only after it completed.
     CHK(S->h_qs.ensure(9));
     CHK(S->qstarts.ensure(9));
@@ -970,13 +971,12 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     // Bounding box.
     const int nparts = std::min(nblk(n, 256), 1024);
     CHK(S->bbpart.ensure(6 * (size_t)nparts));
-    CHK(S->bbox.ensure(6));
     CHK(S->h_bbox.ensure(6));
-    launch_bbox(d_xyz, n, S->bbpart.p, nparts, S->bbox.p, st);
-    HIPCHK(hipMemcpyAsync(S->h_bbox.p, S->bbox.p, 6 * sizeof(double), hipMemcpyDeviceToHost, st));
+    launch_bbox(d_xyz, n, S->bbpart.p, nparts, S->h_bbox.d, st);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     double bb[6];
-    std::memcpy(bb, S->h_bbox.p, sizeof(bb));
+    std::memcpy(bb, S->h_bbox.h, sizeof(bb));
     CHK(check_box(bb));
 
     // Grid vs direct is decided once, on the first build (NBModelABFSState.c:212).
@@ -1043,19 +1043,16 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->colstart.ensure(ncol));
     CHK(S->colcl.ensure(ncol));
     CHK(S->scantmp.ensure(scan_tmp_size(std::max(std::max(nkeys, n + 1), ncol)) + 1024));
-    CHK(S->h_int.ensure(16));
     launch_fill_int(S->count.p, nkeys, 0, st);
     launch_bin(d_xyz, n, g, S->cellv.p, S->key.p, S->count.p, st);
-    launch_scan(S->count.p, S->off.p, nkeys, S->scantmp.p, st);
-    HIPCHK(hipMemcpyAsync(S->cursor.p, S->off.p, nkeys * sizeof(int), hipMemcpyDeviceToDevice, st));
+    CHK(S->tail.ensure(16));
+    launch_key_offsets(S->count.p, nkeys, ncol, g.nzb, n, S->off.p, S->cursor.p, S->padded.p, S->colstart.p, S->scantmp.p,
+                       S->tail.d, st);
     CHK(S->unsorted.ensure(n));
-    launch_sort_slots(S->key.p, n, nkeys, ncol, g.nzb, S->off.p, S->cursor.p, S->unsorted.p, S->sorted.p, S->padded.p,
-                      st);
-    launch_scan(S->padded.p, S->colstart.p, ncol, S->scantmp.p, st);
-    HIPCHK(hipMemcpyAsync(S->h_int.p, S->colstart.p + (ncol - 1), sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(S->h_int.p + 1, S->padded.p + (ncol - 1), sizeof(int), hipMemcpyDeviceToHost, st));
+    launch_sort_slots(S->key.p, n, nkeys, S->off.p, S->cursor.p, S->unsorted.p, S->sorted.p, st);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
-    const int total_padded = S->h_int.p[0] + S->h_int.p[1];
+    const int total_padded = ((volatile int *)S->tail.h)[0];
     S->n_pad = (total_padded + NB_SC - 1) / NB_SC * NB_SC;
     S->ncl = S->n_pad / NB_CL;
     S->nsc = S->ncl / NB_SCC;
@@ -1110,7 +1107,7 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->eoff.ensure(S->nsc + 1));
     CHK(S->nits.ensure(S->nsc));
     CHK(S->ioff.ensure(S->nsc + 1));
-    CHK(S->tail.ensure(4));
+    CHK(S->tail.ensure(16));
     for (int attempt = 0; attempt < 4; attempt++) {
         P.cap = S->cap;
         CHK(S->scratch.ensure((size_t)S->nsc * S->cap));
@@ -1147,13 +1144,11 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     S->img_npairs = 0;
     CHK(S->entries.ensure(S->nent));
     CHK(S->items.ensure(S->nitems));
-    CHK(S->u64.ensure(2));
+    CHK(S->h_np.ensure(1));
     CHK(S->npblock.ensure(S->nsc));
-    launch_compact(S->scratch.p, S->cap, nullptr, S->ncand.p, S->eoff.p, S->nsc, S->entries.p, S->u64.p, S->npblock.p, st);
+    launch_compact(S->scratch.p, S->cap, nullptr, S->ncand.p, S->eoff.p, S->nsc, S->entries.p, S->h_np.d, S->npblock.p, st);
     launch_cut_items(S->counts.p, S->costs.p, S->eoff.p, S->ioff.p, S->nits.p, S->nsc, S->nsc, 0, S->entries.p,
                      S->items.p, st);
-    CHK(S->h_np.ensure(1));
-    HIPCHK(hipMemcpyAsync(S->h_np.p, S->u64.p, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     S->np_pending = true;
 
     // Per-call buffers.
@@ -1566,10 +1561,8 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
         // widened by the cutoff.
         const int nparts = std::min(nblk(n, 256), 1024);
         CHK(S->bbpart.ensure(6 * (size_t)nparts));
-        CHK(S->bbox.ensure(6));
         CHK(S->h_bbox.ensure(6));
-        launch_bbox(d_xyz, n, S->bbpart.p, nparts, S->bbox.p, st);
-        HIPCHK(hipMemcpyAsync(S->h_bbox.p, S->bbox.p, 6 * sizeof(double), hipMemcpyDeviceToHost, st));
+        launch_bbox(d_xyz, n, S->bbpart.p, nparts, S->h_bbox.d, st);
         // Transformations searched: with inverses, t is skipped when its inverse comes later.
         std::vector<int> tl;
         std::vector<double> rt;
@@ -1592,14 +1585,14 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
         HIPCHK(hipMemcpyAsync(S->h_ibb.p, S->ibb.p, 6 * (size_t)nt * sizeof(double), hipMemcpyDeviceToHost, st));
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
-        CHK(check_box(S->h_bbox.p));
+        CHK(check_box(S->h_bbox.h));
         for (int k = 0; k < nt; k++) CHK(check_box(S->h_ibb.p + 6 * k));
         double lower[3], upper[3];
         {
 #pragma clang fp contract(off)
             for (int d = 0; d < 3; d++) {
-                lower[d] = S->h_bbox.p[d];
-                upper[d] = (S->h_bbox.p[3 + d] - S->h_bbox.p[d]) + lower[d];
+                lower[d] = S->h_bbox.h[d];
+                upper[d] = (S->h_bbox.h[3 + d] - S->h_bbox.h[d]) + lower[d];
                 lower[d] += -cutoff;
                 upper[d] += cutoff;
             }
@@ -1692,7 +1685,7 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
             if (S->useGrid) {
                 BuildGrid g2;
                 std::memset(&g2, 0, sizeof(g2));
-                reference_grid(S->h_bbox.p, o.cutoffCellSizeFactor * o.listCutoff, g2);
+                reference_grid(S->h_bbox.h, o.cutoffCellSizeFactor * o.listCutoff, g2);
                 P.pointcell = o.useGridByCell ? 0 : 1;
                 CHK(S->icell.ensure(n));
                 launch_image_cells(d_xyz, n, g2, P.pointcell, S->u, S->has_flags ? S->freef.p : nullptr, S->icell.p,
@@ -1721,7 +1714,7 @@ static int build_images(nbabfs_state *S, const double *d_xyz)
             CHK(S->scantmp.ensure(scan_tmp_size(nb + 1) + 1024));
             launch_image_bounds(P, nsc, ns, S->blo.p, S->bhi.p, S->ibound.p, st);
             launch_scan(S->ibound.p, S->isoff.p, nb, S->scantmp.p, st);
-            CHK(S->tail.ensure(8));
+            CHK(S->tail.ensure(16));
             CHK(S->flag.ensure(1));
             launch_fill_int(S->flag.p, 1, 0, st);
             CHK(S->icounts.ensure(nb));

@@ -133,8 +133,10 @@ void launch_bin(const double *xyz, int n, const BuildGrid &g, int4 *cellv, int *
 size_t scan_tmp_size(int m);
 void launch_scan(const int *in, int *out, int m, int *tmp, hipStream_t s);
 void launch_fill_int(int *p, size_t m, int v, hipStream_t s);
-void launch_sort_slots(const int *key, int n, int nkeys, int ncol, int nzb, int *off, int *cursor, int *unsorted,
-                       int *sorted, int *padded, hipStream_t s);
+void launch_key_offsets(const int *count, int nkeys, int ncol, int nzb, int n, int *off, int *cursor, int *padded,
+                        int *colstart, int *scantmp, int *out, hipStream_t s);
+void launch_sort_slots(const int *key, int n, int nkeys, const int *off, int *cursor, int *unsorted, int *sorted,
+                       hipStream_t s);
 void launch_slots(const int *sorted, const int *key, int n, int nzb, const int *off, const int *colstart,
                   const int *padded, int ncol, const double *xyz, int nsc, int *slot_atom, int *atom_slot, int2 *colcl,
                   hipStream_t s);

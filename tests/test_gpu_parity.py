@@ -166,6 +166,22 @@ def test_pairs_at_the_list_cutoff(oracle_mod, shift, factor):
     assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
 
 
+# The counting sort's two offset scans: one workgroup up to 65,536 keys, many above.  A wide thin layer has the most keys
+# for its atoms (columns of one z-bin).
+@pytest.mark.parametrize("natoms,side", [(2000, 900.0), (60000, 9000.0), (140000, 9600.0)])
+def test_sort_key_counts(oracle_mod, natoms, side):
+    from pdynamo_amd import synthetic
+    rng = np.random.default_rng(natoms)
+    mm = synthetic.random_small_system(natoms, 60.0, 3)
+    c = rng.uniform(0.0, 1.0, (natoms // 2, 3)) * [side, side, 0.6]
+    mm.coordinates3 = np.concatenate([c, c + rng.uniform(-1.0, 1.0, c.shape) * [7.0, 7.0, 0.2]])
+    s = _system(mm)
+    _run(s)
+    o = oracle_mod.OracleABFS(mm, nthreads=8)
+    o.energy(mm.coordinates3)
+    assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
+
+
 def _water_with_14(nwater, box, seed):
     """Waters on a jittered lattice (no overlapping atoms: the Coulomb and 1-4 terms are not small beside the
     LJ term) plus intermolecular "1-4" pairs between atoms 2.5-5 A apart, excluded from the main list as a
