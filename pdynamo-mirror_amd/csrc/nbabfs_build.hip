@@ -184,12 +184,12 @@ __global__ __launch_bounds__(256) void k_colpad(const int *__restrict__ off, int
 
 // The counting sort's offsets and the columns' slots in one workgroup: the exclusive scan of the key counts (off, and
 // cursor as its copy for the scatter), each column's atoms rounded up to whole super-clusters (padded), their scan
-// (colstart), and the slots of all columns into *out.  Each thread scans a contiguous chunk.  One launch of 20 us (13,500
-// keys) for eight of 2 to 4 us with gaps of 6 us between them (dynamics of 30,000 atoms 1344 -> 1246 us, frames of
-// 100,002 atoms 1033 -> 986 us); above NB_KEYSCAN_MAX keys (more than 64 per
-// thread) the scan over many workgroups is the faster one.
+// (colstart), and the slots of all columns into *out.  Each thread scans a contiguous chunk.  One launch of 20 us
+// (13,500 keys; 45 us for 27,000) instead of eight that take 25 us and 35 us of gaps between them (dynamics of 30,000
+// atoms 1344 -> 1246 us, frames of 100,002 atoms 1033 -> 986 us): above NB_KEYSCAN_MAX keys the scan over many workgroups
+// is the faster one.
 #define NB_KEYSCAN_THREADS 1024
-#define NB_KEYSCAN_MAX (64 * NB_KEYSCAN_THREADS)
+#define NB_KEYSCAN_MAX (32 * NB_KEYSCAN_THREADS)
 __device__ __forceinline__ int block_exclusive(int v, int *sW, int &total)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;

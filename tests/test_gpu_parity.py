@@ -166,7 +166,7 @@ def test_pairs_at_the_list_cutoff(oracle_mod, shift, factor):
     assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
 
 
-# The counting sort's two offset scans: one workgroup up to 65,536 keys, many above.  A wide thin layer has the most keys
+# The counting sort's two offset scans: one workgroup up to 32,768 keys, many above.  A wide thin layer has the most keys
 # for its atoms (columns of one z-bin).
 @pytest.mark.parametrize("natoms,side", [(2000, 900.0), (60000, 9000.0), (140000, 9600.0)])
 def test_sort_key_counts(oracle_mod, natoms, side):
