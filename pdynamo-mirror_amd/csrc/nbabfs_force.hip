@@ -97,7 +97,7 @@ __device__ __forceinline__ bool pair_fp64(const AbfsFactors &F, double r2, doubl
 // A, B.  The rows hold three times the coefficients, so that the factor 3 of the
 // Lennard-Jones force costs nothing: elj is 3 E, divided by 3 with the item's
 // total, and fs is minus twice dE/d(r^2).
-__device__ __forceinline__ double switch_coordinate(const AbfsFactors &F, double uShift, double r2)
+__device__ __forceinline__ double switch_coordinate(const TiledFactors &F, double uShift, double r2)
 {
     return fmin(fmax(fma(r2, F.uScale, uShift), 0.0), 1.0);
 }
@@ -114,7 +114,7 @@ __device__ __forceinline__ double min_uniform(double x, double s)
 // F64 (the full-FP64 instance): the seed is v_rsq_f64 (2^-23 or better), and one third-order step leaves rounding alone,
 // 2 ulp of 1/r.
 template <bool F64>
-__device__ __forceinline__ void pair_rows(const AbfsFactors &F, double r2, double u, double qq, double4 C,
+__device__ __forceinline__ void pair_rows(const TiledFactors &F, double r2, double u, double qq, double4 C,
                                           unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
                                           double &elj)
 {
@@ -567,7 +567,7 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // ones).  The persistent queues run one wave per group.
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
 __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((F64 || IMG) ? 4 : 5))) void k_force_tiled(
-    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, AbfsFactors F, int rows_bytes,
+    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, TiledFactors F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
     const int lane = threadIdx.x & 63;
@@ -1235,7 +1235,7 @@ void launch_prepare(const SysDesc *d_desc, int nsys, int max_npad, int tiled, in
 
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
 static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop,
-                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q, const AbfsFactors &F,
+                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q, const TiledFactors &F,
                                   int rows_bytes, int wave_bytes, ForceGuard g, int nitems, int nforce_groups,
                                   int sys1)
 {
@@ -1243,7 +1243,7 @@ static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEve
                           d_desc, items, q, F, rows_bytes, wave_bytes, g, nitems, nforce_groups, sys1);
 }
 
-void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const AbfsFactors &F,
+void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const TiledFactors &F,
                         int nblocks, int max_ntypes, ForceGuard g, hipStream_t s, bool images,
                         hipEvent_t ev_start, hipEvent_t ev_stop, int n14_blocks, bool full_fp64, int sys1)
 {

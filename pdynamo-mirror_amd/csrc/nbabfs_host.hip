@@ -168,7 +168,7 @@ static double coulomb_factor()
 }
 
 // PairwiseInteractionABFS_MakeFactors (pMolecule-1.9.0/extensions/csource/PairwiseInteraction.c:89-141).
-static void make_factors(double damp, double inner, double outer, AbfsFactors &F)
+static void make_factors(double damp, double inner, double outer, TiledFactors &F)
 {
 #pragma clang fp contract(off)
     const double r2d = damp * damp, r2off = outer * outer, r2on = inner * inner;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void k_max_displacement(const double *__restri
 struct nbabfs_state {
     nbabfs_options opt;
     int n = 0, ntypes = 0, n14 = 0;
-    AbfsFactors F;
+    TiledFactors F;
     double escale = 0, escale14 = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -1360,7 +1360,7 @@ static void fill_desc(nbabfs_state *S, SysDesc &D, const double *d_xyz, double *
     D.escale = S->escale;
     D.escale14 = S->escale14;
     D.qscale = std::sqrt(S->escale);
-    const AbfsFactors &F = S->F;
+    const TiledFactors &F = S->F;
     const double damp[7] = {F.qF0 / F.eScale, -F.qAlpha / F.eScale, F.aF0, F.aAlpha, F.bF0, F.bAlpha, F.qAlpha};
     std::memcpy(D.damp, damp, sizeof(damp));
     D.n = S->n;

@@ -42,7 +42,14 @@ struct AbfsFactors {
     double a, b, c, d, qShift1, qShift2, qF0, qAlpha;
     double aF6, aK12, aShift12, aF0, aAlpha;
     double bF3, bK6, bShift6, bF0, bAlpha;
-    // Tiled mixed kernel: u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff, and the
+};
+static_assert(sizeof(AbfsFactors) == 21 * sizeof(double), "the plain kernels' factors: the tiled ones stand in TiledFactors");
+
+// The tiled kernel's factors.  A struct of their own: with them in AbfsFactors every kernel of the plain path took 80
+// more bytes of arguments, and the longer start of k_force_plain moved its pair loop to code addresses at which a call
+// took 1 to 2.7% longer (600 atoms: 516 us per call with the short arguments, 530 with the long; 15,000: 1152 and 1176).
+struct TiledFactors : AbfsFactors {
+    // u = r2 uScale + uShift (0 at the inner, 1 at the outer cutoff), sOn = 1 / inner cutoff, and the
     // Coulomb energy divided by eScale, the leading coefficient of P - 1 = eScale (p0 + u (p1 + u (p2 + u))).
     double uScale, uShift, sOn, p0, p1, p2, eScale, eInv, qShift2e;
     double minus3;              // -3 (an operand in scalar registers, not a pair of vector registers)

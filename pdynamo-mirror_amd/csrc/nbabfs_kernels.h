@@ -228,7 +228,7 @@ void launch_prepare(const SysDesc *d_desc, int nsys, int max_npad, int tiled, in
 // full_fp64: the NBABFS_TILED_FP64 instance (FP64 pair arithmetic and force vectors; not for image items).
 // sys1 >= 0: every item belongs to system sys1 (a single-state launch), so the kernel reads its descriptor without
 // waiting for the items.
-void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const AbfsFactors &F,
+void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const TiledFactors &F,
                         int nblocks, int max_ntypes, ForceGuard g, hipStream_t s, bool images = false,
                         hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr, int n14_blocks = 0,
                         bool full_fp64 = false, int sys1 = -1);
