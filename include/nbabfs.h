@@ -44,9 +44,10 @@ extern "C" {
 #define NBABFS_PLAIN_FP64 1   /* one thread per atom over a full CSR list, FP64 in
                                  the reference expression order (divide, sqrt)      */
 #define NBABFS_TILED_FP64 2   /* the tiled kernel's list, tiles and fixed-point sums
-                                 with FP64 pair arithmetic (1/r to rounding) and
-                                 FP64 force vectors: the mixed path without its
-                                 FP32 parts
+                                 with FP64 pair arithmetic and FP64 force vectors:
+                                 the mixed path without its FP32 parts.  No divide
+                                 or square root, but each pair term as close to its
+                                 exact value as in the reference's expressions
                                  (no image lists)                                    */
 
 /* Upper bound of nbabfs_options.entriesPerItem. */

@@ -97,7 +97,8 @@ __device__ __forceinline__ bool pair_fp64(const AbfsFactors &F, double r2, doubl
 // A, B.  The rows hold three times the coefficients, so that the factor 3 of the
 // Lennard-Jones force costs nothing: elj is 3 E, divided by 3 with the item's
 // total, and fs is minus twice dE/d(r^2).
-__device__ __forceinline__ double switch_coordinate(const TiledFactors &F, double uShift, double r2)
+template <class Factors>
+__device__ __forceinline__ double switch_coordinate(const Factors &F, double uShift, double r2)
 {
     return fmin(fmax(fma(r2, F.uScale, uShift), 0.0), 1.0);
 }
@@ -111,16 +112,29 @@ __device__ __forceinline__ double min_uniform(double x, double s)
     return r;
 }
 
-// F64 (the full-FP64 instance): the seed is v_rsq_f64 (2^-23 or better), and one third-order step leaves rounding alone,
-// 2 ulp of 1/r.
-template <bool F64>
+// The damped region's terms (pair_rows and pair_full), a branch of the whole wave (its lanes select), so the usual path
+// has no execution-mask bookkeeping.  Its factors and tables are read through the descriptor here: as kernel arguments
+// they would hold (and spill) scalar registers over the whole entry loop.  ljScale: the rows' factor.
+__device__ __forceinline__ void pair_damped(double r2Damp, double r2, double qq, unsigned long long mact, const SysDesc *D,
+                                            int off, double ljScale, double &f, double &e1, double &e2)
+{
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(r2 < r2Damp) & mact) != 0ull, 0)) {
+        const GAS double *k = as_global(D->damp);
+        const bool damped = r2 < r2Damp;
+        const double A = as_global(D->ljA)[off >> 6], B = as_global(D->ljB)[off >> 6];
+        e1 = damped ? qq * fma(k[1], r2, k[0]) : e1;
+        e2 = damped ? ljScale * (A * fma(-k[3], r2, k[2]) - B * fma(-k[5], r2, k[4])) : e2;
+        f = damped ? 2.0 * (qq * k[6] + (A * k[3] - B * k[5])) : f;
+    }
+}
+
 __device__ __forceinline__ void pair_rows(const TiledFactors &F, double r2, double u, double qq, double4 C,
                                           unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
                                           double &elj)
 {
-    const double y = F64 ? __builtin_amdgcn_rsq(r2) : (double)__builtin_amdgcn_rsqf((float)r2);
+    const double y = (double)__builtin_amdgcn_rsqf((float)r2);
     const double h = fma(-(r2 * y), y, 1.0);
-    const double s = F64 ? fma(y * h, fma(0.375, h, 0.5), y) : fma(0.5 * y, h, y);
+    const double s = fma(0.5 * y, h, y);
     const double s2 = s * s;
     const double s3 = s2 * s;
     const double s6 = s3 * s3;
@@ -134,17 +148,51 @@ __device__ __forceinline__ void pair_rows(const TiledFactors &F, double r2, doub
     const double inner = fma(s3 + s3, fma(C.x, s6, t1), C.z);
     // Minus twice dE/d(r^2): Coulomb qq s^3 Q, Lennard-Jones 3 s^5 inner (the rows' factor 3).
     double f = s3 * fma(s2, inner, qq * Q);
-    // A branch of the whole wave (its lanes select), so the usual path has no execution-mask bookkeeping.  Its factors and
-    // tables are read through the descriptor here: as kernel arguments they would hold (and spill) scalar registers over
-    // the whole entry loop.
-    if (__builtin_expect((__builtin_amdgcn_ballot_w64(r2 < F.r2Damp) & mact) != 0ull, 0)) {
-        const GAS double *k = as_global(D->damp);
-        const bool damped = r2 < F.r2Damp;
-        const double A = as_global(D->ljA)[off >> 6], B = as_global(D->ljB)[off >> 6];
-        e1 = damped ? qq * fma(k[1], r2, k[0]) : e1;
-        e2 = damped ? 3.0 * (A * fma(-k[3], r2, k[2]) - B * fma(-k[5], r2, k[4])) : e2;
-        f = damped ? 2.0 * (qq * k[6] + (A * k[3] - B * k[5])) : f;
-    }
+    pair_damped(F.r2Damp, r2, qq, mact, D, off, 3.0, f, e1, e2);
+    fs = f;
+    eel = e1;
+    elj = e2;
+}
+
+// The full-FP64 instance's pair terms: no divide or square root, and every term as close to its exact value as the
+// reference's expressions (pair_fp64) come.  Measured on pairs at 200 distances each, default cutoffs, in units of 2^-53 of
+// the term's undamped magnitude and as root mean squares (here / pair_fp64 / the mixed kernel's rows with 1/r to 2 ulp):
+// at 2-2.8 A Coulomb energy 0.6 / 1.6 / 2.4 and force 0.9 / 0.8 / 1.4, Lennard-Jones energy 1.8 / 2.1 / 3.7 and force
+// 2.3 / 2.4 / 4.8; at 8-10 A 3.1 / 7.3 / 7.8, 0.9 / 4.0 / 1.4, 1.0 / 1.1 / 2.9 and 1.5 / 1.6 / 4.4.
+//   * s = 1/r: one third-order step from v_rsq_f64 (2^-23 or better) with the residual of r2 y y to full precision, so
+//     only the last rounding is left.  t + td is 1/r^2 beyond FP64: s2 and s3 each take one rounding of it.
+//   * Coulomb force: the smoothstep as (1 - u)^2 (1 + 2u), which keeps its relative error towards the outer cutoff.
+//   * Coulomb energy: s + qShift1 + P0 min(s - 1/inner, 0) + s u (P1 + u (P2 + u P3)), P - 1 about the inner cutoff
+//     less its value there, so that nothing large cancels; the plain region's added terms are exactly zero.
+//   * Lennard-Jones as the reference squares it: C12 (s^6 - w^2)^2 - C6 (s^3 - w)^2 + C0 (rows 2 C12, 2 C6, 2 C0, w: plain
+//     A, B, C0, 0; switched A aK12, B bK6, 0, bF3 = 1/outer^3; elj is 2 E).  Expanded squares cancel towards the outer cutoff.  In the
+//     plain region both terms take the rounded s^6 (n: that s^6 less s^3 s^3), whose error then cancels at the minimum.
+__device__ __forceinline__ void pair_full(const FullFactors &F, double r2, bool sw, double u, double qq, double4 C,
+                                          unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
+                                          double &elj)
+{
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double p = r2 * y;
+    const double h = fma(-fma(r2, y, -p), y, fma(-p, y, 1.0));
+    const double s = fma(y * h, fma(0.375, h, 0.5), y);
+    const double t = s * s;
+    const double td = t * fma(-r2, t, 1.0);
+    const double s2 = t + td;
+    const double s3 = fma(s, t, s * td);
+    const double s6 = s3 * s3;
+    const double v = 1.0 - u;
+    const double Q = (v * v) * fma(2.0, u, 1.0);
+    const double R = fma(fma(F.P3, u, F.P2), u, F.P1);
+    const double K = fma(F.P0, fmin((s - F.sOn) - F.sOnLow, 0.0), F.q1);
+    double e1 = qq * (s + fma(s * u, R, K));
+    const double l1 = fma(-C.w, C.w, s6), l2 = s3 - C.w;
+    const double n = sw ? 0.0 : fma(-s3, s3, s6);
+    const double a = C.x * l1;
+    double e2 = fma(a, l1, fma(-C.y, fma(l2, l2, n), C.z));
+    const double inner = fma(a + a, s6, -(C.y * fma(l2, s3, n)));
+    const double x = s2 * inner;
+    double f = fma(2.0, x, fma(s3, qq * Q, x));
+    pair_damped(F.r2Damp, r2, qq, mact, D, off, 2.0, f, e1, e2);
     fs = f;
     eel = e1;
     elj = e2;
@@ -555,19 +603,24 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // launch, because a second stream's launch starts 15 us after its fork and joins 11 us after its end, and because the
 // image items fill the GPU as the main items drain: 23,559 atoms in a 50 A cell, 139 us per call with two launches,
 // 126 us with one.
-// F64: the full-FP64 instance (NBABFS_TILED_FP64): the same list, tiles, staging, polynomial rows and fixed-point sums
-// with 1/r to rounding and FP64 force vectors, at four waves per SIMD (128 VGPRs) for its larger accumulators.  With the
-// reference's own expressions (seven divides and a square root per tile, both regions for a wave that holds both) a tile
-// took 790 issue cycles and 20,001 atoms 126 us per call; with the rows it takes 227 and 69 us, and the gradients' error
-// against exact sums (7e-12 of their RMS, the fixed-point rounding) stays as it was.
+// F64: the full-FP64 instance (NBABFS_TILED_FP64): the same list, tiles, staging and fixed-point sums with pair_full and
+// FP64 force vectors, at three waves per SIMD (134 VGPRs; at four the loop keeps two energy sums in scratch, 20,001 atoms
+// 84 us per call instead of 77 with lists cut for three waves).  With the reference's own expressions (seven divides and a
+// square root per tile, both regions for a wave that holds both) a tile took 790 issue cycles and the call 135 us; with
+// the mixed kernel's rows and 1/r to 2 ulp 71 us, but pair terms off by 1.6 to 4 times as much (pair_full).
 // WPG: wavefronts per workgroup.  With 4 (the one-item-per-wave launches),
 // the row table is staged once for four items and a group's LDS stays small
 // enough for five waves per SIMD; the four items of a group belong to one
 // system (batches pad each system's items to a multiple of 4 with empty
 // ones).  The persistent queues run one wave per group.
+template <bool F64>
+struct PairFactors {
+    using type = typename std::conditional<F64, FullFactors, TiledFactors>::type;
+};
+
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((F64 || IMG) ? 4 : 5))) void k_force_tiled(
-    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, TiledFactors F, int rows_bytes,
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 3 : (IMG ? 4 : 5)))) void k_force_tiled(
+    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, typename PairFactors<F64>::type F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
     const int lane = threadIdx.x & 63;
@@ -742,11 +795,15 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((F64 |
                         if (!F64) asm("" : "+v"(px), "+v"(py), "+v"(pz));   // three registers across the pair terms, not six
                         {
                             const double u = switch_coordinate(F, uShift, r2);
-                            const int off = ti + tj + (int)min((unsigned)__double2hiint(u), 32u);
+                            const bool sw = F64 && u > 0.0;
+                            const int off = ti + tj + (F64 ? (sw ? 32 : 0) : (int)min((unsigned)__double2hiint(u), 32u));
                             const double4 C = ROWS_LDS ? *(const double4 *)((const unsigned char *)sR + off)
                                                        : load_slot(rows, off >> 5);
                             double fs, x1, x2;
-                            pair_rows<F64>(F, r2, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
+                            if constexpr (F64)
+                                pair_full(F, r2, sw, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
+                            else
+                                pair_rows(F, r2, u, xi.w * xj.w, C, mact, D, off, fs, x1, x2);
                             // The sums take the active lanes only (the others may hold any value).
                             if (act) {
                                 const acc_t f = (acc_t)fs;
@@ -827,7 +884,13 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu((F64 |
         bad |= fx_atomic_add3(facc, n_pad, I0 * NB_CL + lane, iscale * (double)ix, iscale * (double)iy,
                               iscale * (double)iz);
         // Energies: lane 0 holds the Coulomb total, lane 32 the Lennard-Jones one.
-        const double etot = wave_sum2_f64(eel * F.eScale, elj * (1.0 / 3.0));
+        if constexpr (F64) {
+            elj *= 0.5;
+        } else {
+            eel *= F.eScale;
+            elj *= 1.0 / 3.0;
+        }
+        const double etot = wave_sum2_f64(eel, elj);
         if ((lane & 31) == 0) {
             const int slot = it & (NB_ESLOTS - 1);
             const int kind = (lane >> 5) + (img >= 0 ? 2 : 0);
@@ -1235,7 +1298,7 @@ void launch_prepare(const SysDesc *d_desc, int nsys, int max_npad, int tiled, in
 
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
 static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop,
-                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q, const TiledFactors &F,
+                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q, const typename PairFactors<F64>::type &F,
                                   int rows_bytes, int wave_bytes, ForceGuard g, int nitems, int nforce_groups,
                                   int sys1)
 {
@@ -1245,14 +1308,14 @@ static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEve
 
 void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParams q, const TiledFactors &F,
                         int nblocks, int max_ntypes, ForceGuard g, hipStream_t s, bool images,
-                        hipEvent_t ev_start, hipEvent_t ev_stop, int n14_blocks, bool full_fp64, int sys1)
+                        hipEvent_t ev_start, hipEvent_t ev_stop, int n14_blocks, const FullFactors *full, int sys1)
 {
     if (nblocks + n14_blocks <= 0) return;
     // One item per wave, four waves per group, unless the items come from the persistent queues or the images.
     const int wpg = q.heads != nullptr ? 1 : NB_TILED_WPG;
     const int ngroups = nblk(nblocks, wpg);
     const dim3 grid(ngroups + nblk(n14_blocks, wpg));
-    const int acc = full_fp64 ? 8 : 4;
+    const int acc = full ? 8 : 4;
     const int wave_bytes = (int)tiled_lds_wave(acc);
     // The row table goes to LDS when the group's LDS still lets four groups of four waves (or ten single waves) share a CU
     // (five groups do up to 32 KB: ten types with 16 entries per wave take 27 KB).
@@ -1260,35 +1323,35 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
     const bool rows_lds = tiled_lds_rows(max_ntypes, true) + (size_t)wpg * wave_bytes <= limit;
     const int rows_bytes = (int)tiled_lds_rows(max_ntypes, rows_lds);
     const size_t bytes = rows_bytes + (size_t)wpg * wave_bytes;
-#define NB_TILED_ARGS grid, bytes, s, ev_start, ev_stop, d_desc, items, q, F, rows_bytes, wave_bytes, g, nblocks, ngroups, \
+#define NB_TILED_ARGS(F) grid, bytes, s, ev_start, ev_stop, d_desc, items, q, F, rows_bytes, wave_bytes, g, nblocks, ngroups, \
                       sys1
-    if (full_fp64) {
+    if (full) {
         if (wpg == 1) {
             if (rows_lds)
-                launch_tiled_instance<true, false, true, 1>(NB_TILED_ARGS);
+                launch_tiled_instance<true, false, true, 1>(NB_TILED_ARGS(*full));
             else
-                launch_tiled_instance<false, false, true, 1>(NB_TILED_ARGS);
+                launch_tiled_instance<false, false, true, 1>(NB_TILED_ARGS(*full));
         } else {
             if (rows_lds)
-                launch_tiled_instance<true, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
+                launch_tiled_instance<true, false, true, NB_TILED_WPG>(NB_TILED_ARGS(*full));
             else
-                launch_tiled_instance<false, false, true, NB_TILED_WPG>(NB_TILED_ARGS);
+                launch_tiled_instance<false, false, true, NB_TILED_WPG>(NB_TILED_ARGS(*full));
         }
     } else if (images) {
         if (rows_lds)
-            launch_tiled_instance<true, true, false, NB_TILED_WPG>(NB_TILED_ARGS);
+            launch_tiled_instance<true, true, false, NB_TILED_WPG>(NB_TILED_ARGS(F));
         else
-            launch_tiled_instance<false, true, false, NB_TILED_WPG>(NB_TILED_ARGS);
+            launch_tiled_instance<false, true, false, NB_TILED_WPG>(NB_TILED_ARGS(F));
     } else if (wpg == 1) {
         if (rows_lds)
-            launch_tiled_instance<true, false, false, 1>(NB_TILED_ARGS);
+            launch_tiled_instance<true, false, false, 1>(NB_TILED_ARGS(F));
         else
-            launch_tiled_instance<false, false, false, 1>(NB_TILED_ARGS);
+            launch_tiled_instance<false, false, false, 1>(NB_TILED_ARGS(F));
     } else {
         if (rows_lds)
-            launch_tiled_instance<true, false, false, NB_TILED_WPG>(NB_TILED_ARGS);
+            launch_tiled_instance<true, false, false, NB_TILED_WPG>(NB_TILED_ARGS(F));
         else
-            launch_tiled_instance<false, false, false, NB_TILED_WPG>(NB_TILED_ARGS);
+            launch_tiled_instance<false, false, false, NB_TILED_WPG>(NB_TILED_ARGS(F));
     }
 #undef NB_TILED_ARGS
 }

@@ -218,6 +218,25 @@ static void make_factors(double damp, double inner, double outer, TiledFactors &
     F.minus3 = -3.0;
 }
 
+// The full-FP64 instance's factors, from the reference's definitions in extended precision.
+static void make_full_factors(double inner, double outer, const TiledFactors &T, FullFactors &F)
+{
+    static_cast<AbfsFactors &>(F) = T;
+    F.uScale = T.uScale;
+    F.uShift = T.uShift;
+    F.sOn = T.sOn;
+    F.sOnLow = (double)(1.0L / inner - F.sOn);
+    const long double on = (long double)inner * inner, off = (long double)outer * outer, w = off - on;
+    const long double gamma = w * w * w;
+    const long double a = off * off * (off - 3.0L * on) / gamma, b = 6.0L * off * on / gamma, c = -(off + on) / gamma,
+                      d = 0.4L / gamma;
+    F.q1 = (double)(8.0L * (off * on * ((long double)outer - inner) - 0.2L * (outer * off * off - inner * on * on)) / gamma);
+    F.P0 = (double)((a - 1.0L) - on * (b + on * (c + d * on)));
+    F.P1 = (double)(-w * (b + on * (2.0L * c + 3.0L * d * on)));
+    F.P2 = (double)(-w * w * (c + 3.0L * d * on));
+    F.P3 = (double)(-w * w * w * d);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Device bookkeeping.
 // ------------------------------------------------------------------------------------------------
@@ -364,6 +383,7 @@ struct nbabfs_state {
     nbabfs_options opt;
     int n = 0, ntypes = 0, n14 = 0;
     TiledFactors F;
+    FullFactors F64;        // precision NBABFS_TILED_FP64
     double escale = 0, escale14 = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -906,7 +926,7 @@ static int image_item_cost(const nbabfs_options &o)
 static ItemCut item_cut(const nbabfs_options &o, int per_item)
 {
     const int cu = g_cu_count > 0 ? g_cu_count : 256;
-    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 4 : 5);
+    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 3 : 5);
     return ItemCut{NB_ENTRY_COST * std::max(1, per_item > 0 ? per_item : 16), o.wavesPerCU > 0 ? 0 : held};
 }
 
@@ -1361,7 +1381,8 @@ static void fill_desc(nbabfs_state *S, SysDesc &D, const double *d_xyz, double *
     D.escale14 = S->escale14;
     D.qscale = std::sqrt(S->escale);
     const TiledFactors &F = S->F;
-    const double damp[7] = {F.qF0 / F.eScale, -F.qAlpha / F.eScale, F.aF0, F.aAlpha, F.bF0, F.bAlpha, F.qAlpha};
+    const double es = S->opt.precision == NBABFS_TILED_FP64 ? 1.0 : F.eScale;
+    const double damp[7] = {F.qF0 / es, -F.qAlpha / es, F.aF0, F.aAlpha, F.bF0, F.bAlpha, F.qAlpha};
     std::memcpy(D.damp, damp, sizeof(damp));
     D.n = S->n;
     D.n_pad = S->n_pad;
@@ -1406,13 +1427,13 @@ static int launch_force(nbabfs_state *S, ForceGuard g)
         // The image lists' items follow the main list's, and the mixed kernel takes both in one launch.  The full-FP64
         // and the persistent kernels take main items only: the images' launch then runs beside theirs, on the second
         // stream.
-        const bool fp64 = S->opt.precision == NBABFS_TILED_FP64;
+        const FullFactors *fp64 = S->opt.precision == NBABFS_TILED_FP64 ? &S->F64 : nullptr;
         const int n14 = nblk(S->n14, NB_P14_BLOCK);
         const QueueParams direct{nullptr, S->qstarts.p};
         if (!fp64 && S->opt.wavesPerCU <= 0) {
             if (S->timing && nm + ni > 0) CHK(timing_events(S, 2, ev));
             launch_force_tiled(S->d_desc.p, S->items.p, direct, S->F, nm + ni, S->ntypes, g, st, ni > 0, ev[0], ev[1],
-                               n14, false, 0);
+                               n14, nullptr, 0);
         } else {
             const bool fork = ni > 0 && nm > 0;
             if (fork) {
@@ -1429,7 +1450,7 @@ static int launch_force(nbabfs_state *S, ForceGuard g)
             if (ni > 0) {
                 const int o = nm > 0 ? 2 : 0;
                 launch_force_tiled(S->d_desc.p, S->items.p + nm, direct, S->F, ni, S->ntypes, g, sti, true, ev[o],
-                                   ev[o + 1], 0, false, 0);
+                                   ev[o + 1], 0, nullptr, 0);
             }
             if (nm > 0) {
                 const QueueParams q{S->opt.wavesPerCU > 0 ? S->heads.p : nullptr, S->qstarts.p};
@@ -2001,6 +2022,7 @@ extern "C" int nbabfs_state_create(const nbabfs_options *opt, int natoms, const 
     S->n = natoms;
     S->ntypes = ntypes;
     make_factors(o.dampingCutoff, o.innerCutoff, o.outerCutoff, S->F);
+    make_full_factors(o.innerCutoff, o.outerCutoff, S->F, S->F64);
     S->escale = coulomb_factor() / o.dielectric;
     S->escale14 = S->escale * o.electrostaticScale14;
     if (hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -2028,15 +2050,22 @@ extern "C" int nbabfs_state_create(const nbabfs_options *opt, int natoms, const 
             A14[(size_t)i * ntypes + j] = tableA14 ? tableA14[t] : tableA[t];
             B14[(size_t)i * ntypes + j] = tableB14 ? tableB14[t] : tableB[t];
         }
-    // Polynomial rows of the tiled path: E = C12 s^12 + C6 s^6 + C3 s^3 + C0
-    // for the plain region (r <= innerCutoff) and the force-switched region
-    // (PairwiseInteraction.h:72-119 with the squares expanded).
+    // Rows of the tiled path for the plain region (r <= innerCutoff) and the
+    // force-switched region (PairwiseInteraction.h:72-119).  Mixed: the
+    // polynomial C12 s^12 + C6 s^6 + C3 s^3 + C0, the squares expanded.  Full
+    // FP64: the factors of the squares and the constant (pair_full).
     std::vector<double> R(8 * nt2);
     {
         const AbfsFactors &F = S->F;
         for (size_t k = 0; k < nt2; k++) {
             const double a = A[k], b = B[k], ak = a * F.aK12, bk = b * F.bK6;
             double *p = &R[8 * k];
+            if (o.precision == NBABFS_TILED_FP64) {
+                const double full[8] = {2.0 * a, 2.0 * b, 2.0 * (b * F.bShift6 - a * F.aShift12), 0.0,
+                                        2.0 * ak, 2.0 * bk, 0.0, F.bF3};
+                std::memcpy(p, full, sizeof(full));
+                continue;
+            }
             p[0] = a;
             p[1] = -b;
             p[2] = 0.0;
@@ -2725,7 +2754,7 @@ static int batch_enqueue(nbabfs_batch *B, hipEvent_t ev_start = nullptr, hipEven
             QueueParams q{s0->opt.wavesPerCU > 0 ? B->heads.p : nullptr, B->qstarts.p};
             int maxnt = 0;
             for (auto *s : B->st) maxnt = std::max(maxnt, s->ntypes);
-            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt, g, st, false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64);
+            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt, g, st, false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64 ? &s0->F64 : nullptr);
         }
     } else {
         launch_force_plain(B->d_desc.p, ns, B->max_n, s0->F, g, st, ev_start, ev_stop);

@@ -55,6 +55,14 @@ struct TiledFactors : AbfsFactors {
     double minus3;              // -3 (an operand in scalar registers, not a pair of vector registers)
 };
 
+// The full-FP64 instance's factors (NBABFS_TILED_FP64), in place of the mixed kernel's scaled ones.
+struct FullFactors : AbfsFactors {
+    double uScale, uShift;      // as above
+    double sOn, sOnLow;         // 1 / inner cutoff and what its rounding left
+    double P0, P1, P2, P3;      // P - 1 = P0 + u (P1 + u (P2 + u P3))
+    double q1;                  // qShift1
+};
+
 struct Entry {              // 80 bytes
     int J;                  // j-cluster (local index)
     int cbits;              // bit c set if i-cluster c has any pair with J
