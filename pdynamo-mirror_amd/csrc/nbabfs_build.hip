@@ -1170,20 +1170,37 @@ __global__ __launch_bounds__(256) void k_items_per_sc(const int *__restrict__ co
 
 // Items of the image lists' blocks and where each block's items go, in one workgroup; *out: their number.  A block cuts
 // into n items of cost C / n, and the blocks are laid out by falling item cost (NB_IORDER_BINS steps; the order within a
-// step is free: the items' sums are exact integers).  Blocks at an image's edge hold few entries, so the items differ
-// much more than the main list's, and a long one at the end of a launch is waited for: 23,559 atoms in a 50 A cell took
-// 150 us per call in block order and 139 us in this one.
+// step is free: the tiled kernel's sums are exact integers).  Blocks at an image's edge hold few entries, so the items
+// differ much more than the main list's, and a long one at the end of a launch is waited for: 23,559 atoms in a 50 A cell
+// took 150 us per call in block order and 139 us in this one.  in_order: the blocks' own order, for the plain path, which
+// adds FP64 energies item by item: there the order is part of the result.
 #define NB_IORDER_BINS 256
-__global__ __launch_bounds__(1024) void k_image_items(const int *__restrict__ costs, int m, int per_item,
-                                                      int *__restrict__ nits, int *__restrict__ ioff,
-                                                      int *__restrict__ out)
+__global__ __launch_bounds__(NB_KEYSCAN_THREADS) void k_image_items(const int *__restrict__ costs, int m, int per_item,
+                                                                    int in_order, int *__restrict__ nits,
+                                                                    int *__restrict__ ioff, int *__restrict__ out)
 {
     __shared__ int sH[NB_IORDER_BINS];
     const int t = threadIdx.x;
+    if (in_order) {
+        __shared__ int sW[NB_KEYSCAN_THREADS / 64];
+        const int chunk = (m + NB_KEYSCAN_THREADS - 1) / NB_KEYSCAN_THREADS;
+        const int lo = min(t * chunk, m), hi = min(lo + chunk, m);
+        int v = 0, total;
+        for (int k = lo; k < hi; k++) v += (costs[k] + per_item - 1) / per_item;
+        int o = block_exclusive(v, sW, total);
+        for (int k = lo; k < hi; k++) {
+            const int n = (costs[k] + per_item - 1) / per_item;
+            nits[k] = n;
+            ioff[k] = o;
+            o += n;
+        }
+        if (t == 0) *(volatile int *)out = total;
+        return;
+    }
     auto bin = [&](int c, int n) { return NB_IORDER_BINS - 1 - (int)((long long)(c / n) * (NB_IORDER_BINS - 1) / per_item); };
     if (t < NB_IORDER_BINS) sH[t] = 0;
     __syncthreads();
-    for (int k = t; k < m; k += 1024) {
+    for (int k = t; k < m; k += NB_KEYSCAN_THREADS) {
         const int c = costs[k], n = (c + per_item - 1) / per_item;
         nits[k] = n;
         if (n > 0) atomicAdd(&sH[bin(c, n)], n);
@@ -1198,7 +1215,7 @@ __global__ __launch_bounds__(1024) void k_image_items(const int *__restrict__ co
     if (t < NB_IORDER_BINS) sH[t] = before;
     if (t == NB_IORDER_BINS - 1) *(volatile int *)out = before + own;
     __syncthreads();
-    for (int k = t; k < m; k += 1024) {
+    for (int k = t; k < m; k += NB_KEYSCAN_THREADS) {
         const int c = costs[k], n = (c + per_item - 1) / per_item;
         ioff[k] = n > 0 ? atomicAdd(&sH[bin(c, n)], n) : 0;
     }
@@ -1690,9 +1707,10 @@ bool launch_list_offsets(const int *counts, const int *costs, int nsc, const Ite
     return true;
 }
 
-void launch_image_items(const int *costs, int m, int per_item, int *nits, int *ioff, int *out, hipStream_t s)
+void launch_image_items(const int *costs, int m, int per_item, bool in_order, int *nits, int *ioff, int *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_image_items, dim3(1), dim3(1024), 0, s, costs, m, per_item, nits, ioff, out);
+    hipLaunchKernelGGL(k_image_items, dim3(1), dim3(NB_KEYSCAN_THREADS), 0, s, costs, m, per_item, in_order ? 1 : 0, nits,
+                       ioff, out);
 }
 
 void launch_items_per_sc(const int *costs, int nsc, int per_item, int *nitems, hipStream_t s)

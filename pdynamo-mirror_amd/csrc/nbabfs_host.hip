@@ -1527,7 +1527,8 @@ static int recut_items(nbabfs_state *S, int per_item)
     if (nb > 0) {
         CHK(S->inits.ensure(nb));
         CHK(S->iioff.ensure(nb));
-        launch_image_items(S->icosts.p, nb, image_item_cost(S->opt), S->inits.p, S->iioff.p, S->tail.d + 4, st);
+        launch_image_items(S->icosts.p, nb, image_item_cost(S->opt), S->opt.precision == NBABFS_PLAIN_FP64, S->inits.p,
+                           S->iioff.p, S->tail.d + 4, st);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));

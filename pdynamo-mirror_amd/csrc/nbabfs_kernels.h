@@ -173,7 +173,8 @@ void launch_export_image_pairs(const Entry *entries, int nent, const int *slot_a
                                unsigned long long *cursor, long long cap, long long *keys, hipStream_t s);
 // Items per block (ceil(costs / per_item)); the sum of the block costs into mapped host memory.
 void launch_items_per_sc(const int *costs, int nsc, int per_item, int *nitems, hipStream_t s);
-void launch_image_items(const int *costs, int m, int per_item, int *nits, int *ioff, int *out, hipStream_t s);
+// in_order: the items in block order (else by falling cost, in no fixed order).
+void launch_image_items(const int *costs, int m, int per_item, bool in_order, int *nits, int *ioff, int *out, hipStream_t s);
 // Entry and item offsets (exclusive scans of counts and of ceil(costs / per_item), per_item from the cut and the total
 // cost) and {entries, items, *need, per_item} into out, in one launch; false (nothing launched) when nsc is beyond its
 // single workgroup.

@@ -143,3 +143,37 @@ def test_image_rebuild_on_cell_change_only(oracle_mod):
         assert np.linalg.norm(g - rgrad) / np.linalg.norm(rgrad) <= 1e-5
         assert np.abs(dm - rdm).max() <= 1e-5 * np.abs(rdm).max()
     st.close()
+
+
+def test_plain_fp64_image_energies_repeat():
+    """Plain FP64: the image energies are FP64 sums over the work items, so the items' order is part of the result.
+    Every build of the same lists, by new states and by one state back at the same coordinates, gives the same bits."""
+    from pdynamo_amd import _native, synthetic
+    w, tr, sp = synthetic.periodic_water_box(4000, 49.3, seed=11)
+    o = _native.default_options()
+    o.precision = _native.PLAIN_FP64
+
+    def state():
+        st = _native.NativeState(o, w.charges, w.ljtypes, w.ntypes, w.tableA, w.tableB, exclusions=w.exclusions)
+        st.set_transformations(tr[0], tr[1])
+        st.set_symmetry_parameters(sp)
+        return st
+
+    def images(st):
+        g = np.zeros_like(w.coordinates3)
+        st.energy_host(w.coordinates3, g)
+        dm = np.zeros((3, 3))
+        e, _ = st.image_terms(dm)
+        return tuple(e), g, dm
+
+    kept = state()
+    ref = images(kept)
+    for k in range(8):
+        st = state()
+        e, g, dm = images(st)
+        st.close()
+        assert e == ref[0], (k, e, ref[0])
+        assert np.array_equal(g, ref[1]) and np.array_equal(dm, ref[2])
+        kept.energy_host(w.coordinates3 + 1.0, np.zeros_like(g))       # lists of other coordinates between
+        assert images(kept)[0] == ref[0]
+    kept.close()
