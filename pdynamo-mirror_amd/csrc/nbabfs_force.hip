@@ -656,15 +656,18 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
     unsigned char *region = lds + rows_bytes + (size_t)wave * wave_bytes;
     acc_t *sJ = (acc_t *)(region + NB_LDS_I_BYTES);   // [entry][j-atom] of (x, y, z, J)
     // One item per wave: ask for all it needs, then stage the group's row table (the items of a group belong to one
-    // system).
+    // system; in a batch, its first item's).
     ItemStart st = {};
+    int rows_sys = -1;
     if (!QUEUE) {
+        if (ROWS_LDS && !IMG && sys1 < 0) rows_sys = items[(int)blockIdx.x * WPG].sys;
         w0 = uniform_item(w0);
         const SysDesc *D0 = &descs[sys1 >= 0 ? sys1 : (IMG ? (w0.sys & 0xffff) : w0.sys)];
         st = item_start<IMG>(D0, w0, lane);
         if (ROWS_LDS) {
-            const GAS double *__restrict__ rows0 = as_global(D0->ljrow);
-            const int nr = 2 * D0->ntypes * D0->ntypes;
+            const SysDesc *DR = rows_sys >= 0 ? &descs[rows_sys] : D0;
+            const GAS double *__restrict__ rows0 = as_global(DR->ljrow);
+            const int nr = 2 * DR->ntypes * DR->ntypes;
             for (int k = threadIdx.x; k < nr; k += 64 * WPG) sR[k] = load_slot(rows0, k);
             if (WPG > 1) __syncthreads();
         }
@@ -696,6 +699,12 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 
             it = (int)blockIdx.x * WPG + wave;
             // Empty items pad a batch's systems to whole groups.
             if (it >= nitems || w.count <= 0) break;
+            // An item of another system than the staged rows would be a layout error (reported, never evaluated with the
+            // wrong rows).
+            if (rows_sys >= 0 && w.sys != rows_sys) {
+                raise_error(descs[rows_sys].err, true, NB_ERR_RANGE);
+                break;
+            }
         }
         const SysDesc *D = &descs[sys1 >= 0 ? sys1 : (IMG ? (w.sys & 0xffff) : w.sys)];
         const GAS double *__restrict__ xq = (const GAS double *)D->xyzq;

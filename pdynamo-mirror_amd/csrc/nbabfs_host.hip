@@ -2697,7 +2697,7 @@ static int batch_layout(nbabfs_batch *B, const double *const *d_xyz, double *con
     int total = 0;
     B->max_npad = B->max_n = B->max_n14b = 0;
     for (auto *s : B->st) {
-        total += nblk(s->nitems, NB_TILED_WPG) * NB_TILED_WPG;
+        total += padded_items(s->nitems);
         B->max_npad = std::max(B->max_npad, s->n_pad);
         B->max_n = std::max(B->max_n, s->n);
         B->max_n14b = std::max(B->max_n14b, nblk(s->n14, NB_P14_BLOCK));
@@ -2715,7 +2715,7 @@ static int batch_layout(nbabfs_batch *B, const double *const *d_xyz, double *con
         SysDesc &D = B->h_desc.p[k];
         fill_desc(s, D, d_xyz[k], d_grad ? d_grad[k] : nullptr);
         D.energies = B->energies.d + NB_NENERGIES * (size_t)k;
-        const int padded = nblk(s->nitems, NB_TILED_WPG) * NB_TILED_WPG;
+        const int padded = padded_items(s->nitems);
         if (padded > 0)
             hipLaunchKernelGGL(k_remap_items, dim3(nblk(padded, 256)), dim3(256), 0, st, s->items.p, s->nitems, padded,
                                k, B->items.p + first);

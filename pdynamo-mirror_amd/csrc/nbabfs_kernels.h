@@ -238,6 +238,7 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
 // Waves per workgroup of the one-item-per-wave pair launches; a batch pads each system's items to a multiple of it
 // (items of one workgroup share a system and its LJ row table).
 #define NB_TILED_WPG 4
+inline int padded_items(int nitems) { return (nitems + NB_TILED_WPG - 1) / NB_TILED_WPG * NB_TILED_WPG; }
 // The plain FP64 CSR pass of nsys systems in one launch (blockIdx.y = system; rows from the descriptors).
 void launch_force_plain(const SysDesc *d_desc, int nsys, int max_n, const AbfsFactors &F, ForceGuard g, hipStream_t s,
                         hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
