@@ -619,7 +619,7 @@ struct PairFactors {
 };
 
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(F64 ? 3 : (IMG ? 4 : 5)))) void k_force_tiled(
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(tiled_waves(F64, IMG)))) void k_force_tiled(
     const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, typename PairFactors<F64>::type F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {

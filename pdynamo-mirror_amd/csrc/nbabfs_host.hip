@@ -921,12 +921,14 @@ static int image_item_cost(const nbabfs_options &o)
     return std::max(NB_MIN_ITEM_COST, NB_IMAGE_ENTRY_COST * per);
 }
 
-// The cut of the main list for entriesPerItem; the waves the GPU holds at once are five per SIMD (mixed) or three (full
-// FP64).  The persistent queues cut every list alike.
-static ItemCut item_cut(const nbabfs_options &o, int per_item)
+// The cut of the main list for entriesPerItem, for the waves that its launch's instance lets the GPU hold at once (with
+// crystal symmetry the one that takes image items too; between cuts for its four waves per SIMD and for five no call of
+// 2,400 to 23,559 atoms in a cell differs beyond the runs of one side, 110 us for the largest).  The persistent queues
+// cut every list alike.
+static ItemCut item_cut(const nbabfs_options &o, int per_item, bool images)
 {
     const int cu = g_cu_count > 0 ? g_cu_count : 256;
-    const int held = 4 * cu * (o.precision == NBABFS_TILED_FP64 ? 3 : 5);
+    const int held = 4 * cu * tiled_waves(o.precision == NBABFS_TILED_FP64, images);
     return ItemCut{NB_ENTRY_COST * std::max(1, per_item > 0 ? per_item : 16), o.wavesPerCU > 0 ? 0 : held};
 }
 
@@ -1122,7 +1124,7 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     CHK(S->ncand.ensure(S->nsc));
     // Search, then the entry and item offsets; the totals and the capacity
     // check reach the host through mapped memory in one synchronisation.
-    const ItemCut cut = item_cut(o, o.entriesPerItem);
+    const ItemCut cut = item_cut(o, o.entriesPerItem, S->has_sym);
     CHK(S->costs.ensure(S->nsc));
     CHK(S->eoff.ensure(S->nsc + 1));
     CHK(S->nits.ensure(S->nsc));
@@ -1514,7 +1516,7 @@ static int recut_items(nbabfs_state *S, int per_item)
     if (S->nsc <= 0) return NBABFS_STATUS_CONTINUE;
     const int nb = (int)S->slots.size() * S->nsc;
     CHK(S->tail.ensure(16));
-    const ItemCut cut = item_cut(S->opt, per_item);
+    const ItemCut cut = item_cut(S->opt, per_item, S->has_sym);
     if (!launch_list_offsets(S->counts.p, S->costs.p, S->nsc, cut, S->eoff.p, S->nits.p, S->ioff.p, S->flag.p, S->tail.d,
                              st)) {
         const int units = std::max(NB_MIN_ITEM_COST, cut.most);

@@ -5,6 +5,8 @@ compiled from that header evaluates them.
 """
 
 import os
+import re
+import shutil
 import subprocess
 
 import numpy as np
@@ -25,6 +27,10 @@ int main()
             int n;
             std::cin >> n;
             std::cout << padded_items(n) << "\n";
+        } else if (what == "waves") {
+            int full_fp64, images;
+            std::cin >> full_fp64 >> images;
+            std::cout << tiled_waves(full_fp64 != 0, images != 0) << "\n";
         }
     }
 }
@@ -59,3 +65,24 @@ def test_batch_groups_hold_one_system(rules):
         owner = np.repeat(np.arange(len(counts)), padded)
         assert owner.size % group == 0
         assert (owner.reshape(-1, group) == owner.reshape(-1, group)[:, :1]).all()
+
+
+def test_lists_are_cut_for_the_waves_the_kernel_holds(rules, tmp_path):
+    """tiled_waves, for which a list is cut to whole rounds of waves, is what the registers of the built kernel's
+    instances allow (512 per lane and SIMD, in steps of 8)."""
+    from pdynamo_amd import build
+    if not os.path.exists(build.LIB):
+        build.build()
+    lib = shutil.copy(build.LIB, tmp_path)
+    llvm = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(build.HIPCC))), "llvm", "bin")
+    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", lib], cwd=tmp_path, capture_output=True, check=True)
+    notes = "".join(subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", str(f)], capture_output=True, text=True,
+                                   check=True).stdout for f in sorted(tmp_path.glob("*gfx950*")))
+    found = 0
+    # Template arguments: rows in LDS, images, full FP64, waves per workgroup.
+    for img, full, rest in re.findall(r"\.name: +_Z13k_force_tiledILb[01]ELb([01])ELb([01])ELi4E(.*?)\.vgpr_spill_count",
+                                      notes, re.S):
+        vgprs = int(re.search(r"\.vgpr_count: +(\d+)", rest).group(1))
+        assert rules(["waves %s %s" % (full, img)]) == [[512 // ((vgprs + 7) // 8 * 8)]], (img, full, vgprs)
+        found += 1
+    assert found == 6
