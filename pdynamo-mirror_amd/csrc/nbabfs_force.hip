@@ -612,14 +612,15 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // the row table is staged once for four items and a group's LDS stays small
 // enough for five waves per SIMD; the four items of a group belong to one
 // system (batches pad each system's items to a multiple of 4 with empty
-// ones).  The persistent queues run one wave per group.
+// ones).  The persistent queues run one wave per group, at four waves per SIMD: their loop over items takes 111 VGPRs, and
+// at five it spilled (30,000 atoms on four waves per CU 135 us per call, 131 without the spills; on twelve no difference).
 template <bool F64>
 struct PairFactors {
     using type = typename std::conditional<F64, FullFactors, TiledFactors>::type;
 };
 
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(tiled_waves(F64, IMG)))) void k_force_tiled(
+__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(tiled_waves(F64, IMG, WPG == 1)))) void k_force_tiled(
     const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, typename PairFactors<F64>::type F, int rows_bytes,
     int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {

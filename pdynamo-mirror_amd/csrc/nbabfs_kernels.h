@@ -96,8 +96,12 @@ __host__ __device__ inline int entry_cost(int cbits)
 #define NB_IMAGE_ENTRY_COST 6  // the average entry of the image lists (a cell's faces)
 #define NB_MIN_ITEM_COST 34     // twice the largest entry's cost: a block's equal steps are then longer than any entry
 
-// Waves per SIMD of the pair kernel's instances (k_force_tiled says why), which its list is cut for.
-__host__ __device__ constexpr int tiled_waves(bool full_fp64, bool images) { return full_fp64 ? 3 : (images ? 4 : 5); }
+// Waves per SIMD of the pair kernel's instances (k_force_tiled says why), which its list is cut for (the persistent
+// queues' lists are not).
+__host__ __device__ constexpr int tiled_waves(bool full_fp64, bool images, bool queue = false)
+{
+    return full_fp64 ? 3 : (images || queue ? 4 : 5);
+}
 
 // The cut of a list: `most` is the nominal cost of an item, `held` the waves the GPU holds at once (0: always the nominal
 // cost).

@@ -28,9 +28,9 @@ int main()
             std::cin >> n;
             std::cout << padded_items(n) << "\n";
         } else if (what == "waves") {
-            int full_fp64, images;
-            std::cin >> full_fp64 >> images;
-            std::cout << tiled_waves(full_fp64 != 0, images != 0) << "\n";
+            int full_fp64, images, queue;
+            std::cin >> full_fp64 >> images >> queue;
+            std::cout << tiled_waves(full_fp64 != 0, images != 0, queue != 0) << "\n";
         }
     }
 }
@@ -80,9 +80,10 @@ def test_lists_are_cut_for_the_waves_the_kernel_holds(rules, tmp_path):
                                    check=True).stdout for f in sorted(tmp_path.glob("*gfx950*")))
     found = 0
     # Template arguments: rows in LDS, images, full FP64, waves per workgroup.
-    for img, full, rest in re.findall(r"\.name: +_Z13k_force_tiledILb[01]ELb([01])ELb([01])ELi4E(.*?)\.vgpr_spill_count",
-                                      notes, re.S):
+    for img, full, wpg, rest in re.findall(r"\.name: +_Z13k_force_tiledILb[01]ELb([01])ELb([01])ELi(\d)E"
+                                           r"(.*?)\.vgpr_spill_count", notes, re.S):
         vgprs = int(re.search(r"\.vgpr_count: +(\d+)", rest).group(1))
-        assert rules(["waves %s %s" % (full, img)]) == [[512 // ((vgprs + 7) // 8 * 8)]], (img, full, vgprs)
+        queue = int(wpg == "1")
+        assert rules(["waves %s %s %d" % (full, img, queue)]) == [[512 // ((vgprs + 7) // 8 * 8)]], (img, full, wpg, vgprs)
         found += 1
-    assert found == 6
+    assert found == 10
