@@ -29,9 +29,10 @@ pytestmark = pytest.mark.gpu
 TOL = {"mixed": (1e-6, 1e-5, 1e-5), "fp64": (1e-11, 1e-10, 1e-9)}
 
 
-def _state(fx, precision="mixed"):
+def _state(fx, precision="mixed", waves=0):
     from pdynamo_amd import _native
     o = _native.default_options()
+    o.wavesPerCU = waves
     o.precision = _native.MIXED if precision == "mixed" else _native.PLAIN_FP64
     o.cutoffCellSizeFactor = float(fx["options"][2])
     o.useGridByCell = 1 if bool(fx.get("grid_by_cell", True)) else 0
@@ -56,9 +57,20 @@ def _check_call(e6, grad, dEdM, ref_e6, ref_grad, ref_dEdM, tol):
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
 @pytest.mark.parametrize("path", IMAGE_FIXTURES, ids=lambda p: os.path.basename(p)[:-4])
 def test_image_fixtures(path, precision):
+    _image_fixture(path, precision, 0)
+
+
+@pytest.mark.parametrize("path", IMAGE_FIXTURES, ids=lambda p: os.path.basename(p)[:-4])
+def test_image_fixtures_persistent(path):
+    """wavesPerCU > 0: the persistent launch takes main items only, and the image items run in a launch of their own
+    beside it, on the second stream."""
+    _image_fixture(path, "mixed", 12)
+
+
+def _image_fixture(path, precision, waves):
     fx = dict(np.load(path, allow_pickle=False))
-    print("image fixture", os.path.basename(path), precision, flush=True)
-    st = _state(fx, precision)
+    print("image fixture", os.path.basename(path), precision, waves, flush=True)
+    st = _state(fx, precision, waves)
     off = 0
     keys0 = image_fixture_keys(fx)
     for k, (xyz, sp) in enumerate(zip(fx["coords"], fx["cells"])):
@@ -177,3 +189,33 @@ def test_plain_fp64_image_energies_repeat():
         kept.energy_host(w.coordinates3 + 1.0, np.zeros_like(g))       # lists of other coordinates between
         assert images(kept)[0] == ref[0]
     kept.close()
+
+
+def test_autotune_with_images(oracle_mod):
+    """The work-item autotuner on a periodic state (its persistent candidates launch the image items apart): the lists
+    stay, and energies, gradients and dE/dM stay within the tolerances of the oracle."""
+    from pdynamo_amd import _native, synthetic
+    w, tr, sp = synthetic.periodic_water_box(800, 29.0, seed=13)
+    st = _native.NativeState(_native.default_options(), w.charges, w.ljtypes, w.ntypes, w.tableA, w.tableB,
+                             exclusions=w.exclusions)
+    st.set_transformations(tr[0], tr[1])
+    st.set_symmetry_parameters(sp)
+    g = np.zeros_like(w.coordinates3)
+    st.energy_host(w.coordinates3, g)
+    images = st.images()
+    x = _native.DeviceArray.from_numpy(w.coordinates3, st)
+    epi, wpc, ms = st.autotune(x.ptr)
+    assert epi in (8, 12, 16, 24, 32, 48) and wpc in (0, 12) and ms > 0.0
+    assert st.images() == images
+    g[:] = 0.0
+    e, present, rebuilt = st.energy_host(w.coordinates3, g)
+    dm = np.zeros((3, 3))
+    ie, _ = st.image_terms(dm)
+    assert not rebuilt
+    orc = oracle_mod.OracleABFS(w, transformations=tr)
+    rterms, rgrad, rdm, _ = orc.energy_sym(w.coordinates3, sp)
+    t = dict(rterms)
+    ref = [t.get(l, 0.0) for l in IMAGE_LABELS]
+    _check_call(list(e) + list(ie), g, dm, ref, rgrad, rdm, TOL["mixed"])
+    x.free()
+    st.close()

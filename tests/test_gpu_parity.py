@@ -182,6 +182,25 @@ def test_sort_key_counts(oracle_mod, natoms, side):
     assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
 
 
+def test_more_super_clusters_than_one_workgroup_scans(oracle_mod):
+    """Above 65,536 super-clusters the entry and item offsets come from block scans and the nominal cut: a wide thin
+    layer of pairs of atoms (one or two to a column, some 85,000 columns with atoms) has that many without millions of
+    atoms."""
+    from pdynamo_amd import synthetic
+    natoms, side = 240000, 9900.0
+    rng = np.random.default_rng(natoms)
+    mm = synthetic.random_small_system(natoms, 60.0, 3)
+    c = rng.uniform(0.0, 1.0, (natoms // 2, 3)) * [side, side, 0.6]
+    mm.coordinates3 = np.concatenate([c, c + rng.uniform(-1.0, 1.0, c.shape) * [7.0, 7.0, 0.2]])
+    s = _system(mm)
+    _, terms, grad = _run(s)
+    assert s.configuration.nbState.Statistics()["clusters"] > 8 * 65536
+    o = oracle_mod.OracleABFS(mm, nthreads=8)
+    rterms, rgrad, _ = o.energy(mm.coordinates3)
+    assert np.array_equal(s.configuration.nbState.Pairs(), o.records.canonical())
+    _check(terms, grad, rterms, rgrad, 1e-6, 1e-5, "", o.abs_sums(mm.coordinates3))
+
+
 def _water_with_14(nwater, box, seed):
     """Waters on a jittered lattice (no overlapping atoms: the Coulomb and 1-4 terms are not small beside the
     LJ term) plus intermolecular "1-4" pairs between atoms 2.5-5 A apart, excluded from the main list as a
