@@ -1027,9 +1027,8 @@ __global__ __launch_bounds__(NB_COMPACT_THREADS) void k_compact(const Entry *__r
 // Work items of a compacted list: the entries of block s (a super-cluster, or
 // an (image, super-cluster) block of the image lists: images != 0, each item's
 // sys field then carries (image + 1) << 16) are cut at equal steps of their
-// summed cost into the block's n items.  Entry i starts item q when its
-// exclusive cost prefix p reaches q's step, q = p n / C; a step is longer than
-// any entry's cost (NB_MIN_ITEM_COST), so no item is empty.
+// summed cost into the block's n items.  An entry starts item q when its
+// exclusive cost prefix reaches q's step (item_of).
 __global__ __launch_bounds__(256) void k_cut_items(const int *__restrict__ counts, const int *__restrict__ costs,
                                                    const int *__restrict__ eoff, const int *__restrict__ ioff,
                                                    const int *__restrict__ nits, int nsc, int sys, int images,
@@ -1060,9 +1059,9 @@ __global__ __launch_bounds__(256) void k_cut_items(const int *__restrict__ count
         const int p = before + incl - c;
         if (k < cnt) {
             // q of this entry and of the one before it (whose prefix is p minus its own cost: only the step matters).
-            const int q = (int)((long long)p * n / total);
+            const int q = item_of(p, n, total);
             const int cp = k > 0 ? entry_cost(entries[e0 + k - 1].cbits) : 0;
-            const int qp = k > 0 ? (int)((long long)(p - cp) * n / total) : -1;
+            const int qp = k > 0 ? item_of(p - cp, n, total) : -1;
             if (q != qp) {
                 WorkItem &o = own[q];
                 o.first = e0 + k;
@@ -1128,7 +1127,7 @@ __global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__r
     }
     const int per_item = item_cost(cut, tc, m);
     int si = 0;
-    for (int k = lo; k < hi; k++) si += (costs[k] + per_item - 1) / per_item;
+    for (int k = lo; k < hi; k++) si += items_of(costs[k], per_item);
     int ii = si;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -1144,7 +1143,7 @@ __global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__r
     }
     int e = be + ie - se, i = bi + ii - si;
     for (int k = lo; k < hi; k++) {
-        const int ni = (costs[k] + per_item - 1) / per_item;
+        const int ni = items_of(costs[k], per_item);
         eoff[k] = e;
         ioff[k] = i;
         nits[k] = ni;
@@ -1165,7 +1164,7 @@ __global__ __launch_bounds__(256) void k_items_per_sc(const int *__restrict__ co
                                                       int *__restrict__ nitems)
 {
     int s = blockIdx.x * 256 + threadIdx.x;
-    if (s < nsc) nitems[s] = (costs[s] + per_item - 1) / per_item;
+    if (s < nsc) nitems[s] = items_of(costs[s], per_item);
 }
 
 // Items of the image lists' blocks and where each block's items go, in one workgroup; *out: their number.  A block cuts
@@ -1174,7 +1173,6 @@ __global__ __launch_bounds__(256) void k_items_per_sc(const int *__restrict__ co
 // differ much more than the main list's, and a long one at the end of a launch is waited for: 23,559 atoms in a 50 A cell
 // took 150 us per call in block order and 139 us in this one.  in_order: the blocks' own order, for the plain path, which
 // adds FP64 energies item by item: there the order is part of the result.
-#define NB_IORDER_BINS 256
 __global__ __launch_bounds__(NB_KEYSCAN_THREADS) void k_image_items(const int *__restrict__ costs, int m, int per_item,
                                                                     int in_order, int *__restrict__ nits,
                                                                     int *__restrict__ ioff, int *__restrict__ out)
@@ -1186,10 +1184,10 @@ __global__ __launch_bounds__(NB_KEYSCAN_THREADS) void k_image_items(const int *_
         const int chunk = (m + NB_KEYSCAN_THREADS - 1) / NB_KEYSCAN_THREADS;
         const int lo = min(t * chunk, m), hi = min(lo + chunk, m);
         int v = 0, total;
-        for (int k = lo; k < hi; k++) v += (costs[k] + per_item - 1) / per_item;
+        for (int k = lo; k < hi; k++) v += items_of(costs[k], per_item);
         int o = block_exclusive(v, sW, total);
         for (int k = lo; k < hi; k++) {
-            const int n = (costs[k] + per_item - 1) / per_item;
+            const int n = items_of(costs[k], per_item);
             nits[k] = n;
             ioff[k] = o;
             o += n;
@@ -1197,13 +1195,12 @@ __global__ __launch_bounds__(NB_KEYSCAN_THREADS) void k_image_items(const int *_
         if (t == 0) *(volatile int *)out = total;
         return;
     }
-    auto bin = [&](int c, int n) { return NB_IORDER_BINS - 1 - (int)((long long)(c / n) * (NB_IORDER_BINS - 1) / per_item); };
     if (t < NB_IORDER_BINS) sH[t] = 0;
     __syncthreads();
     for (int k = t; k < m; k += NB_KEYSCAN_THREADS) {
-        const int c = costs[k], n = (c + per_item - 1) / per_item;
+        const int c = costs[k], n = items_of(c, per_item);
         nits[k] = n;
-        if (n > 0) atomicAdd(&sH[bin(c, n)], n);
+        if (n > 0) atomicAdd(&sH[item_bin(c, n, per_item)], n);
     }
     __syncthreads();
     int own = 0, before = 0;
@@ -1216,8 +1213,8 @@ __global__ __launch_bounds__(NB_KEYSCAN_THREADS) void k_image_items(const int *_
     if (t == NB_IORDER_BINS - 1) *(volatile int *)out = before + own;
     __syncthreads();
     for (int k = t; k < m; k += NB_KEYSCAN_THREADS) {
-        const int c = costs[k], n = (c + per_item - 1) / per_item;
-        ioff[k] = n > 0 ? atomicAdd(&sH[bin(c, n)], n) : 0;
+        const int c = costs[k], n = items_of(c, per_item);
+        ioff[k] = n > 0 ? atomicAdd(&sH[item_bin(c, n, per_item)], n) : 0;
     }
 }
 

@@ -134,6 +134,17 @@ __host__ __device__ inline int item_cost(const ItemCut &c, long long total, int 
     return (int)(t > NB_MIN_ITEM_COST ? t : NB_MIN_ITEM_COST);
 }
 
+// Items of a block of this cost, and the item of a block's entry whose exclusive cost prefix is p: equal steps of the
+// block's total.  A step is longer than any entry's cost when per_item is at least NB_MIN_ITEM_COST, so no item is empty.
+__host__ __device__ inline int items_of(int cost, int per_item) { return (cost + per_item - 1) / per_item; }
+__host__ __device__ inline int item_of(int p, int n, int total) { return (int)((long long)p * n / total); }
+// Place of a block's n items in the image lists' order by falling item cost, in NB_IORDER_BINS steps.
+#define NB_IORDER_BINS 256
+__host__ __device__ inline int item_bin(int cost, int n, int per_item)
+{
+    return NB_IORDER_BINS - 1 - (int)((long long)(cost / n) * (NB_IORDER_BINS - 1) / per_item);
+}
+
 // List construction (nbabfs_build.hip).
 void launch_bbox(const double *xyz, int n, double *part, int nparts, double *out, hipStream_t s);
 void launch_bin(const double *xyz, int n, const BuildGrid &g, int4 *cellv, int *key, int *count, hipStream_t s);

@@ -17,6 +17,7 @@ HARNESS = r"""
 #include "nbabfs_kernels.h"
 #include <iostream>
 #include <string>
+#include <vector>
 int main()
 {
     std::string what;
@@ -31,6 +32,40 @@ int main()
             int full_fp64, images, queue;
             std::cin >> full_fp64 >> images >> queue;
             std::cout << tiled_waves(full_fp64 != 0, images != 0, queue != 0) << "\n";
+        } else if (what == "entry_costs") {
+            for (int cbits = 0; cbits < 256; cbits++) std::cout << entry_cost(cbits) << " ";
+            std::cout << NB_MIN_ITEM_COST << "\n";
+        } else if (what == "item_cost") {
+            ItemCut c;
+            long long total;
+            int nsc;
+            std::cin >> c.most >> c.held >> total >> nsc;
+            std::cout << item_cost(c, total, nsc) << "\n";
+        } else if (what == "cut") {         // the entries of a block: the items' first entries
+            int per_item, m, total = 0, p = 0;
+            std::cin >> per_item >> m;
+            std::vector<int> cost(m);
+            for (int &c : cost) {
+                std::cin >> c;
+                total += c;
+            }
+            const int n = items_of(total, per_item);
+            std::cout << n;
+            for (int k = 0; k < m; k++) {
+                const int q = item_of(p, n, total), before = k > 0 ? item_of(p - cost[k - 1], n, total) : -1;
+                if (q != before) std::cout << " " << q << " " << k;
+                p += cost[k];
+            }
+            std::cout << "\n";
+        } else if (what == "bins") {
+            int per_item, m, c;
+            std::cin >> per_item >> m;
+            for (int k = 0; k < m; k++) {
+                std::cin >> c;
+                const int n = items_of(c, per_item);
+                std::cout << n << " " << (n > 0 ? item_bin(c, n, per_item) : -1) << " ";
+            }
+            std::cout << NB_IORDER_BINS << "\n";
         }
     }
 }
@@ -87,3 +122,72 @@ def test_lists_are_cut_for_the_waves_the_kernel_holds(rules, tmp_path):
         assert rules(["waves %s %s %d" % (full, img, queue)]) == [[512 // ((vgprs + 7) // 8 * 8)]], (img, full, wpg, vgprs)
         found += 1
     assert found == 10
+
+
+def test_no_work_item_is_empty(rules):
+    """The cut of a block's entries at equal steps of their cost: every item of the block starts at exactly one entry, in
+    order, the first at the first entry, and no item costs more than a step and an entry; for costs of every kind, the
+    smallest cost per item, and totals just above a whole number of items."""
+    costs = rules(["entry_costs"])[0]
+    least = costs.pop()
+    top, some = max(costs), sorted(set(costs) - {0})
+    assert costs[0] == 0 and least == 2 * top
+    rng = np.random.default_rng(4)
+    blocks = [[top] * m for m in range(1, 300)] + [[some[0]] * m for m in range(1, 300)]
+    blocks += [rng.choice(some, rng.integers(1, 700)).tolist() for _ in range(300)]
+    blocks += [[top] * m + [some[0]] * r for m in (2, 4, 64) for r in range(1, 13)]
+    blocks += [[some[0]] * r + [top] * m for m in (2, 4, 64) for r in range(1, 13)]
+    cases = [(per, b) for b in blocks for per in (least, least + 1, 44, 176, 1408)]
+    for (per, b), got in zip(cases, rules(["cut %d %d %s" % (per, len(b), " ".join(map(str, b))) for per, b in cases])):
+        n, q, first = got[0], got[1::2], got[2::2]
+        assert n == -(-sum(b) // per) and q == list(range(n)) and first[0] == 0
+        ends = first[1:] + [len(b)]
+        assert all(0 < e - f for f, e in zip(first, ends))
+        assert all(sum(b[f:e]) <= sum(b) / n + top for f, e in zip(first, ends))
+
+
+def test_cost_per_item_follows_its_rules(rules):
+    """item_cost: the nominal cost without a limit of waves; from a quarter of it for short lists; whole rounds of waves for
+    long ones, half an item per block included; never below the smallest cost."""
+    least = rules(["entry_costs"])[0][-1]
+    rng = np.random.default_rng(5)
+    cases = [(int(m), int(h), int(t), int(b)) for m, h, t, b in
+             zip(rng.choice([11, 44, 176, 352, 1408], 4000), rng.choice([0, 3072, 4096, 5120], 4000),
+                 np.exp(rng.uniform(0.0, 20.0, 4000)), rng.integers(1, 4000, 4000))]
+    for (most, held, total, nsc), (got,) in zip(cases, rules(["item_cost %d %d %d %d" % c for c in cases])):
+        nominal = max(most, least)
+        assert got >= least
+        if held == 0:
+            assert got == nominal
+        elif total < most * (held // 16):
+            assert max(most // 4, least) <= got <= nominal
+        elif total < most * held // 2:
+            assert got == nominal
+        elif got > least and got != most:
+            rounds = (total + most * held // 2) // (most * held)
+            assert total / got + nsc // 2 <= rounds * held
+            assert got <= 3 * most + 1
+
+
+def test_image_items_tile_their_list_by_falling_cost(rules):
+    """The image lists' layout: the blocks of a step of cost follow those of the steps above it, so the offsets made from
+    the steps' totals give every item one place."""
+    rng = np.random.default_rng(6)
+    for per in (34, 66, 96, 768):
+        c = np.concatenate([rng.integers(0, 20 * per, 3000), np.arange(0, 3 * per)])
+        got = rules(["bins %d %d %s" % (per, c.size, " ".join(map(str, c)))])[0]
+        bins = got.pop()
+        n, step = np.array(got[0::2]), np.array(got[1::2])
+        assert (n == -(-c // per)).all()
+        used = n > 0
+        assert (step[used] >= 0).all() and (step[used] < bins).all()
+        each = c[used] // n[used]
+        order = np.argsort(each, kind="stable")
+        assert (np.diff(step[used][order]) <= 0).all()
+        start = np.concatenate([[0], np.cumsum(np.bincount(step[used], weights=n[used], minlength=bins))]).astype(int)
+        place, cursor = [], start[:-1].copy()
+        for k in rng.permutation(np.flatnonzero(used)):
+            place.extend(range(cursor[step[k]], cursor[step[k]] + n[k]))
+            cursor[step[k]] += n[k]
+        assert np.array_equal(np.sort(place), np.arange(n.sum()))
+        assert (cursor == start[1:]).all()

@@ -1,17 +1,12 @@
-"""CPU checks that the pair kernel's results cannot depend on the order of its work items.
+"""CPU checks that the tiled kernel's results cannot depend on the order of its work items.
 
-Two parts of the device code decide this, restated here in numpy:
+The fixed-point sums (``fx_split``/``fx_value`` in csrc/nbabfs_internal.h) decide this, restated here in numpy: every
+force and energy contribution becomes two int64 words, hi = rint(v / 2^16) and lo = rint((v - hi 2^16) 2^32), added with
+integer atomics.  Integer addition is associative, so any order of the items gives the same words, and the words convert
+to the same double.  An item's energy is added as twice its value, with twice the range.
 
-* the fixed-point sums (``fx_split``/``fx_value`` in csrc/nbabfs_internal.h): every force and energy
-  contribution becomes two int64 words, hi = rint(v / 2^16) and lo = rint((v - hi 2^16) 2^32), added with
-  integer atomics.  Integer addition is associative, so any order of the items gives the same words, and the
-  words convert to the same double.
-* the longest-first item order (``k_item_order`` in csrc/nbabfs_build.hip): a histogram of the costs kept in
-  four copies (wave w adds into copy w % 4), an exclusive scan over (bin, copy) and a scatter.  It must be a
-  permutation of the items with non-increasing cost, whatever the assignment of items to waves.
-
-The plain FP64 path does not read work items at all (one thread per atom over sorted CSR rows), so its results
-are independent of the item order by construction.
+The plain FP64 path adds in FP64: its rows do not read work items (one thread per atom over sorted CSR rows), and its
+image items keep one order (tests/test_gpu_images.py).  How items are cut and laid out: tests/test_item_rules_cpu.py.
 """
 
 import numpy as np
@@ -20,8 +15,8 @@ HI_UNIT = 2.0 ** 16
 LO_SCALE = 2.0 ** 32
 
 
-def fx_split(v):
-    v = np.clip(v, -2.0 ** 66, 2.0 ** 66)
+def fx_split(v, limit=2.0 ** 66):
+    v = np.clip(v, -limit, limit)
     hi = np.rint(v / HI_UNIT)
     r = v - hi * HI_UNIT                     # exact (Sterbenz: |r| <= 2^15)
     lo = np.rint(r * LO_SCALE)
@@ -48,31 +43,18 @@ def test_fixed_point_sums_do_not_depend_on_item_order():
     assert np.max(np.abs(back[small] - v[small])) <= 2.0 ** -32
 
 
-def item_order(cost, maxcost, threads=1024, copies=4, unroll=8):
-    """k_item_order's scatter for one assignment of items to threads (thread t takes items t, t + threads, ...)."""
-    n = cost.size
-    bins = maxcost + 1
-    hist = np.zeros((bins, copies), np.int64)
-    owner = (np.arange(n) % threads) // 64 % copies          # copy of the wave that holds item k
-    np.add.at(hist, (maxcost - cost, owner), 1)
-    flat = hist.reshape(-1)
-    start = np.concatenate([[0], np.cumsum(flat)[:-1]]).reshape(bins, copies)
-    out = np.full(n, -1, np.int64)
-    cursor = start.copy()
-    # any interleaving of the atomics inside one (bin, copy) only permutes equal-cost items
-    order = np.random.default_rng(1).permutation(n)
-    for k in order:
-        b, c = maxcost - cost[k], owner[k]
-        out[cursor[b, c]] = k
-        cursor[b, c] += 1
-    return out
-
-
-def test_item_order_is_a_longest_first_permutation():
-    rng = np.random.default_rng(7)
-    for n, per_item in [(13855, 48), (79436, 16), (1000, 12), (5, 8)]:
-        maxcost = 8 * per_item
-        cost = np.minimum(rng.binomial(maxcost, 0.6, n), maxcost)
-        out = item_order(cost, maxcost)
-        assert np.array_equal(np.sort(out), np.arange(n))
-        assert np.all(np.diff(cost[out]) <= 0)
+def test_item_energies_keep_their_range_and_rounding():
+    """Twice an item's energy: up to 2^66 kJ/mol is inside the range, the sum of 4,096 such items stays inside int64, and
+    an ordinary item's energy is held to 2^-34 kJ/mol, so that four times the items round to the error of one split."""
+    rng = np.random.default_rng(8)
+    e = np.concatenate([rng.uniform(-1.0, 1.0, 4094) * 2.0 ** 66, [2.0 ** 66, -2.0 ** 66]])
+    hi, lo = fx_split(2.0 * e, 2.0 ** 67)
+    assert np.abs(hi).max() == 2 ** 51 and abs(sum(int(h) for h in hi)) < 2 ** 63
+    for h, l, v in zip(hi, lo, e):
+        assert 0.5 * fx_value(int(h), int(l)) == v
+    e = rng.normal(0.0, 300.0, 20000)
+    hi, lo = fx_split(2.0 * e, 2.0 ** 67)
+    back = 0.5 * (hi.astype(np.float64) * HI_UNIT + lo.astype(np.float64) / LO_SCALE)
+    assert np.max(np.abs(back - e)) <= 2.0 ** -34
+    words = {(int(hi[p].sum()), int(lo[p].sum())) for p in (np.random.default_rng(k).permutation(e.size) for k in range(5))}
+    assert len(words) == 1
