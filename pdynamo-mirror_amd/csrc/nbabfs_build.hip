@@ -1084,9 +1084,9 @@ __global__ __launch_bounds__(256) void k_cut_items(const int *__restrict__ count
 }
 
 // Entry and item offsets of the super-clusters from their entry counts, and
-// the totals (entries, items, search capacity needed, cost per item) into
-// out[0..3], in one workgroup (each thread scans a contiguous chunk).  The cut
-// follows the list's total cost (item_cost), so the entries come first.
+// the totals (entries, items, search capacity needed) into out[0..2], in one
+// workgroup (each thread scans a contiguous chunk).  The cut follows the list's
+// total cost (item_cost), so the entries come first.
 #define NB_OFFS_THREADS 1024
 #define NB_OFFS_MAX (64 * NB_OFFS_THREADS)
 __global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__restrict__ counts,
@@ -1155,7 +1155,6 @@ __global__ __launch_bounds__(NB_OFFS_THREADS) void k_list_offsets(const int *__r
         o[0] = te;
         o[1] = ti;
         o[2] = *need;
-        o[3] = per_item;
     }
 }
 

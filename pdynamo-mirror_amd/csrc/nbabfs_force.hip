@@ -599,7 +599,8 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // A wave costs about 5 us beside its entries, and an entry's loads are a chain as long as its tiles: what a wave needs
 // first is asked for at once (ItemStart), and an item's entry headers come with one load.
 // IMG: the launch holds image items too (sys >> 16: the image plus one), beside the main list's or alone.  The j-record
-// is transformed once per entry; the image's part of the item's end takes four waves per SIMD (107 VGPRs, no spill).  One
+// is transformed once per entry; the image's part of the item's end takes four waves per SIMD (107 VGPRs, none spilled; 49
+// to 56 scalar registers are, into lanes of vector registers, and some 150 instructions in the loops read them back).  One
 // launch, because a second stream's launch starts 15 us after its fork and joins 11 us after its end, and because the
 // image items fill the GPU as the main items drain: 23,559 atoms in a 50 A cell, 139 us per call with two launches,
 // 126 us with one.
@@ -761,7 +762,7 @@ __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(tiled_
         acc_t fx[NB_SCC], fy[NB_SCC], fz[NB_SCC];
 #pragma unroll
         for (int c = 0; c < NB_SCC; c++) fx[c] = fy[c] = fz[c] = (acc_t)0;
-        // Two factors kept in vector registers: their multiply-adds already read one scalar operand.
+        // Kept in vector registers: its multiply-add already reads one scalar operand.
         double uShift = F.uShift;
         asm("" : "+v"(uShift));
         double eel = 0.0, elj = 0.0;
@@ -1321,7 +1322,7 @@ void launch_force_tiled(const SysDesc *d_desc, const WorkItem *items, QueueParam
                         hipEvent_t ev_start, hipEvent_t ev_stop, int n14_blocks, const FullFactors *full, int sys1)
 {
     if (nblocks + n14_blocks <= 0) return;
-    // One item per wave, four waves per group, unless the items come from the persistent queues or the images.
+    // One item per wave, four waves per group, unless the items come from the persistent queues.
     const int wpg = q.heads != nullptr ? 1 : NB_TILED_WPG;
     const int ngroups = nblk(nblocks, wpg);
     const dim3 grid(ngroups + nblk(n14_blocks, wpg));

@@ -423,7 +423,6 @@ struct nbabfs_state {
     int u = 0;
     DBuf<unsigned char> stencil;
     int n_pad = 0, ncl = 0, nsc = 0, nent = 0, nitems = 0, cap = 512;
-    int item_units = NB_MIN_ITEM_COST;   // cost per item of the current cut of the main list
     DBuf<int> slot_atom, atom_slot;
     DBuf<int4> cellv;
     DBuf<float4> blo, bhi, centre;
@@ -1141,10 +1140,8 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
                                  S->tail.d, st)) {
             launch_scan(S->counts.p, S->eoff.p, S->nsc, S->scantmp.p, st);
             // A list this long is cut at the nominal cost (the rule's total would have to come to the host first).
-            S->item_units = std::max(NB_MIN_ITEM_COST, cut.most);
-            launch_items_per_sc(S->costs.p, S->nsc, S->item_units, S->nits.p, st);
+            launch_items_per_sc(S->costs.p, S->nsc, std::max(NB_MIN_ITEM_COST, cut.most), S->nits.p, st);
             launch_scan(S->nits.p, S->ioff.p, S->nsc, S->scantmp.p, st);
-            ((volatile int *)S->tail.h)[3] = S->item_units;
             hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->eoff.p, S->counts.p, S->ioff.p, S->nits.p,
                                S->nsc, S->flag.p, S->tail.d);
         }
@@ -1157,7 +1154,6 @@ static int build_list(nbabfs_state *S, const double *d_xyz)
     }
     S->nent = ((volatile int *)S->tail.h)[0];
     S->nitems = ((volatile int *)S->tail.h)[1];
-    S->item_units = ((volatile int *)S->tail.h)[3];
     S->nent_main = S->nent;
     S->nitems_main = S->nitems;
     S->desc_valid = false;
@@ -1426,9 +1422,9 @@ static int launch_force(nbabfs_state *S, ForceGuard g)
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     if (S->opt.precision != NBABFS_PLAIN_FP64) {
         const int nm = S->nitems_main, ni = S->nitems - S->nitems_main;
-        // The image lists' items follow the main list's, and the mixed kernel takes both in one launch.  The full-FP64
-        // and the persistent kernels take main items only: the images' launch then runs beside theirs, on the second
-        // stream.
+        // The image lists' items follow the main list's, and the mixed kernel takes both in one launch.  The persistent
+        // kernel takes main items only: the images' launch then runs beside it, on the second stream.  (Full FP64 has no
+        // image lists.)
         const FullFactors *fp64 = S->opt.precision == NBABFS_TILED_FP64 ? &S->F64 : nullptr;
         const int n14 = nblk(S->n14, NB_P14_BLOCK);
         const QueueParams direct{nullptr, S->qstarts.p};
@@ -1519,10 +1515,8 @@ static int recut_items(nbabfs_state *S, int per_item)
     const ItemCut cut = item_cut(S->opt, per_item, S->has_sym);
     if (!launch_list_offsets(S->counts.p, S->costs.p, S->nsc, cut, S->eoff.p, S->nits.p, S->ioff.p, S->flag.p, S->tail.d,
                              st)) {
-        const int units = std::max(NB_MIN_ITEM_COST, cut.most);
-        launch_items_per_sc(S->costs.p, S->nsc, units, S->nits.p, st);
+        launch_items_per_sc(S->costs.p, S->nsc, std::max(NB_MIN_ITEM_COST, cut.most), S->nits.p, st);
         launch_scan(S->nits.p, S->ioff.p, S->nsc, S->scantmp.p, st);
-        ((volatile int *)S->tail.h)[3] = units;
         hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, st, S->eoff.p, S->counts.p, S->ioff.p, S->nits.p, S->nsc,
                            S->flag.p, S->tail.d);
     }
@@ -1535,7 +1529,6 @@ static int recut_items(nbabfs_state *S, int per_item)
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     S->nitems_main = ((volatile int *)S->tail.h)[1];
-    S->item_units = ((volatile int *)S->tail.h)[3];
     const int nimg_items = nb > 0 ? ((volatile int *)S->tail.h)[4] : 0;
     S->nitems = S->nitems_main + nimg_items;
     CHK(S->items.ensure(std::max(S->nitems, 1)));

@@ -114,8 +114,10 @@ struct ItemCut {
 // entries per item, 462 with 8 and 600 with 4, and a state's cut has to serve single calls and batches alike (they give
 // the same bits).  Two rules leave the nominal cost:
 //   * A list of less than held / 16 nominal items (3,500 atoms of water) is one wave's chain long whatever the GPU could
-//     hold: it is cut into held / 16 items, down to a quarter of the nominal cost (648 atoms: 56 -> 42 us per call; such
-//     lists are a few percent of an uneven batch).
+//     hold: it is cut into held / 16 items, down to a quarter of the nominal cost (648 atoms: 56 -> 42 us per call).
+//     Batches of such lists gain too or lose little, us per call with the nominal cut and with this rule: 16 systems of
+//     900 atoms 65 and 55, 24 of 1,500 82 and 76, 64 of 1,500 129 and 127, 64 of 500 to 1,500 96 and 95, 64 of 3,000 to
+//     3,500 245 and 246, 16 of 3,400 96 and 98, the 64 droplets 412 and 417.
 //   * A list of about a whole number of rounds of waves is cut to fill them (20,001 atoms in full FP64: 144 -> 127 us).
 __host__ __device__ inline int item_cost(const ItemCut &c, long long total, int nsc)
 {
@@ -168,7 +170,7 @@ void launch_slot_records(const double *xyz, const int *slot_atom, int n_pad, con
 void launch_search(const SearchParams &P, int nsc, const double *xyz, const int *slot_atom, const float4 *blo,
                    const float4 *bhi, const int2 *colcl, Entry *scratch, int *ncand, int *counts, int *costs,
                    int *overflow, hipStream_t s);
-// images: the number of image items when the blocks are those of the image lists (else 0).
+// images: 1 when the blocks are those of the image lists, else 0.
 void launch_cut_items(const int *counts, const int *costs, const int *eoff, const int *ioff, const int *nits,
                       int nblocks, int nsc, int sys, const Entry *entries, WorkItem *items, hipStream_t s,
                       int images = 0);
@@ -189,13 +191,13 @@ void launch_image_bounds(const SearchParams &P, int nsc, int nimg, const float4 
 void launch_add_int(int *p, int m, int v, hipStream_t s);
 void launch_export_image_pairs(const Entry *entries, int nent, const int *slot_atom, long long n, int img,
                                unsigned long long *cursor, long long cap, long long *keys, hipStream_t s);
-// Items per block (ceil(costs / per_item)); the sum of the block costs into mapped host memory.
+// Items per block: ceil(costs / per_item).
 void launch_items_per_sc(const int *costs, int nsc, int per_item, int *nitems, hipStream_t s);
 // in_order: the items in block order (else by falling cost, in no fixed order).
 void launch_image_items(const int *costs, int m, int per_item, bool in_order, int *nits, int *ioff, int *out, hipStream_t s);
 // Entry and item offsets (exclusive scans of counts and of ceil(costs / per_item), per_item from the cut and the total
-// cost) and {entries, items, *need, per_item} into out, in one launch; false (nothing launched) when nsc is beyond its
-// single workgroup.
+// cost) and {entries, items, *need} into out, in one launch; false (nothing launched) when nsc is beyond its single
+// workgroup.
 bool launch_list_offsets(const int *counts, const int *costs, int nsc, const ItemCut &cut, int *eoff, int *nits,
                          int *ioff, const int *need, int *out, hipStream_t s);
 // nblocks compaction blocks; the pairs of each block are stored into npairs_block and, when npairs is given, their
