@@ -159,9 +159,9 @@ __device__ __forceinline__ void pair_rows(const TiledFactors &F, double r2, doub
 // the term's undamped magnitude and as root mean squares (here / pair_fp64 / the mixed kernel's rows with 1/r to 2 ulp):
 // at 2-2.8 A Coulomb energy 0.6 / 1.6 / 2.4 and force 0.9 / 0.8 / 1.4, Lennard-Jones energy 1.8 / 2.1 / 3.7 and force
 // 2.3 / 2.4 / 4.8; at 8-10 A 3.1 / 7.3 / 7.8, 0.9 / 4.0 / 1.4, 1.0 / 1.1 / 2.9 and 1.5 / 1.6 / 4.4.
-//   * s = 1/r: one third-order step from v_rsq_f64 (2^-23 or better) with the residual of r2 y y to full precision, so
-//     only the last rounding is left.  t + td is 1/r^2 beyond FP64: s2 and s3 each take one rounding of it.
-//   * Coulomb force: the smoothstep as (1 - u)^2 (1 + 2u), which keeps its relative error towards the outer cutoff.
+//   * s = 1/r: one third-order step from the FP32 seed y, whose square t is exact in FP64, and so is the residual 1 - r2 t
+//     to its last bits: only the step's rounding is left.  t + td is 1/r^2 beyond FP64: s2 and s3 each take one rounding
+//     of it.
 //   * Coulomb energy: s + qShift1 + P0 min(s - 1/inner, 0) + s u (P1 + u (P2 + u P3)), P - 1 about the inner cutoff
 //     less its value there, so that nothing large cancels; the plain region's added terms are exactly zero.
 //   * Lennard-Jones as the reference squares it: C12 (s^6 - w^2)^2 - C6 (s^3 - w)^2 + C0 (rows 2 C12, 2 C6, 2 C0, w: plain
@@ -171,22 +171,21 @@ __device__ __forceinline__ void pair_full(const FullFactors &F, double r2, bool 
                                           unsigned long long mact, const SysDesc *D, int off, double &fs, double &eel,
                                           double &elj)
 {
-    const double y = __builtin_amdgcn_rsq(r2);
-    const double p = r2 * y;
-    const double h = fma(-fma(r2, y, -p), y, fma(-p, y, 1.0));
+    const double y = (double)__builtin_amdgcn_rsqf((float)r2);
+    const double t = y * y;
+    const double h = fma(-r2, t, 1.0);
     const double s = fma(y * h, fma(0.375, h, 0.5), y);
-    const double t = s * s;
-    const double td = t * fma(-r2, t, 1.0);
+    const double td = t * fma(h, h, h);
     const double s2 = t + td;
     const double s3 = fma(s, t, s * td);
     const double s6 = s3 * s3;
-    const double v = 1.0 - u;
-    const double Q = (v * v) * fma(2.0, u, 1.0);
+    const double Q = fma(u * u, fma(2.0, u, F.minus3), 1.0);
     const double R = fma(fma(F.P3, u, F.P2), u, F.P1);
     const double K = fma(F.P0, fmin((s - F.sOn) - F.sOnLow, 0.0), F.q1);
     double e1 = qq * (s + fma(s * u, R, K));
     const double l1 = fma(-C.w, C.w, s6), l2 = s3 - C.w;
-    const double n = sw ? 0.0 : fma(-s3, s3, s6);
+    const double nr = fma(-s3, s3, s6);
+    const double n = __hiloint2double(sw ? 0 : __double2hiint(nr), __double2loint(nr));    // below 2^-1042 when switched
     const double a = C.x * l1;
     double e2 = fma(a, l1, fma(-C.y, fma(l2, l2, n), C.z));
     const double inner = fma(a + a, s6, -(C.y * fma(l2, s3, n)));
@@ -605,10 +604,10 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // image items fill the GPU as the main items drain: 23,559 atoms in a 50 A cell, 139 us per call with two launches,
 // 126 us with one.
 // F64: the full-FP64 instance (NBABFS_TILED_FP64): the same list, tiles, staging and fixed-point sums with pair_full and
-// FP64 force vectors, at three waves per SIMD (134 VGPRs; at four the loop keeps two energy sums in scratch, 20,001 atoms
-// 84 us per call instead of 77 with lists cut for three waves).  With the reference's own expressions (seven divides and a
-// square root per tile, both regions for a wave that holds both) a tile took 790 issue cycles and the call 135 us; with
-// the mixed kernel's rows and 1/r to 2 ulp 71 us, but pair terms off by 1.6 to 4 times as much (pair_full).
+// FP64 force vectors, at three waves per SIMD (134 VGPRs; at four the loop keeps two energy sums in scratch).  Us per call
+// of 20,001 atoms and of 16 images of 30,000: 75 and 937; at four waves 83 and 934; with the reference's own expressions
+// (seven divides and a square root per tile, both regions for a wave that holds both) 141 and 1918; with the mixed kernel's
+// rows and 1/r to 2 ulp 73 and 766, but pair terms off by 1.6 to 4 times as much (pair_full).
 // WPG: wavefronts per workgroup.  With 4 (the one-item-per-wave launches),
 // the row table is staged once for four items and a group's LDS stays small
 // enough for five waves per SIMD; the four items of a group belong to one

@@ -231,6 +231,7 @@ static void make_full_factors(double inner, double outer, const TiledFactors &T,
     const long double a = off * off * (off - 3.0L * on) / gamma, b = 6.0L * off * on / gamma, c = -(off + on) / gamma,
                       d = 0.4L / gamma;
     F.q1 = (double)(8.0L * (off * on * ((long double)outer - inner) - 0.2L * (outer * off * off - inner * on * on)) / gamma);
+    F.minus3 = T.minus3;
     F.P0 = (double)((a - 1.0L) - on * (b + on * (c + d * on)));
     F.P1 = (double)(-w * (b + on * (2.0L * c + 3.0L * d * on)));
     F.P2 = (double)(-w * w * (c + 3.0L * d * on));

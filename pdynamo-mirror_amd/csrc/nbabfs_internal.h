@@ -61,6 +61,7 @@ struct FullFactors : AbfsFactors {
     double sOn, sOnLow;         // 1 / inner cutoff and what its rounding left
     double P0, P1, P2, P3;      // P - 1 = P0 + u (P1 + u (P2 + u P3))
     double q1;                  // qShift1
+    double minus3;              // as above
 };
 
 struct Entry {              // 80 bytes
