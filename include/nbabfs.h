@@ -45,8 +45,9 @@ extern "C" {
                                  the reference expression order (divide, sqrt)      */
 #define NBABFS_TILED_FP64 2   /* the tiled kernel's list, tiles and fixed-point sums
                                  with FP64 pair arithmetic and FP64 force vectors:
-                                 the mixed path without its FP32 parts.  No divide
-                                 or square root, but each pair term as close to its
+                                 the mixed path without its FP32 parts (the seed of
+                                 1/r is refined to its last rounding).  No divide or
+                                 square root, but each pair term as close to its
                                  exact value as in the reference's expressions
                                  (no image lists)                                    */
 
