@@ -590,6 +590,12 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
     return u;
 }
 
+// The factors that an instance of the kernel takes.
+template <bool F64>
+struct PairFactors {
+    using type = typename std::conditional<F64, FullFactors, TiledFactors>::type;
+};
+
 // Waves per SIMD.  A tile is a chain of two LDS reads and about forty dependent FP64 instructions, so the issue slots
 // fill only with enough waves: five fit in 96 VGPRs, with no spill inside the entry loop, because the loop holds no
 // 64-bit lane offsets, one LDS address for all tiles (records at a 16-byte-aligned stride with the type beside the
@@ -614,15 +620,10 @@ __device__ __forceinline__ WorkItem uniform_item(const WorkItem &w)
 // system (batches pad each system's items to a multiple of 4 with empty
 // ones).  The persistent queues run one wave per group, at four waves per SIMD: their loop over items takes 111 VGPRs, and
 // at five it spilled (30,000 atoms on four waves per CU 135 us per call, 131 without the spills; on twelve no difference).
-template <bool F64>
-struct PairFactors {
-    using type = typename std::conditional<F64, FullFactors, TiledFactors>::type;
-};
-
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
 __global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(tiled_waves(F64, IMG, WPG == 1)))) void k_force_tiled(
-    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp, typename PairFactors<F64>::type F, int rows_bytes,
-    int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
+    const SysDesc *__restrict__ descs, const WorkItem *__restrict__ items, QueueParams qp,
+    typename PairFactors<F64>::type F, int rows_bytes, int wave_bytes, ForceGuard guard, int nitems, int nforce_groups, int sys1)
 {
     const int lane = threadIdx.x & 63;
     const int wave = WPG == 1 ? 0 : (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1308,7 +1309,8 @@ void launch_prepare(const SysDesc *d_desc, int nsys, int max_npad, int tiled, in
 
 template <bool ROWS_LDS, bool IMG, bool F64, int WPG>
 static void launch_tiled_instance(dim3 grid, size_t bytes, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop,
-                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q, const typename PairFactors<F64>::type &F,
+                                  const SysDesc *d_desc, const WorkItem *items, QueueParams q,
+                                  const typename PairFactors<F64>::type &F,
                                   int rows_bytes, int wave_bytes, ForceGuard g, int nitems, int nforce_groups,
                                   int sys1)
 {

@@ -2608,7 +2608,7 @@ struct nbabfs_batch {
     PinBuf<SysDesc> h_desc;
     DBuf<WorkItem> items;
     DBuf<int> heads, qstarts;
-    MappedBuf<int> flags;               // [k]: epoch when system k must be rebuilt; [nsys]: epoch of the last test
+    MappedBuf<int> flags;           // [k]: epoch when system k must be rebuilt; [nsys]: epoch of the last test
     // Guard words of the batch's passes: [0] the epoch when some system must be rebuilt, [1] the test's epoch.
     DBuf<int> gguard;
     std::vector<CheckDesc> check_shadow;   // the test's descriptors on the device
@@ -2751,7 +2751,8 @@ static int batch_enqueue(nbabfs_batch *B, hipEvent_t ev_start = nullptr, hipEven
             QueueParams q{s0->opt.wavesPerCU > 0 ? B->heads.p : nullptr, B->qstarts.p};
             int maxnt = 0;
             for (auto *s : B->st) maxnt = std::max(maxnt, s->ntypes);
-            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt, g, st, false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64 ? &s0->F64 : nullptr);
+            launch_force_tiled(B->d_desc.p, B->items.p, q, s0->F, n_persistent_blocks(s0->opt, B->nitems), maxnt, g, st,
+                               false, ev_start, ev_stop, 0, B->precision == NBABFS_TILED_FP64 ? &s0->F64 : nullptr);
         }
     } else {
         launch_force_plain(B->d_desc.p, ns, B->max_n, s0->F, g, st, ev_start, ev_stop);
